@@ -12,8 +12,8 @@ output so the caller's data is untouched), records the fastest with ``amt_zgemm_
 and remembers the bucket for the rest of the process. The result of a product does not
 depend on the split beyond rounding.
 
-Products on the library's large-tile path (FP32 overlaps with both output sides >= 256)
-have their split fixed by accuracy; the hook says so and they are left alone.
+Large FP32 overlaps (both output sides >= 256) keep the built-in choice: the hook says so and
+they are left alone.
 
 It is off by default: on the Si64 and Si8 shapes the heuristic was within a few per cent of
 the best candidate, and tuning the many buckets of a short run (band counts change as bands
@@ -22,7 +22,6 @@ converge) costs more than it saves unless the process runs long enough to reuse 
 
 from __future__ import annotations
 
-import math
 import os
 
 import torch
@@ -41,28 +40,10 @@ def enabled() -> bool:
 
 
 def heuristic_split(m: int, n: int, k: int, batch: int, prec: int = 0, op: int = 1) -> int:
-    """The library's built-in choice (``plan_gemm`` / ``choose_split`` in gemm.hip): the tile
-    (80 rows where that pads less, for FP32 NN, FP32 NC with m < 256 and FP64 NN, unless the
-    FP32 chunks would then need the two-level kernel; else 64 rows; 64 columns), then the
-    smallest split giving about 1024 workgroups and, in FP32 (prec 0), K chunks of at most
-    1024; then as many splits as fit in the same number of 1024-workgroup rounds; at least 256
-    of k per split, at most 256 splits."""
-
-    def split(rows):
-        tiles = ((m + rows - 1) // rows) * ((n + 63) // 64) * batch
-        if tiles >= 512:
-            return 1
-        single = (k + 1023) // 1024 if prec == 0 else 1
-        want = max((1024 + tiles - 1) // tiles, single)
-        rounds = max(1, math.ceil(tiles * want / 1024 - 0.05))
-        want = max(rounds * 1024 // tiles, single)
-        return int(max(1, min(want, (k + 255) // 256, 256)))
-
-    tall = (m + 79) // 80 * 80 < (m + 63) // 64 * 64 and (op == 0 or (prec == 0 and m < 256))
-    ns = split(80 if tall else 64)
-    if tall and prec == 0 and (k + ns - 1) // ns > 1024:
-        ns = split(64)
-    return ns
+    """The library's split for the product (``plan_gemm`` in gemm.hip), read from the size of the
+    workspace it asks for: one partial product per split, none without a split."""
+    partials = int(lib().amt_zgemm_workspace(prec, op, m, n, k, batch))
+    return max(1, partials // (m * n * batch * (16 if prec else 8)))
 
 
 def bucket(prec: int, op: int, m: int, n: int, k: int, batch: int) -> tuple:
@@ -93,7 +74,7 @@ def tune_zgemm(run, prec: int, op: int, m: int, n: int, k: int, batch: int) -> i
     candidates = {min(kmax, 256, max(1, int(round(h * f)))) for f in NEIGHBOURS} - {h}
     for split in [0] + sorted(candidates):
         rc = lib().amt_zgemm_set_split(prec, op, m, n, k, batch, split)
-        if rc == 2:  # a large-tile product: its split is fixed, nothing to tune
+        if rc == 2:  # a large overlap: nothing to tune
             _TUNED[key] = 0
             return 0
         check(rc, "zgemm_set_split")

@@ -16,21 +16,36 @@
 // accumulator differs (measured on gfx950): accumulator element q of lane l is
 // D[4 (l / 16) + q][l % 16] for FP32 and D[l / 16 + 4 q][l % 16] for FP64.
 //
-// Tiling: a 256-thread workgroup (4 wavefronts) computes a 64 x 64 complex tile; each
-// wavefront a 32 x 32 quarter as 2 x 2 MFMA blocks. K advances 16 at a time through two
-// LDS buffers, stored k-major so fragment reads are unit-stride across lanes: the next K
-// tile's global loads are issued before this tile's MFMAs and stored into the other buffer
-// after them, so one barrier per tile suffices and the load latency hides under the MFMAs. Long-K /
-// small-output products (projections onto a few hundred bands) are split along K
-// into enough workgroups to fill 256 CUs, with a deterministic second-pass reduction.
+// Tiling: a 256-thread workgroup computes 16 W rows x 64 columns, W = 1..7 chosen for the row
+// count (plan_gemm): each of the four wavefronts owns 16 columns and all 16 W rows, so 8 bands
+// compute 16 rows, 45 compute 48, 160 two times 80, 440 four times 112, where fixed 64-row tiles
+// computed 64, 64, 192 and 448. K advances 128 bytes of a row at a time (16 complex64, 8
+// complex128) through two LDS buffers: the next tile's 16-byte global loads are issued before
+// this tile's MFMAs and stored after them, one barrier per tile. Rows past M are clamped to the
+// last row and columns of an NN product past N to the last ones (their results are not stored),
+// so whole K tiles load without a test: a test per element had put a wait between the loads.
+// Only the last, partial K tile of a chunk tests each element.
 //
-// FP32 accumulation over a long K chunk is two-level: the MFMA's FP32 accumulators cover
-// kFlushTiles * BK of K and are then added into FP64 registers, so the rounding error of a
-// long contraction (subspace overlaps over ~10^5 plane waves) grows with that length, not
-// with K. One FP32 accumulator over all of K = 81k left relative errors of ~6e-5 in the
-// Gram matrices of a 440-band Davidson, enough to stall an SCF. Chunks of at most
-// kLongChunk (every split-K launch of the projector products) keep the single level and
-// its higher occupancy; split partials are summed in FP64 either way.
+// LDS holds A (and B of an NC product, whose rows run along K too) as rows of 144 bytes: eight
+// 16-byte chunks and 16 bytes of padding, which spreads the 16 rows that a fragment read touches
+// over all banks. One 16-byte read gives a lane its fragment of one MFMA step in FP64 and of two
+// in FP32: lane group g = lane / 16 reads chunk 4 p + g, i.e. the K index of step (p, s) is
+// (4 p + g) * (16 / sizeof(C)) + s; any order of K is the same sum as long as A and B agree. B of
+// an NN product stays [k][column], read 8 (16) bytes at a time from rows of 72 (64) elements.
+//
+// FP32 accumulation over a long K is two-level: the MFMA's FP32 accumulators cover flush_k() of K
+// and are then added into FP64 registers, so the rounding error of a long contraction (subspace
+// overlaps over ~10^5 plane waves) grows with that length, not with K. One FP32 accumulator over
+// all of K = 81k left relative errors of ~6e-5 in the Gram matrices of a 440-band Davidson,
+// enough to stall an SCF. The additions cost 2 to 5 % of a product; split partials are summed in
+// FP64 too.
+//
+// What bounds it: the matrix cores. Of a wavefront's cycles on 440 x 3852 x 40 000 (FP32, NC) 81 %
+// are MFMA at the 2.14 GHz the chip holds under them. Measured (TFLOP/s at 8 real flops per
+// complex multiply-add; in brackets 64- and 80-row tiles with a test per element):
+//   FP32 160 x 1152 x 37073 NC 135 (118), 160 x 37073 x 1152 NN 128 (90), 640 x 160 x 37073 NC
+//   122 (100), 45 x 3852 x 80989 NC 127 (84), 440 x 80989 x 3852 NN 149 (113), 440 x 3852 x 80989
+//   NC 150 (107); FP64 160 x 1152 x 37073 NC 73 (46), its NN 76 (53), 45 x 3852 x 80989 NC 65 (39).
 #include <array>
 #include <cmath>
 #include <map>
@@ -63,38 +78,48 @@ struct Mfma<double> {
   static __device__ __forceinline__ int row(int lane, int q) { return (lane >> 4) + 4 * q; }
 };
 
-constexpr int BM = 64, BN = 64, BK = 16;
-constexpr int kFlushTiles = 4;
+constexpr int BN = 64;            // columns of a tile
+constexpr int kChunks = 8;        // 16-byte chunks of one operand row and K tile
+// K between the two-level form's additions into FP64: 64 for NN products, 256 for NC ones
+template <int OP>
+constexpr int flush_k() {
+  return OP == 0 ? 64 : 256;
+}
 
-// Tile shapes TM: 1 = 64 x 64 tiles (each wavefront 32 x 32 as 2 x 2 MFMA blocks); 2 (FP32,
-// single level) = 128 x 128 tiles, each wavefront 64 x 64 as 4 x 4 blocks, half the operand
-// traffic per MFMA for large products; kTall = 80 x 64 tiles, the four wavefronts side by
-// side, each 80 x 16 as 5 x 1 blocks: 160-, 480- or 800-row operands (the Si64 band blocks
-// and their multiples) fill them exactly, where 64-row tiles compute 20 % of padding.
-constexpr int kTall = 5;
-
-template <int TM>
-struct TileShape {
-  static constexpr int rows = TM == kTall ? 80 : BM * TM, cols = TM == kTall ? 64 : BN * TM;
-  static constexpr int wave_rows = TM == kTall ? 5 : 2 * TM, wave_cols = TM == kTall ? 1 : 2 * TM;  // MFMA blocks
+template <typename R>
+struct Vec16;  // 16 bytes of a row: two complex64 or one complex128
+template <>
+struct Vec16<float> {
+  typedef float T __attribute__((ext_vector_type(4)));
+  typedef float U __attribute__((ext_vector_type(4), aligned(8)));  // rows start at any element
+};
+template <>
+struct Vec16<double> {
+  typedef double T __attribute__((ext_vector_type(2)));
+  typedef double U __attribute__((ext_vector_type(2), aligned(16)));
 };
 
-template <typename R, int OP, bool kTwoLevel, int TM>
-__global__ __launch_bounds__(256, TM == 2 ? 2 : 1) void k_zgemm(int M, int N, int K, int kchunk, int nsplit,
+template <typename R, int OP, bool kTwoLevel, int W>
+__global__ __launch_bounds__(256, 2) void k_zgemm(int M, int N, int K, int kchunk, int nsplit,
                                                const typename Cplx<R>::T* __restrict__ A, long long lda,
                                                long long sA, const typename Cplx<R>::T* __restrict__ B,
                                                long long ldb, long long sB, typename Cplx<R>::T* __restrict__ Cm,
                                                long long ldc, long long sC, R alpha, R beta,
                                                typename Cplx<R>::T* __restrict__ part, int mfast) {
-  static_assert(TM != 2 || !kTwoLevel, "the two-level accumulation uses the 64- or 80-row tiles");
   using C = typename Cplx<R>::T;
   using acc_t = typename Mfma<R>::acc_t;
-  constexpr int TBM = TileShape<TM>::rows, TBN = TileShape<TM>::cols;
-  constexpr int WBR = TileShape<TM>::wave_rows, WBC = TileShape<TM>::wave_cols;  // MFMA blocks per wave
-  constexpr int KQ = TM == kTall ? 4 : 4 * TM;  // consecutive k (or columns) per thread in a 64-wide load
-  constexpr int AE = TBM * BK / 256;            // A elements per thread and K tile
-  __shared__ C As[2][BK][TBM + 1];  // double-buffered K tiles
-  __shared__ C Bs[2][BK][TBN + 1];
+  using V = typename Vec16<R>::T;
+  using VU = typename Vec16<R>::U;
+  constexpr int E = 16 / sizeof(C);        // elements per chunk, MFMA steps per fragment read
+  constexpr int BK = kChunks * E;          // K per tile
+  constexpr int ROWS = 16 * W;
+  constexpr int NA = (ROWS + 31) / 32;     // A chunks per thread
+  constexpr int NB = 2;                    // B chunks per thread (64 x 8, or BK x 64 / E)
+  constexpr int CPR = BN / E;              // chunks per K row of an NN product's B tile
+  constexpr int LDB = sizeof(C) == 8 ? BN + 8 : BN;  // elements per K row of it in LDS
+  constexpr int BSZ = OP == 0 ? BK * LDB * (int)sizeof(C) / 16 : BN * (kChunks + 1);
+  __shared__ V As[2][ROWS][kChunks + 1];
+  __shared__ V Bs[2][BSZ];
   // XCD-aware order: workgroups are handed to the 8 XCDs round-robin by linear id, so
   // logical tile t = (id % 8) * (T8 / 8) + id / 8 gives each XCD a contiguous run of tiles
   // that share an operand panel in its L2: the N-tiles of one M-tile and K-chunk (A panel),
@@ -106,187 +131,238 @@ __global__ __launch_bounds__(256, TM == 2 ? 2 : 1) void k_zgemm(int M, int N, in
   const unsigned txy = tl % gxy;
   const int bz = (int)(tl / gxy);
   const int batch = bz / nsplit, split = bz % nsplit;
-  const int m0 = (int)(mfast ? txy % gy : txy / gx) * TBM, n0 = (int)(mfast ? txy / gy : txy % gx) * TBN;
+  const int m0 = (int)(mfast ? txy % gy : txy / gx) * ROWS, n0 = (int)(mfast ? txy / gy : txy % gx) * BN;
   const int kbeg = split * kchunk;
   const int kend = (kbeg + kchunk < K) ? kbeg + kchunk : K;
   A += (long long)batch * sA;
   B += (long long)batch * sB;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = TM == kTall ? 0 : (wave >> 1) * 32 * TM, wc = TM == kTall ? wave * 16 : (wave & 1) * 32 * TM;
-  acc_t p1[WBR][WBC], p2[WBR][WBC], p3[WBR][WBC];  // Gauss's three products
+  const int l15 = lane & 15, grp = lane >> 4;
+  acc_t p1[W], p2[W], p3[W];  // Gauss's three products
 #pragma unroll
-  for (int a = 0; a < WBR; ++a)
+  for (int a = 0; a < W; ++a)
 #pragma unroll
-    for (int b = 0; b < WBC; ++b)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        p1[a][b][q] = 0;
-        p2[a][b][q] = 0;
-        p3[a][b][q] = 0;
-      }
+    for (int q = 0; q < 4; ++q) {
+      p1[a][q] = 0;
+      p2[a][q] = 0;
+      p3[a][q] = 0;
+    }
+  // C_re and C_im of one accumulator element; conj(B) turns the signs of the P2 terms
+  auto re_of = [](auto t1, auto t2) { return OP == 0 ? t1 - t2 : t1 + t2; };
+  auto im_of = [](auto t1, auto t2, auto t3) { return OP == 0 ? t3 - t1 - t2 : t3 - t1 + t2; };
   // second-level FP64 sums of the FP32 accumulators (two-level form only)
-  double sumr[kTwoLevel ? WBR : 1][kTwoLevel ? WBC : 1][4], sumi[kTwoLevel ? WBR : 1][kTwoLevel ? WBC : 1][4];
+  double sumr[kTwoLevel ? W : 1][4], sumi[kTwoLevel ? W : 1][4];
   auto flush = [&]() {
     if constexpr (kTwoLevel) {
 #pragma unroll
-      for (int a = 0; a < WBR; ++a)
+      for (int a = 0; a < W; ++a)
 #pragma unroll
-        for (int b = 0; b < WBC; ++b)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const double t1 = p1[a][b][q], t2 = p2[a][b][q], t3 = p3[a][b][q];
-            sumr[a][b][q] += t1 - t2;
-            sumi[a][b][q] += t3 - t1 - t2;
-            p1[a][b][q] = 0;
-            p2[a][b][q] = 0;
-            p3[a][b][q] = 0;
-          }
+        for (int q = 0; q < 4; ++q) {
+          const double t1 = p1[a][q], t2 = p2[a][q], t3 = p3[a][q];
+          sumr[a][q] += re_of(t1, t2);
+          sumi[a][q] += im_of(t1, t2, t3);
+          p1[a][q] = 0;
+          p2[a][q] = 0;
+          p3[a][q] = 0;
+        }
     }
   };
   if constexpr (kTwoLevel) {
 #pragma unroll
-    for (int a = 0; a < WBR; ++a)
+    for (int a = 0; a < W; ++a)
 #pragma unroll
-      for (int b = 0; b < WBC; ++b)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          sumr[a][b][q] = 0.0;
-          sumi[a][b][q] = 0.0;
-        }
+      for (int q = 0; q < 4; ++q) {
+        sumr[a][q] = 0.0;
+        sumi[a][q] = 0.0;
+      }
   }
-  // Global -> register loads of one K tile (bounds-checked, conj(B) for NC), and the store of
-  // those registers into an LDS buffer: A k-major As[k][row]; B k-major Bs[k][col].
-  // The 80-row tile loads A as AE single elements per thread (16 threads per row of 16 k).
-  C ra[TM == kTall ? AE : KQ], rb[KQ];
-  auto gload = [&](int k0) {
-    if constexpr (TM == kTall) {
+  // A chunk (row, c): id = tid + 256 u, row = id / 8, c = id % 8. The first K tile's addresses.
+  const C* pa[NA];
 #pragma unroll
-      for (int u = 0; u < AE; ++u) {
-        const int idx = tid + 256 * u, row = idx / BK, gm = m0 + row, gk = k0 + idx % BK;
-        ra[u] = (gm < M && gk < kend) ? A[(long long)gm * lda + gk] : cmake<C>(0, 0);
-      }
+  for (int u = 0; u < NA; ++u) {
+    const int row = m0 + tid / kChunks + 32 * u;
+    pa[u] = A + (long long)(row < M ? row : M - 1) * lda + kbeg + (tid % kChunks) * E;
+  }
+  const C* pb[NB];
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    if constexpr (OP == 0) {
+      const int e = tid + 256 * u, k = e / CPR, c = n0 + (e % CPR) * E;
+      pb[u] = B + (long long)(kbeg + k) * ldb + c;
     } else {
-      const int row = tid / (BK / KQ), kq = (tid % (BK / KQ)) * KQ;
-      const int gm = m0 + row;
-#pragma unroll
-      for (int u = 0; u < KQ; ++u) {
-        const int gk = k0 + kq + u;
-        ra[u] = (gm < M && gk < kend) ? A[(long long)gm * lda + gk] : cmake<C>(0, 0);
-      }
+      const int col = n0 + tid / kChunks + 32 * u;
+      pb[u] = B + (long long)(col < N ? col : N - 1) * ldb + kbeg + (tid % kChunks) * E;
     }
-    if (OP == 0) {
-      const int kk = tid >> 4, c0 = (tid & 15) * KQ;
-      const int gk = k0 + kk;
+  }
+  const long long stepb = OP == 0 ? (long long)BK * ldb : BK;
+  // Column chunks of an NN tile past N read the last E columns instead; one that starts at the
+  // last column (FP32, N - n0 odd) finds it in its second element.
+  bool last_col[NB];
 #pragma unroll
-      for (int u = 0; u < KQ; ++u) {
-        const int gn = n0 + c0 + u;
-        rb[u] = (gk < kend && gn < N) ? B[(long long)gk * ldb + gn] : cmake<C>(0, 0);
-      }
-    } else {
-      const int col = tid / (BK / KQ), kq = (tid % (BK / KQ)) * KQ;
-      const int gn = n0 + col;
+  for (int u = 0; u < NB; ++u) {
+    const int c = n0 + ((tid + 256 * u) % CPR) * E;
+    last_col[u] = OP == 0 && E == 2 && N >= E && c == N - 1;
+    if (OP == 0 && c > N - E && N >= E) pb[u] -= c - (N - E);
+  }
+  V ra[NA], rb[NB];
+  // whole K tile: no test, so the loads of a tile are all in flight together
+  auto gload = [&]() {
 #pragma unroll
-      for (int u = 0; u < KQ; ++u) {
-        const int gk = k0 + kq + u;
-        C v = (gn < N && gk < kend) ? B[(long long)gn * ldb + gk] : cmake<C>(0, 0);
-        v.y = -v.y;
-        rb[u] = v;
+    for (int u = 0; u < NA; ++u) {
+      if (ROWS % 32 == 0 || u < NA - 1 || tid < 128) ra[u] = *reinterpret_cast<const VU*>(pa[u]);
+      pa[u] += BK;
+    }
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      rb[u] = *reinterpret_cast<const VU*>(pb[u]);
+      pb[u] += stepb;
+    }
+  };
+  // the last K tile of a chunk (and every tile of a one-column FP32 NN product): element by
+  // element, zeros past kend
+  auto gload_tail = [&](int k0) {
+    const int left = kend - k0 - (tid % kChunks) * E;  // elements of this thread's row chunk that exist
+    auto some = [](const C* q, int have) {
+      V v;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        C x = cmake<C>(0, 0);
+        if (e < have) x = q[e];
+        v[2 * e] = x.x;
+        v[2 * e + 1] = x.y;
       }
+      return v;
+    };
+#pragma unroll
+    for (int u = 0; u < NA; ++u) {
+      if (ROWS % 32 == 0 || u < NA - 1 || tid < 128) ra[u] = some(pa[u], left);
+      pa[u] += BK;
+    }
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      if constexpr (OP == 0) {
+        const int e = tid + 256 * u, c = n0 + (e % CPR) * E;
+        rb[u] = some(pb[u], k0 + e / CPR < kend ? (N >= E ? E : N - c) : 0);
+      } else {
+        rb[u] = some(pb[u], left);
+      }
+      pb[u] += stepb;
     }
   };
   auto sstore = [&](int buf) {
-    if constexpr (TM == kTall) {
 #pragma unroll
-      for (int u = 0; u < AE; ++u) {
-        const int idx = tid + 256 * u;
-        As[buf][idx % BK][idx / BK] = ra[u];
+    for (int u = 0; u < NA; ++u)
+      if (ROWS % 32 == 0 || u < NA - 1 || tid < 128) As[buf][tid / kChunks + 32 * u][tid % kChunks] = ra[u];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      if constexpr (OP == 0) {
+        const int e = tid + 256 * u;
+        V v = rb[u];
+        if constexpr (E == 2) {
+          v[0] = last_col[u] ? v[2] : v[0];
+          v[1] = last_col[u] ? v[3] : v[1];
+        }
+        Bs[buf][(e / CPR) * (LDB / E) + e % CPR] = v;
+      } else {
+        Bs[buf][(tid / kChunks + 32 * u) * (kChunks + 1) + tid % kChunks] = rb[u];
+      }
+    }
+  };
+  // the fragments of steps (p, 0 .. E - 1) and their MFMAs
+  struct Frag {
+    V a[W], b;
+  };
+  auto fragments = [&](Frag& f, int buf, int p) {
+#pragma unroll
+    for (int r = 0; r < W; ++r) f.a[r] = As[buf][r * 16 + l15][p * 4 + grp];
+    if constexpr (OP == 0) {
+      const C* bs = reinterpret_cast<const C*>(&Bs[buf][0]) + (p * 4 + grp) * E * LDB + wave * 16 + l15;
+#pragma unroll
+      for (int s = 0; s < E; ++s) {
+        const C b = bs[s * LDB];
+        f.b[2 * s] = b.x;
+        f.b[2 * s + 1] = b.y;
       }
     } else {
-      const int row = tid / (BK / KQ), kq = (tid % (BK / KQ)) * KQ;
-#pragma unroll
-      for (int u = 0; u < KQ; ++u) As[buf][kq + u][row] = ra[u];
-    }
-    if (OP == 0) {
-      const int kk = tid >> 4, c0 = (tid & 15) * KQ;
-#pragma unroll
-      for (int u = 0; u < KQ; ++u) Bs[buf][kk][c0 + u] = rb[u];
-    } else {
-      const int col = tid / (BK / KQ), kq = (tid % (BK / KQ)) * KQ;
-#pragma unroll
-      for (int u = 0; u < KQ; ++u) Bs[buf][kq + u][col] = rb[u];
+      f.b = Bs[buf][(wave * 16 + l15) * (kChunks + 1) + p * 4 + grp];
     }
   };
-  auto compute = [&](int buf) {
+  auto products = [&](const Frag& f) {
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int kr = ks * 4 + (lane >> 4);
-      C a[WBR], b[WBC];
+    for (int s = 0; s < E; ++s) {
+      const R bx = f.b[2 * s], by = f.b[2 * s + 1], bz2 = OP == 0 ? bx + by : bx - by;
 #pragma unroll
-      for (int rb2 = 0; rb2 < WBR; ++rb2) a[rb2] = As[buf][kr][wr + rb2 * 16 + (lane & 15)];
-#pragma unroll
-      for (int cb = 0; cb < WBC; ++cb) b[cb] = Bs[buf][kr][wc + cb * 16 + (lane & 15)];
-#pragma unroll
-      for (int rb2 = 0; rb2 < WBR; ++rb2)
-#pragma unroll
-        for (int cb = 0; cb < WBC; ++cb) {
-          p1[rb2][cb] = Mfma<R>::mma(a[rb2].x, b[cb].x, p1[rb2][cb]);
-          p2[rb2][cb] = Mfma<R>::mma(a[rb2].y, b[cb].y, p2[rb2][cb]);
-          p3[rb2][cb] = Mfma<R>::mma(a[rb2].x + a[rb2].y, b[cb].x + b[cb].y, p3[rb2][cb]);
-        }
+      for (int r = 0; r < W; ++r) {
+        const R ax = f.a[r][2 * s], ay = f.a[r][2 * s + 1];
+        p1[r] = Mfma<R>::mma(ax, bx, p1[r]);
+        p2[r] = Mfma<R>::mma(ay, by, p2[r]);
+        p3[r] = Mfma<R>::mma(ax + ay, bz2, p3[r]);
+      }
     }
   };
-  int tiles = 0;
-  // double-buffered: the next tile's global loads are in flight while this tile's MFMAs run,
-  // and one barrier per tile separates the store of the next buffer from the reads of this one
-  if (kbeg < kend) {
-    gload(kbeg);
-    sstore(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = kbeg; k0 < kend; k0 += BK) {
-    const bool more = k0 + BK < kend;
-    if (more) gload(k0 + BK);
-    compute(buf);
+  const int nt = kbeg < kend ? (kend - kbeg + BK - 1) / BK : 0;                 // K tiles
+  const int nfull = OP == 0 && N < E ? 0 : (kbeg < kend ? (kend - kbeg) / BK : 0);  // of which whole
+  auto gload_tile = [&](int tile) {
+    if (tile < nfull)
+      gload();
+    else if (tile < nt)
+      gload_tail(kbeg + tile * BK);
+  };
+  // A tile's turn: its first fragments are in f0 and the next tile's values in ra, rb. The next
+  // tile goes to the other buffer and its successor's loads are issued; the barrier that makes it
+  // visible and the read of its first fragments lie between the two halves of the MFMAs.
+  Frag f0, f1;
+  int buf = 0, tile = 0;
+  auto step = [&](auto load, bool more) {
+    fragments(f1, buf, 1);
     if (more) sstore(buf ^ 1);
+    load();
+    products(f0);
     __syncthreads();
     buf ^= 1;
+    if (more) fragments(f0, buf, 0);
+    products(f1);
+    ++tile;
     if constexpr (kTwoLevel) {
-      if (++tiles == kFlushTiles) {
-        flush();
-        tiles = 0;
-      }
+      if (tile % (flush_k<OP>() / BK) == 0) flush();
     }
+  };
+  if (nt > 0) {
+    gload_tile(0);
+    sstore(0);
+    gload_tile(1);
+    __syncthreads();
+    fragments(f0, 0, 0);
+    while (tile + 2 < nfull) step(gload, true);
+    while (tile < nt) step([&] { gload_tile(tile + 2); }, tile + 1 < nt);
   }
   flush();
 #pragma unroll
-  for (int rb = 0; rb < WBR; ++rb)
+  for (int r = 0; r < W; ++r)
 #pragma unroll
-    for (int cb = 0; cb < WBC; ++cb)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int row = m0 + wr + rb * 16 + Mfma<R>::row(lane, q);
-        const int col = n0 + wc + cb * 16 + (lane & 15);
-        if (row < M && col < N) {
-          C v;
-          if constexpr (kTwoLevel)
-            v = cmake<C>((R)sumr[rb][cb][q], (R)sumi[rb][cb][q]);
-          else
-            v = cmake<C>(p1[rb][cb][q] - p2[rb][cb][q], p3[rb][cb][q] - p1[rb][cb][q] - p2[rb][cb][q]);
-          if (part) {
-            part[(((long long)batch * nsplit + split) * M + row) * N + col] = v;
-          } else {
-            C* dst = Cm + (long long)batch * sC + (long long)row * ldc + col;
-            C o = cmake<C>(alpha * v.x, alpha * v.y);
-            if (beta != (R)0) {
-              const C old = *dst;
-              o.x += beta * old.x;
-              o.y += beta * old.y;
-            }
-            *dst = o;
+    for (int q = 0; q < 4; ++q) {
+      const int row = m0 + r * 16 + Mfma<R>::row(lane, q);
+      const int col = n0 + wave * 16 + l15;
+      if (row < M && col < N) {
+        C v;
+        if constexpr (kTwoLevel)
+          v = cmake<C>((R)sumr[r][q], (R)sumi[r][q]);
+        else
+          v = cmake<C>(re_of(p1[r][q], p2[r][q]), im_of(p1[r][q], p2[r][q], p3[r][q]));
+        if (part) {
+          part[(((long long)batch * nsplit + split) * M + row) * N + col] = v;
+        } else {
+          C* dst = Cm + (long long)batch * sC + (long long)row * ldc + col;
+          C o = cmake<C>(alpha * v.x, alpha * v.y);
+          if (beta != (R)0) {
+            const C old = *dst;
+            o.x += beta * old.x;
+            o.y += beta * old.y;
           }
+          *dst = o;
         }
       }
+    }
 }
 
 // Sum of the split partials in FP64: each output element is summed by kReduceGroups threads
@@ -334,57 +410,90 @@ __global__ __launch_bounds__(kReduceGroups * kReduceCols) void k_splitk_reduce(
   *dst = o;
 }
 
-// Split-K factor: a tuned value for the shape's bucket (tiles of M and N, K in 256s,
-// batch) when one was recorded with set_zgemm_split, else: the smallest split that gives
-// about 1024 workgroups (four 64 x 64 tiles per CU) and, in FP32, K chunks of at most
-// kLongChunk (the single-level kernel, at twice the two-level one's occupancy); then as
-// many splits as still fit in the same number of 1024-workgroup rounds (a few per cent over
-// a round does not count as another), so the chunks get shorter at no extra round. At least
-// 256 of K per split, at most 256 splits. Measured on the Si64 projections and overlaps
-// (K = 37 073): 1.5-1.7x faster than about 1024 workgroups alone.
+// ----------------------------------------------------------------------- choices
 static std::mutex g_split_mutex;
 static std::map<std::array<int, 6>, int> g_split_table;
 
 static std::array<int, 6> split_key(int prec, int op, int m, int n, int k, int batch) {
-  return {prec, op, (m + BM - 1) / BM, (n + BN - 1) / BN, (k + 255) / 256, batch};
+  return {prec, op, (m + 63) / 64, (n + 63) / 64, (k + 255) / 256, batch};
 }
 
-constexpr int kLongChunk = 1024;
+// Longest K that one FP32 accumulator covers. NC products (overlaps, projections: K the plane
+// waves) carry FP64 sums beyond 256 of K whatever their split; NN products (rotations, projector
+// applications) beyond 1024.
+constexpr int single_level_k(int op) { return op == 1 ? flush_k<1>() : 1024; }
+constexpr int kMinChunk = 64;
+// FP32 NC products with both output sides at least this are left alone by the split tuning.
+constexpr int kBigSide = 256;
 
-static int choose_split(int prec, int op, int m, int n, int k, int batch, int tile_rows) {
-  const long long kmax = (k + 255) / 256;
-  {
+// Tile rows in 16s, widest kernel of each kind (registers: two wavefronts per SIMD).
+constexpr int kMaxW = 7, kMaxWLong = 5;
+
+struct GemmPlan {
+  int w;        // rows of a tile in 16s
+  int ns;       // K splits
+  int kchunk;   // K per split, a multiple of the K tile
+  bool two;     // FP64 second-level sums
+};
+
+static bool split_is_tunable(int prec, int op, int m, int n, int k) {
+  return !(prec == kFP32 && op == 1 && m >= kBigSide && n >= kBigSide && k > 0);
+}
+
+// W and the split along K, by the time a plan takes in units of one 16-row K tile of one
+// workgroup (0.18 us: 12 MFMAs of 32 or 6 of 64 cycles in each wavefront):
+//   (ceil(workgroups / 256 CUs) + 0.8) * (K tiles + 2) * (W + 0.35)  + the partials' traffic,
+// the 2 standing for a workgroup's start and end, the 0.35 for a tile's work beside its rows
+// (barrier, B operand) and the 0.8 for the last workgroups of a CU, which have fewer wavefronts
+// beside them to hide their waits (so a few long workgroups per CU lose to more, shorter ones).
+// The first factor is what uneven rounds cost: 160 x 37 073 x 1152 (580
+// column tiles) in 32-row tiles fills its last round better than in 80-row ones. Against a sweep
+// of every W and split the choice is within 5 % on the Si8, Si64 and Si214 shapes.
+// Whether a product carries FP64 sums depends on its chunk (NC) or its K (NN) only
+// (single_level_k), so the split does not change its error: 3.7-4.1e-7 (relative norm, random
+// operands) on every NC shape above, where single accumulators over 256 to 1024 of K gave 4.1
+// to 7.9e-7.
+static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
+  const int csize = prec == kFP64 ? 16 : 8, bk = kChunks * 16 / csize;
+  const double cols = (double)((n + BN - 1) / BN) * batch, out = (double)m * n * batch * csize;
+  GemmPlan best{1, 1, bk, false};
+  double best_cost = 1e300;
+  int lo = 1, hi = (k + kMinChunk - 1) / kMinChunk;
+  hi = hi > 256 ? 256 : hi < 1 ? 1 : hi;
+  if (split_is_tunable(prec, op, m, n, k)) {
     std::lock_guard<std::mutex> lock(g_split_mutex);
     auto it = g_split_table.find(split_key(prec, op, m, n, k, batch));
-    if (it != g_split_table.end()) {
-      long long s = it->second;
-      if (s > kmax) s = kmax;
-      return s < 1 ? 1 : (int)s;
+    if (it != g_split_table.end()) lo = hi = it->second < hi ? it->second : hi;
+  }
+  double rows[kMaxW + 1];
+  for (int w = 1; w <= kMaxW; ++w) rows[w] = (double)((m + 16 * w - 1) / (16 * w)) * cols;
+  for (int want = lo; want <= hi; want += 1 + want / 8) {
+    int kchunk = ((k + want - 1) / want + bk - 1) / bk * bk;
+    if (kchunk < bk) kchunk = bk;
+    const int ns = k > 0 ? (k + kchunk - 1) / kchunk : 1;
+    if (best_cost < 1e300 && (long long)batch * ns > 65535) break;
+    const bool two = prec == kFP32 && (op == 1 ? kchunk : k) > single_level_k(op);
+    const double tiles = kchunk / bk + 2, extra = ns > 1 ? 20.0 + 2.0 * out * ns / 1.3e6 : 0.0;
+    for (int w = 1; w <= (prec == kFP64 || two ? kMaxWLong : kMaxW); ++w) {
+      const double cost = (std::ceil(rows[w] * ns / 256.0) + 0.8) * tiles * (w + 0.35) * (two ? 1.1 : 1.0) + extra;
+      if (cost < best_cost) {
+        best_cost = cost;
+        best.w = w;
+        best.ns = ns;
+        best.kchunk = kchunk;
+        best.two = two;
+      }
     }
   }
-  const long long tiles = (long long)((m + tile_rows - 1) / tile_rows) * ((n + BN - 1) / BN) * batch;
-  if (tiles >= 512) return 1;
-  long long want = (1024 + tiles - 1) / tiles;
-  const long long single = prec == kFP32 ? (k + kLongChunk - 1) / kLongChunk : 1;
-  if (single > want) want = single;
-  long long rounds = (long long)std::ceil((double)(tiles * want) / 1024.0 - 0.05);
-  if (rounds < 1) rounds = 1;
-  const long long fill = rounds * 1024 / tiles;
-  want = fill > single ? fill : single;
-  if (want > kmax) want = kmax;
-  if (want > 256) want = 256;
-  if (want < 1) want = 1;
-  return (int)want;
+  return best;
 }
-
-static bool takes_large_tiles(int prec, int op, int m, int n, int k, int batch);
 
 int set_zgemm_split(int prec, int op, int m, int n, int k, int batch, int split) {
   if (split < 0 || split > 256) {
     set_error("zgemm split must be 0 (heuristic) .. 256");
     return 1;
   }
-  if (takes_large_tiles(prec, op, m, n, k, batch)) return 2;  // K chunks fixed by accuracy
+  if (!split_is_tunable(prec, op, m, n, k)) return 2;
   std::lock_guard<std::mutex> lock(g_split_mutex);
   const auto key = split_key(prec, op, m, n, k, batch);
   if (split == 0)
@@ -394,77 +503,12 @@ int set_zgemm_split(int prec, int op, int m, int n, int k, int batch, int split)
   return 0;
 }
 
-// Large FP32 NC products (overlaps and projections: both output sides >= kBigSide, K the
-// plane waves) use 128 x 128 tiles with K chunks of at most kBigChunk: one FP32
-// accumulator per chunk (as accurate as the two-level form for these lengths) and the
-// FP64 split reduction, at the cost of writing and reading the partial products once per
-// chunk (about 5 % of the product's time). Measured on the Si214 overlaps 1.4-2x faster
-// than 64 x 64 tiles; NN products (rotations, projector application) were not faster and
-// keep 64 x 64. Beyond kBigWorkspace of partials the two-level form is used instead.
-constexpr int kBigSide = 256;
-constexpr int kBigChunk = 512;
-constexpr size_t kBigWorkspace = size_t(24) << 30;
-
-struct GemmPlan {
-  int tm;  // tile shape (1, 2 or kTall)
-  int ns;  // K splits (before rounding the chunk to BK)
-};
-
-static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
-  if (prec == kFP32 && op == 1 && m >= kBigSide && n >= kBigSide && k > 0) {
-    const long long tiles = (long long)((m + 2 * BM - 1) / (2 * BM)) * ((n + 2 * BN - 1) / (2 * BN)) * batch;
-    long long ns = (k + kBigChunk - 1) / kBigChunk;
-    if (tiles < 512) {
-      long long want = (1024 + tiles - 1) / tiles;
-      const long long kmax = (k + 255) / 256;
-      if (want > kmax) want = kmax;
-      if (want > ns) ns = want;
-    }
-    const size_t bytes = ns > 1 ? (size_t)batch * ns * m * n * 8 : 0;
-    if (batch * ns <= 65535 && bytes <= kBigWorkspace) return {2, (int)ns};
-  }
-  // 80-row tiles where they leave fewer padded rows than 64-row ones (m = 160, 480, ...), for
-  // the products where they measured faster (Si64 shapes, 160-row blocks): FP32 NN and NC with
-  // m < 256 on the single-level kernel (10-21 %), FP64 NN (3-5 %). Their two-level FP32 form
-  // and FP64 NC products run at one wave per SIMD and were slower.
-  bool tall = (m + 79) / 80 * 80 < (m + 63) / 64 * 64 && (prec == kFP32 ? (op == 0 || m < 256) : op == 0);
-  int ns = choose_split(prec, op, m, n, k, batch, tall ? TileShape<kTall>::rows : TileShape<1>::rows);
-  if (tall && prec == kFP32 && (k + ns - 1) / ns > kLongChunk) {
-    tall = false;
-    ns = choose_split(prec, op, m, n, k, batch, TileShape<1>::rows);
-  }
-  return {tall ? kTall : 1, ns};
-}
-
-static bool takes_large_tiles(int prec, int op, int m, int n, int k, int batch) {
-  return plan_gemm(prec, op, m, n, k, batch).tm == 2;
-}
-
 size_t zgemm_workspace_bytes(int prec, int op, int m, int n, int k, int batch) {
   const GemmPlan g = plan_gemm(prec, op, m, n, k, batch);
   if (g.ns <= 1) return 0;
   const size_t c = prec == kFP64 ? 16 : 8;
   return (size_t)batch * g.ns * m * n * c;
 }
-
-template <typename R, bool kTwoLevel, int TM>
-static void launch_tile(int op, dim3 grid, hipStream_t s, int m, int n, int k, int kchunk, int ns, const void* a,
-                        long long lda, long long sa, const void* b, long long ldb, long long sb, void* c,
-                        long long ldc, long long sc, double alpha, double beta, typename Cplx<R>::T* part) {
-  using C = typename Cplx<R>::T;
-  const int mfast = op == 0 && grid.y > 1 && grid.x >= grid.y;
-  if constexpr (TM == 1 || TM == kTall) {
-    if (op == 0) {
-      hipLaunchKernelGGL((k_zgemm<R, 0, kTwoLevel, TM>), grid, dim3(256), 0, s, m, n, k, kchunk, ns, (const C*)a,
-                         lda, sa, (const C*)b, ldb, sb, (C*)c, ldc, sc, (R)alpha, (R)beta, part, mfast);
-      return;
-    }
-  }
-  // 128 x 128 tiles are planned for NC products only
-  hipLaunchKernelGGL((k_zgemm<R, 1, kTwoLevel, TM>), grid, dim3(256), 0, s, m, n, k, kchunk, ns, (const C*)a,
-                     lda, sa, (const C*)b, ldb, sb, (C*)c, ldc, sc, (R)alpha, (R)beta, part, 0);
-}
-
 
 template <typename R>
 static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, long long lda, long long sa,
@@ -473,7 +517,7 @@ static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, lon
   using C = typename Cplx<R>::T;
   if (m <= 0 || n <= 0 || batch <= 0) return 0;
   const GemmPlan g = plan_gemm(std::is_same<R, double>::value ? kFP64 : kFP32, op, m, n, k, batch);
-  int ns = k <= 0 ? 1 : g.ns;
+  const int ns = g.ns, kchunk = g.kchunk;
   const size_t need = ns > 1 ? (size_t)batch * ns * m * n * sizeof(C) : 0;
   C* part = nullptr;
   if (ns > 1) {
@@ -484,32 +528,37 @@ static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, lon
     }
     part = static_cast<C*>(ws);
   }
-  int kchunk = (k + ns - 1) / ns;
-  kchunk = ((kchunk + BK - 1) / BK) * BK;
-  if (kchunk < BK) kchunk = BK;
-  ns = (k + kchunk - 1) / kchunk;
-  if (ns < 1) ns = 1;
   if ((long long)batch * ns > 65535) {
     set_error("zgemm: batch x split exceeds the grid limit");
     return 1;
   }
-  const int trows = g.tm == 2 ? TileShape<2>::rows : g.tm == kTall ? TileShape<kTall>::rows : TileShape<1>::rows;
-  const int tcols = g.tm == 2 ? TileShape<2>::cols : g.tm == kTall ? TileShape<kTall>::cols : TileShape<1>::cols;
-  const dim3 grid((n + tcols - 1) / tcols, (m + trows - 1) / trows, batch * ns);
+  const dim3 grid((n + BN - 1) / BN, (m + 16 * g.w - 1) / (16 * g.w), batch * ns);
+  const int mfast = op == 0 && grid.y > 1 && grid.x >= grid.y;
   C* const p = ns > 1 ? part : nullptr;
-#define AMT_TILE(TWO, SHAPE) \
-  launch_tile<R, TWO, SHAPE>(op, grid, s, m, n, k, kchunk, ns, a, lda, sa, b, ldb, sb, c, ldc, sc, alpha, beta, p)
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, m, n, k, kchunk, ns, (const C*)a, lda, sa, (const C*)b, ldb, sb,
+                       (C*)c, ldc, sc, (R)alpha, (R)beta, p, mfast);
+  };
+#define AMT_W(TWO, W)                \
+  case W:                            \
+    if (op == 0)                     \
+      launch(k_zgemm<R, 0, TWO, W>); \
+    else                             \
+      launch(k_zgemm<R, 1, TWO, W>); \
+    break;
   if constexpr (std::is_same<R, float>::value) {
-    if (g.tm == 2)
-      AMT_TILE(false, 2);
-    else if (kchunk > kLongChunk)
-      g.tm == kTall ? AMT_TILE(true, kTall) : AMT_TILE(true, 1);
-    else
-      g.tm == kTall ? AMT_TILE(false, kTall) : AMT_TILE(false, 1);
+    if (g.two) {
+      switch (g.w) { AMT_W(true, 1) AMT_W(true, 2) AMT_W(true, 3) AMT_W(true, 4) AMT_W(true, 5) }
+    } else {
+      switch (g.w) {
+        AMT_W(false, 1) AMT_W(false, 2) AMT_W(false, 3) AMT_W(false, 4) AMT_W(false, 5) AMT_W(false, 6)
+        AMT_W(false, 7)
+      }
+    }
   } else {
-    g.tm == kTall ? AMT_TILE(false, kTall) : AMT_TILE(false, 1);
+    switch (g.w) { AMT_W(false, 1) AMT_W(false, 2) AMT_W(false, 3) AMT_W(false, 4) AMT_W(false, 5) }
   }
-#undef AMT_TILE
+#undef AMT_W
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error(std::string("zgemm launch: ") + hipGetErrorString(e));

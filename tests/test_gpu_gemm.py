@@ -137,3 +137,39 @@ def test_zgemm_fp32_large_tiles_long_contraction():
     # rounding is bounded by eps * sum |a_re + a_im| |b_re + b_im|, up to twice the bound of
     # four real products (measured 1.1e-6 here; the four-product form passed 1e-6)
     assert float((got - want).abs().max() / want.abs().max()) < 2e-6
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("m", [1, 15, 17, 33, 48, 65, 80, 97, 112, 113, 160])
+def test_zgemm_tile_edges(dtype, m):
+    """Every tile height (16 to 112 rows) with one row more or less, against numpy in FP64 on the
+    same inputs: columns around the 64 of a tile and the two of an FP32 chunk, K around one, two
+    and four K tiles (8 or 16) and past the length that carries FP64 sums, row strides that leave
+    rows 8-byte aligned. The bound is the summation's own: with u the unit roundoff, a sum of k
+    products in one accumulator is off by at most (k + 8) u times the sum of the magnitudes, in the
+    three-product form at most three times that (an FP32 accumulator covers at most 1024 of k). A
+    NaN in the last row of A stays in the last row of the product."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    u = 2.0**-53 if dtype == "complex128" else 2.0**-24
+    dt = getattr(torch, dtype)
+    for n in (1, 2, 63, 64, 65, 131):
+        for k in (1, 7, 8, 9, 16, 17, 33, 64, 127, 1027, 2051):
+            big = torch.from_numpy(_c((m, k + 3), m + k)).to(dt)
+            bnn, bnc = torch.from_numpy(_c((k, n + 1), n)).to(dt), torch.from_numpy(_c((n, k + 1), n + 7)).to(dt)
+            a = big[:, 1 : 1 + k]
+            for op, b in ((0, bnn[:, :n]), (1, bnc[:, :k])):
+                dev = [x.cuda() for x in (big, bnn if op == 0 else bnc)]
+                da, db = dev[0][:, 1 : 1 + k], dev[1][:, :n] if op == 0 else dev[1][:, :k]
+                got = ops.zgemm(da, db, op).cpu().to(torch.complex128).numpy()
+                x, y = a.to(torch.complex128).numpy(), b.to(torch.complex128).numpy()
+                y = y if op == 0 else y.conj().T
+                size = (np.abs(x.real) + np.abs(x.imag)) @ (np.abs(y.real) + np.abs(y.imag))
+                assert (np.abs(got - x @ y) <= 3.0 * (min(k, 1024) + 8) * u * size).all(), (n, k, op)
+        if m > 1:
+            bad = dev[0].clone()
+            bad[-1] = float("nan")
+            got = ops.zgemm(bad[:, 1 : 1 + k], db, op)
+            assert bool(torch.isfinite(torch.view_as_real(got[:-1])).all()) and bool(got[-1].isnan().all())
