@@ -94,7 +94,7 @@ def tune_zgemm(run, prec: int, op: int, m: int, n: int, k: int, batch: int) -> i
 
 
 # ----------------------------------------------------------------------- FFT launch shapes
-#: (grid length, precision) -> (plane workgroup, sticks per workgroup) chosen so far
+#: (length of a cubic grid or shape, precision) -> (plane workgroup, sticks per workgroup) chosen so far
 _FFT: dict = {}
 
 
@@ -135,7 +135,8 @@ def tune_fft_launch(plan, prec: int, psi: torch.Tensor, v: torch.Tensor, k0: int
     (length, precision) and applied to later plans of that length without timing again. The
     result of H.psi does not depend on it (every stick and plane is transformed by the same
     arithmetic whatever the grouping)."""
-    key = (plan.shape[0], prec)
+    n1, n2, n3 = plan.shape
+    key = (n1 if n1 == n2 == n3 else plan.shape, prec)
     info = plan.info
     if key not in _FFT:
         info[12 + prec] = info[14 + prec] = -1  # the timing below leaves the plan on its last candidate

@@ -126,6 +126,18 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
     delete h;
     return 1;
   }
+  // The compile-time-length kernels work in axes (stick axis, plane, plane): the first choice that
+  // makes the plane square. Cubic grids keep their order.
+  const int orders[3][3] = {{0, 1, 2}, {1, 0, 2}, {2, 0, 1}};
+  for (const auto& o : orders) {
+    if (p.fast || dims[o[1]] != dims[o[2]] || !fast_length_supported(dims[o[0]]) || !fast_length_supported(dims[o[1]]))
+      continue;
+    p.fast = true;
+    for (int a = 0; a < 3; ++a) p.axis[a] = o[a];
+    p.permuted = o[0] != 0;
+  }
+  const int q1 = p.dim(0), q2 = p.dim(1), q3 = p.dim(2);  // lengths along the plan's axes
+  bool narrow = p.fast;
   p.npw.assign(npw, npw + nk);
   for (int k = 0; k < nk; ++k) {
     if (npw[k] <= 0 || npw[k] > npw_pad) {
@@ -155,17 +167,19 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
         return 1;
       }
     }
+    if (std::max(hmax[p.axis[1]], hmax[p.axis[2]]) > lane_plane_half_width(q2)) narrow = false;
     std::vector<int> colid(n), ii(n);
     std::vector<int> cols;
     cols.reserve(n);
     for (int g = 0; g < n; ++g) {
       const int* m = miller + 3 * (off + g);
       const int i = ((m[0] % n1) + n1) % n1, j = ((m[1] % n2) + n2) % n2, kk = ((m[2] % n3) + n3) % n3;
-      ii[g] = i;
-      colid[g] = j * n3 + kk;
+      const int at[3] = {i, j, kk}, col = at[p.axis[1]] * q3 + at[p.axis[2]];
+      ii[g] = at[p.axis[0]];
+      colid[g] = col;
       flat[(size_t)k * npw_pad + g] = (int)(((long long)i * n2 + j) * n3 + kk);
       kin64[(size_t)k * npw_pad + g] = kinetic[off + g];
-      cols.push_back(j * n3 + kk);
+      cols.push_back(col);
     }
     std::sort(cols.begin(), cols.end());
     cols.erase(std::unique(cols.begin(), cols.end()), cols.end());
@@ -180,12 +194,12 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
   p.smax = smax;
   p.nsticks.resize(nk);
   std::vector<int> jk((size_t)nk * smax, -1);
-  std::vector<int> smap((size_t)nk * n1 * smax, -1);
+  std::vector<int> smap((size_t)nk * q1 * smax, -1);
   for (int k = 0; k < nk; ++k) {
     p.nsticks[k] = (int)sticks[k].size();
     for (int s = 0; s < p.nsticks[k]; ++s) jk[(size_t)k * smax + s] = sticks[k][s];
     for (int g = 0; g < npw[k]; ++g) {
-      int& slot = smap[((size_t)k * n1 + ipos[k][g]) * smax + stick_of[k][g]];
+      int& slot = smap[((size_t)k * q1 + ipos[k][g]) * smax + stick_of[k][g]];
       if (slot != -1) {
         set_error("plan_create: two plane waves map to one grid point");
         delete h;
@@ -195,32 +209,32 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
     }
   }
   // rows j (plane index along axis 1) that hold at least one stick, per k
-  std::vector<int> rows((size_t)nk * n2, 0), nrows(nk, 0);
+  std::vector<int> rows((size_t)nk * q2, 0), nrows(nk, 0);
   for (int k = 0; k < nk; ++k) {
-    std::vector<char> used(n2, 0);
-    for (int v : sticks[k]) used[v / n3] = 1;
-    for (int j = 0; j < n2; ++j)
-      if (used[j]) rows[(size_t)k * n2 + nrows[k]++] = j;
+    std::vector<char> used(q2, 0);
+    for (int v : sticks[k]) used[v / q3] = 1;
+    for (int j = 0; j < q2; ++j)
+      if (used[j]) rows[(size_t)k * q2 + nrows[k]++] = j;
   }
-  p.fast = (n1 == n2 && n2 == n3 && fast_length_supported(n1));
+  p.narrow = narrow;
   // per-row stick masks and first-stick indices for the compile-time plane kernels
   std::vector<unsigned long long> rowmask, livemask;
   std::vector<int> rowstart;
-  if (n2 <= 128 && n3 <= 128) {
-    rowmask.assign((size_t)nk * n2 * 2, 0ull);
-    rowstart.assign((size_t)nk * n2, 0);
+  if (q2 <= 128 && q3 <= 128) {
+    rowmask.assign((size_t)nk * q2 * 2, 0ull);
+    rowstart.assign((size_t)nk * q2, 0);
     livemask.assign((size_t)nk * 2, 0ull);
     for (int k = 0; k < nk; ++k) {
-      std::vector<int> count(n2, 0);
+      std::vector<int> count(q2, 0);
       for (int v : sticks[k]) {
-        const int j = v / n3, kk = v % n3;
-        rowmask[((size_t)k * n2 + j) * 2 + (kk >> 6)] |= 1ull << (kk & 63);
+        const int j = v / q3, kk = v % q3;
+        rowmask[((size_t)k * q2 + j) * 2 + (kk >> 6)] |= 1ull << (kk & 63);
         livemask[(size_t)k * 2 + (j >> 6)] |= 1ull << (j & 63);
         ++count[j];
       }
       int run = 0;
-      for (int j = 0; j < n2; ++j) {
-        rowstart[(size_t)k * n2 + j] = run;
+      for (int j = 0; j < q2; ++j) {
+        rowstart[(size_t)k * q2 + j] = run;
         run += count[j];
       }
     }
@@ -242,14 +256,18 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
     int pt = std::max(threads_needed(p.ap[2], n2, tpt), threads_needed(p.ap[1], n3, tpt));
     pt = ((pt + 63) / 64) * 64;
     if (pt < 64) pt = 64;
-    const long long plds = (long long)n2 * n3 * csz;
+    const long long plds = (long long)q2 * q3 * csz;
     // 0 marks a precision whose plane does not fit one workgroup on this device. The
     // compile-time-length kernels use a fixed 256-thread workgroup (512 for the density)
     // and add the row lists, first-stick indices and 128-bit stick masks (24 n2 bytes).
-    if (p.fast)
-      p.plane_threads[prec] = (plds + 24LL * n2 <= lds_max) ? 256 : 0;
-    else
+    // The one-lane kernel (narrow plans) holds the rows with sticks only and needs neither.
+    if (p.fast) {
+      p.whole_plane[prec] = plds + 24LL * q2 <= lds_max;
+      p.plane_threads[prec] = p.whole_plane[prec] || (narrow && lane_plane_supported(q2, prec)) ? 256 : 0;
+    } else {
       p.plane_threads[prec] = (pt <= 1024 && plds <= lds_max) ? pt : 0;
+      p.whole_plane[prec] = p.plane_threads[prec] > 0;
+    }
   }
   p.plane_fit[0] = p.plane_threads[0];
   p.plane_fit[1] = p.plane_threads[1];
@@ -316,7 +334,7 @@ int amt_plan_set_launch(amt_plan_t* h, int precision, int plane_threads, int sti
   }
   Plan& p = h->p;
   if (!p.fast) {
-    set_error("plan_set_launch: only the compile-time-length kernels of cubic grids have these launch shapes");
+    set_error("plan_set_launch: only the compile-time-length kernels (two axes of one length) have these launch shapes");
     return 1;
   }
   const int wdef = precision == kFP64 ? 32 : 64;
@@ -340,16 +358,19 @@ int amt_plan_nsticks(const amt_plan_t* h, int* out) {
   return 0;
 }
 
-// Bytes of the local H.psi / density workspace for `rows` band rows: their sticks, or, where
-// the plane does not fit LDS (full-grid route), whole grids for min(rows, ~1 GiB of grids).
+// Bytes of the local H.psi / density workspace for `rows` band rows: their sticks (and V_eff in
+// the plan's axes), or, where the plane does not fit LDS (full-grid route), whole grids for
+// min(rows, ~1 GiB of grids).
 static size_t local_ws_bytes(const Plan& p, int prec, long long rows) {
   if (rows <= 0 || (prec != kFP32 && prec != kFP64)) return 0;
   const size_t elem = prec == kFP64 ? 16 : 8;
-  if (p.plane_threads[prec] > 0) return (size_t)rows * p.n1 * p.smax * elem;
+  const size_t sticks = p.plane_threads[prec] > 0 ? p.field_bytes(prec) + (size_t)rows * p.dim(0) * p.smax * elem : 0;
+  if (sticks > 0 && p.whole_plane[prec]) return sticks;
   const size_t grid = (size_t)p.n1 * p.n2 * p.n3 * elem;
   long long g = (long long)((size_t(1) << 30) / grid);
   if (g < 1) g = 1;
-  return (size_t)(rows < g ? rows : g) * grid;
+  const size_t grids = (size_t)(rows < g ? rows : g) * grid;  // the density takes them where only H.psi has a kernel
+  return sticks > grids ? sticks : grids;
 }
 
 size_t amt_plan_stick_bytes(const amt_plan_t* h, int precision, int nbands) {
@@ -367,12 +388,12 @@ int amt_plan_set_route(amt_plan_t* h, int precision, int full_grid) {
   return 0;
 }
 
-static int check_plane(const Plan& p, int prec) {
+static int check_plane(const Plan& p, int prec, bool whole = false) {
   if (prec != kFP32 && prec != kFP64) {
     set_error("precision must be 0 (fp32) or 1 (fp64)");
     return 1;
   }
-  if (p.plane_threads[prec] == 0) {
+  if (p.plane_threads[prec] == 0 || (whole && !p.whole_plane[prec])) {
     set_error("the " + std::to_string(p.n2) + "x" + std::to_string(p.n3) + " plane does not fit one workgroup's LDS at " +
               (prec == kFP64 ? "fp64" : "fp32"));
     return 1;
@@ -507,7 +528,7 @@ int amt_hpsi_local_noalloc(const amt_plan_t* h, int precision, const void* psi, 
     return 1;
   }
   const Plan& p = h->p;
-  if (check_plane(p, precision)) return 1;
+  if (check_plane(p, precision, true)) return 1;
   if (nb <= 0 || nkk <= 0 || k0 < 0 || k0 + nkk > p.nk) {
     set_error("hpsi_local_noalloc: band/k range outside the plan");
     return 1;
@@ -556,7 +577,7 @@ int amt_density(const amt_plan_t* h, int precision, const void* psi, int nb, int
     set_error("density: band/k range outside the plan");
     return 1;
   }
-  if (p.plane_threads[precision] == 0)
+  if (p.plane_threads[precision] == 0 || !p.whole_plane[precision])
     return launch_density_full_grid(p, precision, psi, nb, k0, band_list, band_weight, nlist, sticks,
                                     local_ws_bytes(p, precision, (long long)nb * nkk), part, rho, beta, scale,
                                     (hipStream_t)stream);

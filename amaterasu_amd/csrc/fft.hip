@@ -296,6 +296,18 @@ __global__ void k_density_plane(const C* __restrict__ sticks, const int* __restr
   }
 }
 
+// rho at the plan's axes (i, r, c) of a permuted plan from part in their order
+__global__ void k_density_reduce_permuted(const double* __restrict__ part, int nchunk, long long ngrid, int m2, int m3,
+                                          long long s1, long long s2, long long s3, double* __restrict__ rho,
+                                          double beta, double scale) {
+  const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= ngrid) return;
+  double s = 0.0;
+  for (int c = 0; c < nchunk; ++c) s += part[(long long)c * ngrid + p];
+  double* r = rho + p / ((long long)m2 * m3) * s1 + p / m3 % m2 * s2 + p % m3 * s3;
+  *r = (beta == 0.0 ? 0.0 : beta * *r) + scale * s;
+}
+
 __global__ void k_density_reduce(const double* __restrict__ part, int nchunk, long long ngrid,
                                  double* __restrict__ rho, double beta, double scale) {
   const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -462,8 +474,12 @@ static int density_t(const Plan& p, const void* psi_, int nb, int k0, int nkk, c
                        chunk, p.n1, p.n2, p.n3, p.smax, nb, k0, p.ap[1], p.ap[2], tw[1], tw[2], part);
     if (check(hipGetLastError(), "density_plane launch")) return 1;
   }
-  hipLaunchKernelGGL(k_density_reduce, dim3((unsigned)((ngrid + 255) / 256)), dim3(256), 0, s, part, nchunk,
-                     ngrid, rho, beta, scale);
+  const dim3 rgrid((unsigned)((ngrid + 255) / 256));
+  if (p.permuted)
+    hipLaunchKernelGGL(k_density_reduce_permuted, rgrid, dim3(256), 0, s, part, nchunk, ngrid, p.dim(1), p.dim(2),
+                       p.stride(0), p.stride(1), p.stride(2), rho, beta, scale);
+  else
+    hipLaunchKernelGGL(k_density_reduce, rgrid, dim3(256), 0, s, part, nchunk, ngrid, rho, beta, scale);
   return check(hipGetLastError(), "density_reduce launch");
 }
 
@@ -471,7 +487,7 @@ int launch_density(const Plan& p, int prec, const void* psi, int nb, int k0, int
                    const double* weight, int nlist, int chunk, void* sticks, double* part, double* rho, double beta,
                    double scale, hipStream_t s) {
   const int maxpts = prec == kFP64 ? density_max_pts<double>() : density_max_pts<float>();
-  if ((p.n2 * p.n3 + maxpts - 1) / maxpts > 1024) {
+  if (!p.fast && (p.n2 * p.n3 + maxpts - 1) / maxpts > 1024) {
     set_error("density: plane too large for the register accumulator");
     return 1;
   }

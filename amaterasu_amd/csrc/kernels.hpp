@@ -47,7 +47,20 @@ struct Plan {
   unsigned long long* d_rowmask = nullptr;  // [nk][n2][2]
   int* d_rowstart = nullptr;                // [nk][n2]
   unsigned long long* d_livemask = nullptr; // [nk][2]: rows j that hold sticks (n2 <= 128)
-  bool fast = false;           // cubic grid of a length with compile-time kernels
+  // Compile-time-length kernels: the plan's own axes are axis[0] (along the sticks), axis[1] and
+  // axis[2] (the plane, of one length); d_stick_*, d_rows, row masks and V_eff inside the kernels
+  // are in that order. Axes other than 0, 1, 2 make it `permuted`; every other plan keeps them.
+  bool fast = false;
+  int axis[3] = {0, 1, 2};
+  bool permuted = false;
+  bool narrow = false;         // plane-axis Miller indices within lane_plane_half_width
+  int length(int natural) const { return natural == 0 ? n1 : natural == 1 ? n2 : n3; }
+  int dim(int a) const { return length(axis[a]); }
+  long long stride(int a) const { return axis[a] == 0 ? (long long)n2 * n3 : axis[a] == 1 ? n3 : 1; }
+  // V_eff in the plan's axes, at the start of the local workspace of a permuted plan
+  size_t field_bytes(int prec) const {
+    return permuted ? ((size_t)n1 * n2 * n3 * (prec == kFP64 ? 8 : 4) + 255) / 256 * 256 : 0;
+  }
   double* d_kin64 = nullptr;   // [nk][npw_pad] |k+G|^2/2 (0 on padding)
   float* d_kin32 = nullptr;
   double2* d_tw64[3] = {nullptr, nullptr, nullptr};
@@ -65,6 +78,7 @@ struct Plan {
   int stick_threads[2] = {0, 0};   // workgroup size of the stick kernels
   int plane_threads[2] = {0, 0};   // workgroup size of the plane kernel (0: full-grid route)
   int plane_fit[2] = {0, 0};       // the plane kernel's size where it fits (amt_plan_set_route restores it)
+  bool whole_plane[2] = {false, false};  // a whole plane fits LDS: density kernel and allocation-free call
   // launch shapes of the compile-time-length kernels (amt_plan_set_launch; an autotuner picks them)
   int plane_nth[2] = {256, 256};   // plane kernel workgroup: 256 or 512 threads
   int fast_stick_w[2] = {64, 32};  // sticks per workgroup of the stick kernels: the default or half
@@ -72,8 +86,10 @@ struct Plan {
 
 void set_error(const std::string& msg);
 
-// Compile-time-length kernels (fft_fast.hip) for cubic grids of the listed lengths.
+// Compile-time-length kernels (fft_fast.hip) for grids with two axes of one listed length.
 bool fast_length_supported(int n);
+bool lane_plane_supported(int n, int prec);
+int lane_plane_half_width(int n);
 int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
                      const void* veff, void* sticks, hipStream_t s, int stage);
 int launch_density_fast(const Plan& p, int prec, const void* psi, int nb, int k0, int nkk, const int* list,

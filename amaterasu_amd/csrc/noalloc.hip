@@ -55,9 +55,9 @@ static void* scratch_on_current_device() {
 
 // Band rows whose stick workspace fits the scratch array in one launch (0: not even one).
 long long noalloc_rows_per_launch(const Plan& p, int prec) {
-  const long long row_bytes = (long long)p.n1 * p.smax * (prec == kFP64 ? 16 : 8);
+  const long long row_bytes = (long long)p.dim(0) * p.smax * (prec == kFP64 ? 16 : 8);
   if (row_bytes <= 0) return 0;
-  const long long rows = (long long)AMT_NOALLOC_SCRATCH_BYTES / row_bytes;
+  const long long rows = ((long long)AMT_NOALLOC_SCRATCH_BYTES - (long long)p.field_bytes(prec)) / row_bytes;
   return rows < 65535 ? rows : 65535;
 }
 
@@ -68,7 +68,7 @@ int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int
                        const void* veff, hipStream_t s) {
   const long long rows_max = noalloc_rows_per_launch(p, prec);
   if (rows_max < 1) {
-    const long long row_bytes = (long long)p.n1 * p.smax * (prec == kFP64 ? 16 : 8);
+    const long long row_bytes = (long long)p.dim(0) * p.smax * (prec == kFP64 ? 16 : 8);
     set_error("hpsi_local_noalloc: one band row needs " + std::to_string(row_bytes) +
               " bytes of stick workspace, more than the fixed scratch of " +
               std::to_string((long long)AMT_NOALLOC_SCRATCH_BYTES) + " bytes; use amt_hpsi_local with a workspace");

@@ -50,7 +50,7 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
 int amt_plan_destroy(amt_plan_t* plan);
 /* info[0..15] = n1, n2, n3, nk, npw_pad, smax, stick_w{fp32,fp64}, stick_threads{fp32,fp64},
  * plane_threads{fp32,fp64} (0 = plane does not fit LDS at that precision: full-grid route),
- * and for cubic grids with compile-time-length kernels (else 0) the launch shapes of
+ * and for grids with compile-time-length kernels (else 0) the launch shapes of
  * amt_plan_set_launch: plane workgroup{fp32,fp64}, sticks per workgroup{fp32,fp64}. */
 int amt_plan_info(const amt_plan_t* plan, int* info, int len);
 /* Tuning hook, no counterpart in the reference: the launch shape of the compile-time-length

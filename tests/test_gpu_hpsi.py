@@ -307,3 +307,42 @@ def test_launch_shapes_give_identical_results(si_pseudo, precision):
         assert torch.equal(o, outs[0])
     with pytest.raises(AmtError, match="plane_threads must be"):
         check(lib().amt_plan_set_launch(plan.handle, prec, 384, 0), "plan_set_launch")
+
+
+@pytest.mark.parametrize("shape", [(21, 21, 21), (24, 24, 24), (45, 45, 45), (60, 60, 60), (63, 63, 63), (72, 72, 72),
+                                   (84, 84, 84), (100, 100, 100), (108, 108, 108), (128, 128, 128),
+                                   (24, 33, 33), (33, 24, 33), (33, 33, 24), (84, 20, 84), (20, 84, 84), (27, 108, 108)])
+def test_plane_kernels_match_full_grid_route(shape):
+    """Every plane kernel (one and four lanes per row, four-step) and every order of a grid with two
+    equal axes, against the library's full-grid route on the same plan: H.psi and density of two
+    ragged k-points, for spheres of the usual half width of the grid and for wide ones that reach
+    past it (which the one-lane kernel leaves to the others). Bounds: a transform pair over N
+    points is off by about log2(N) unit roundoffs of the largest value; 64 of them are allowed."""
+    import torch
+
+    from amaterasu_amd._lib import FP32, FP64
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    cell = np.diag(np.array(shape) / 4.0)
+    g = torch.Generator(device="cuda").manual_seed(sum(shape))
+    n = min(shape)
+    for half in (n / 4.0 - 0.4, min(n / 4.0 + 3.0, n / 2.0 - 2.0)):
+        ecut = 0.5 * (half * 2.0 * np.pi / (n / 4.0)) ** 2
+        spheres = [GSphere.build(cell, ecut * f, kpoint=np.array(k)) for f, k in ((1.0, (0, 0, 0)), (0.9, (0.4, -0.3, 0.1)))]
+        nb = 3
+        for prec, dt, u in ((FP32, torch.complex64, 2.0**-24), (FP64, torch.complex128, 2.0**-53)):
+            plan = DevicePlan(shape, spheres)
+            psi = torch.randn((2, nb, plan.npw_pad), dtype=dt, device="cuda", generator=g)
+            for k in range(2):
+                psi[k, :, plan.npw[k]:] = 0
+            v = torch.randn(shape, dtype=torch.float64, device="cuda", generator=g)
+            rows, weights = np.array([0, 2, 3, 5]), np.array([1.0, 0.5, 2.0, 0.25])
+            got, rho = plan.hpsi(psi, v), torch.ones(shape, dtype=torch.float64, device="cuda")
+            plan.accumulate_density(psi, rows, weights, rho, beta=0.5, scale=0.1, chunk=3)
+            plan.set_route(prec, True)
+            want, rho_want = plan.hpsi(psi, v), torch.ones(shape, dtype=torch.float64, device="cuda")
+            plan.accumulate_density(psi, rows, weights, rho_want, beta=0.5, scale=0.1, chunk=3)
+            bound = 64 * u * np.log2(np.prod(shape))
+            assert float((got - want).abs().max() / want.abs().max()) < bound, (half, prec)
+            assert float((rho - rho_want).abs().max() / rho_want.abs().max()) < bound, (half, prec)
