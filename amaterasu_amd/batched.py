@@ -29,7 +29,7 @@ import numpy as np
 import torch
 
 from . import ops
-from .eigen import _lowest_eigenpairs, orthonormalize
+from .eigen import NAN_SILENT, _lowest_eigenpairs, orthonormalize, raise_not_finite
 
 
 @dataclass
@@ -249,7 +249,10 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
             out_norm = norms
         else:
             out_norm[torch.as_tensor(running, device=dev)] = norms[torch.as_tensor(running, device=dev)]
-        active = (norms > tolerance).cpu().numpy() & running[:, None]
+        flags = torch.stack([norms > tolerance, torch.isnan(norms)]).cpu().numpy()  # one device read
+        active = flags[0] & running[:, None]
+        if (flags[1].any(axis=1) & running & (m < NAN_SILENT)).any():
+            raise_not_finite()
         finished = running & ~active.any(axis=1)
         running &= ~finished
         if not running.any():

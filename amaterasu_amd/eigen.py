@@ -451,6 +451,8 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
         norms = next_norms if sg is None else next_norms.clone()
         active = torch.nonzero(norms > tolerance).flatten()
         if active.numel() == 0:
+            if m < NAN_SILENT and bool(torch.isnan(norms).any()):
+                raise_not_finite()
             break
         corr = ops.precondition(res, vec, kin, active, rows_checked=True)  # rows of nonzero(norms)
         new = orthogonalize_against(corr, basis[:m], overwrite=True)
@@ -479,10 +481,20 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
     return DavidsonResult(eps, vec, norms, iteration, converged)
 
 
-#: Projected matrices at least this large go to the library's own Hermitian eigensolver
-#: (device tridiagonalisation); smaller ones to torch.linalg.eigh.
-HEEV_MIN = 96
+#: Projected matrices of these sizes go to the library's own Hermitian eigensolver (device
+#: tridiagonalisation), the others to torch.linalg.eigh (rocSOLVER zheevd). Measured on MI355X (us,
+#: lowest quarter or more of the spectrum, library against zheevd): 8 93/220, 20 128/542, 40
+#: 190/1061, 60 248/1761, 80 337/1559, 128 559/3052, 320 1558/9360.
+HEEV_MIN = 2
 HEEV_MAX = 2048
+
+#: zheevd reports a matrix that is not finite, the library's solver returns NaN: below this size,
+#: where zheevd used to be the solver, the iteration raises its error when it finds NaN residuals.
+NAN_SILENT = 96
+
+
+def raise_not_finite():
+    raise torch.linalg.LinAlgError("davidson: the projected matrix contains non-finite values")
 
 
 def _lowest_eigenpairs(proj: torch.Tensor, nbands: int, workspace_tag: str = "heev"):

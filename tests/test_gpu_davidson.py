@@ -154,3 +154,35 @@ def test_orthonormalisation_refinement_and_its_fallback(monkeypatch, dtype, cond
     monkeypatch.undo()
     monkeypatch.setattr(eigen, "_cholesky_orthonormalize", lambda v: calls.append(1) or second(v))
     check(block_of(cond_hard), None)
+
+
+@pytest.mark.parametrize("nb", [1, 2, 5, 20])
+def test_small_projected_matrices(nb):
+    """Projected matrices of 1 to 80 rows (the library's eigensolver from 2 on) in the per-k and the
+    k-batched iteration, against the dense eigenvalues of the operator; an operator that is not
+    finite raises, as zheevd did. Bound: residual norms below 1e-8 put an eigenvalue within 1e-8
+    of the spectrum, and well within it by the gap (Weyl); 1e-8 is asserted."""
+    import torch
+
+    from amaterasu_amd.batched import solve_batched
+    from amaterasu_amd.eigen import davidson
+
+    n, nk = 300, 2
+    g = torch.Generator(device="cuda").manual_seed(nb)
+    kin = torch.linspace(0.1, 30.0, n, dtype=torch.float64, device="cuda").repeat(nk, 1)
+    a = 0.05 * torch.randn((nk, n, n), dtype=torch.complex128, device="cuda", generator=g)
+    a = (a + a.mH) / 2 + torch.diag_embed(kin.to(torch.complex128))
+    guess = torch.randn((nk, nb, n), dtype=torch.complex128, device="cuda", generator=g) / (1 + kin[:, None, :])
+    want = torch.stack([torch.linalg.eigvalsh(a[k].cpu()) for k in range(nk)])[:, :nb]
+    each = [davidson(lambda x, k=k: x @ a[k].T.contiguous(), guess[k], kin[k], tolerance=1e-8, max_iterations=60)
+            for k in range(nk)]
+    both = solve_batched(lambda x: torch.stack([x[k] @ a[k].T.contiguous() for k in range(nk)]), guess, kin, [n] * nk,
+                         tolerance=1e-8, max_iterations=60)
+    for k in range(nk):
+        assert each[k].converged and bool(both.converged[k])
+        assert float((each[k].eigenvalues.cpu() - want[k]).abs().max()) < 1e-8
+        assert float((both.eigenvalues[k].cpu() - want[k]).abs().max()) < 1e-8
+    with pytest.raises(torch.linalg.LinAlgError):
+        davidson(lambda x: x * float("nan"), guess[0], kin[0], tolerance=1e-8, max_iterations=3)
+    with pytest.raises(torch.linalg.LinAlgError):
+        solve_batched(lambda x: x * float("nan"), guess, kin, [n] * nk, tolerance=1e-8, max_iterations=3)
