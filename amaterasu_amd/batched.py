@@ -72,7 +72,11 @@ def _pad_diag(m: torch.Tensor, used: torch.Tensor, value: float, step: float = 0
 
 def _cholesky_rows(block: torch.Tensor, used: torch.Tensor):
     """L^{-1} block per k (rows >= used[k] are zero and stay zero); None where it fails."""
-    s = _pad_diag(_herm(_bgram(block, block)), used, 1.0)
+    s = _bgram(block, block)
+    if 0 < s.shape[-1] <= ops.CHOL_MAX:
+        linv, stats = ops.chol_inverse(s, used.to(torch.int32))
+        return _brot(linv, block), stats[:, 0]
+    s = _pad_diag(_herm(s), used, 1.0)
     low, info = torch.linalg.cholesky_ex(s)
     eye = torch.eye(s.shape[-1], dtype=s.dtype, device=s.device).repeat(s.shape[0], 1, 1)
     linv = torch.linalg.solve_triangular(low, eye, upper=False)
@@ -104,27 +108,38 @@ def _eigh(m: torch.Tensor, used, fill: float):
     return torch.gather(w, 1, order), torch.gather(u, 2, order[:, None, :].expand(-1, n, -1))
 
 
+def _keep_rows(v: torch.Tensor, used: torch.Tensor):
+    """The second Cholesky pass over rows that are all kept."""
+    again, info = _cholesky_rows(v, used)
+    return torch.where((info == 0)[:, None, None], again, v), used
+
+
 def _gram_rows(block: torch.Tensor, used: torch.Tensor, threshold: float):
     """Per k: keep directions with singular value > threshold * s_max, orthonormal
     (the routes of ``eigen.orthogonalize_against``). Returns (rows, kept)."""
-    g = _herm(_bgram(block, block))
-    gp = _pad_diag(g.clone(), used, 1.0)
-    low, info = torch.linalg.cholesky_ex(gp)
-    eye = torch.eye(g.shape[-1], dtype=g.dtype, device=g.device).repeat(g.shape[0], 1, 1)
-    linv = torch.linalg.solve_triangular(low, eye, upper=False)
-    # the padded identity block adds at most sqrt(pad) to both Frobenius norms; use the
-    # used block alone: zero the padded rows/cols before measuring
-    n = g.shape[-1]
-    live = (torch.arange(n, device=g.device)[None, :] < used[:, None]).to(g.dtype)
-    mask = live[:, :, None] * live[:, None, :]
-    lo = 1.0 / torch.linalg.matrix_norm(linv * mask)
-    hi = torch.linalg.matrix_norm(low * mask)
-    ok = (used == 0) | ((info == 0) & torch.isfinite(lo) & (lo > threshold * hi))
-    if bool(ok.all().item()):
-        v = _brot(linv, block)
-        again, info2 = _cholesky_rows(v, used)
-        good = info2 == 0
-        return torch.where(good[:, None, None], again, v), used
+    raw = _bgram(block, block)
+    if 0 < raw.shape[-1] <= ops.CHOL_MAX:
+        linv, stats = ops.chol_inverse(raw, used.to(torch.int32))
+        lo, hi = torch.rsqrt(stats[:, 2:].sum(1)), torch.sqrt(stats[:, 1])  # 1/||L^{-1}||_F, ||L||_F of the used blocks
+        ok = (used == 0) | ((stats[:, 0] == 0) & torch.isfinite(lo) & (lo > threshold * hi))
+        if bool(ok.all().item()):
+            return _keep_rows(_brot(linv, block), used)
+    g = _herm(raw)
+    if g.shape[-1] > ops.CHOL_MAX:
+        gp = _pad_diag(g.clone(), used, 1.0)
+        low, info = torch.linalg.cholesky_ex(gp)
+        eye = torch.eye(g.shape[-1], dtype=g.dtype, device=g.device).repeat(g.shape[0], 1, 1)
+        linv = torch.linalg.solve_triangular(low, eye, upper=False)
+        # the padded identity block adds at most sqrt(pad) to both Frobenius norms; use the
+        # used block alone: zero the padded rows/cols before measuring
+        n = g.shape[-1]
+        live = (torch.arange(n, device=g.device)[None, :] < used[:, None]).to(g.dtype)
+        mask = live[:, :, None] * live[:, None, :]
+        lo = 1.0 / torch.linalg.matrix_norm(linv * mask)
+        hi = torch.linalg.matrix_norm(low * mask)
+        ok = (used == 0) | ((info == 0) & torch.isfinite(lo) & (lo > threshold * hi))
+        if bool(ok.all().item()):
+            return _keep_rows(_brot(linv, block), used)
     # padded rows get negative eigenvalues: they sort last after the flip, and
     # s = sqrt(max(w, 0)) = 0 drops them
     w, u = _eigh(g, used, -1.0)

@@ -674,6 +674,34 @@ int amt_fft3d(const amt_fft_plan_t* h, int precision, int batch, void* data, int
   return launch_fft3d(h->f, precision, batch, data, sign, scale, (hipStream_t)stream);
 }
 
+constexpr int kCholMax = 512;
+
+size_t amt_chol_workspace(int n, int batch) {
+  return n < 1 || n > kCholMax || batch < 1 ? 0 : chol_workspace_bytes(n, batch);
+}
+
+int amt_chol_inverse(int precision, int n, const void* gram, const int* used, int batch, void* linv, double* stats,
+                     void* ws, size_t ws_bytes, void* stream) {
+  if (!gram || !linv || !stats || !ws || (precision != kFP32 && precision != kFP64) || n < 1 || n > kCholMax ||
+      batch < 1 || batch > 65535) {
+    set_error("chol_inverse: bad argument (1 <= n <= 512)");
+    return 1;
+  }
+  if (ws_bytes < chol_workspace_bytes(n, batch)) {
+    set_error("chol_inverse: workspace smaller than amt_chol_workspace()");
+    return 1;
+  }
+  return launch_chol_inverse(precision, n, gram, used, batch, linv, stats, ws, (hipStream_t)stream);
+}
+
+int amt_lowdin(int precision, int n, const void* gram, void* rot, double* emax, void* stream) {
+  if (!gram || !rot || !emax || (precision != kFP32 && precision != kFP64) || n < 1 || n > kCholMax) {
+    set_error("lowdin: bad argument (1 <= n <= 512)");
+    return 1;
+  }
+  return launch_lowdin(precision, n, gram, rot, emax, (hipStream_t)stream);
+}
+
 size_t amt_zgemm_workspace(int precision, int op, int m, int n, int k, int batch) {
   return zgemm_workspace_bytes(precision, op, m, n, k, batch);
 }

@@ -140,6 +140,13 @@ int set_zgemm_split(int prec, int op, int m, int n, int k, int batch, int split)
 size_t heev_workspace_bytes(int n);
 int launch_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws, size_t ws_bytes, hipStream_t s);
 
+// Inverse Cholesky factor of Gram matrices and the Loewdin series (chol.hip).
+int chol_blocks(int n);
+size_t chol_workspace_bytes(int n, int batch);
+int launch_chol_inverse(int prec, int n, const void* g, const int* used, int batch, void* linv, double* stats, void* ws,
+                        hipStream_t s);
+int launch_lowdin(int prec, int n, const void* g, void* rot, double* emax, hipStream_t s);
+
 // Learned starting density (mlp.hip).
 int mlp_param_count();
 int mlp_train_waves(long long npts);

@@ -5,7 +5,8 @@ Mirrors ``scf/eigen/__init__.py:31-46`` (``solve``), ``scf/eigen/davidson.py:48-
 ``scf/eigen/precond.py:27-46``. The block-sized work runs in libamaterasu_amd:
 residuals and the Teter-Payne-Allan step are fused kernels, every Gram/projected
 matrix and every rotation is an MFMA complex GEMM. The small dense factorisations
-(Cholesky, Hermitian eigensolve) stay in FP64 on the GPU (torch.linalg on ROCm).
+(Cholesky, Hermitian eigensolve) stay in FP64 on the GPU (amt_chol_inverse, amt_lowdin and
+amt_heev; torch.linalg on ROCm past their sizes).
 
 One step differs in method, not in result: ``orthogonalize_against`` orthonormalises
 the projected block by CholeskyQR2 when the Cholesky factor of its Gram matrix proves
@@ -82,7 +83,12 @@ def _cholesky_orthonormalize(block: torch.Tensor):
     """L^{-1} block with L L^H = block block^H; None if the Cholesky fails. One host
     synchronisation: the factorisation's status and the finiteness of L^{-1} (a finite
     L^{-1} times a finite block is finite) are read together."""
-    s = _hermitian(_gram(block, block))
+    s = _gram(block, block)
+    if 0 < s.shape[0] <= ops.CHOL_MAX:
+        linv, stats = ops.chol_inverse(s)
+        st = stats.cpu().numpy()
+        return _rotate(linv, block) if st[0] == 0 and np.isfinite(st[2:].sum()) else None
+    s = _hermitian(s)
     lower, info = torch.linalg.cholesky_ex(s)
     eye = torch.eye(s.shape[0], dtype=s.dtype, device=s.device)
     linv = torch.linalg.solve_triangular(lower, eye, upper=False)
@@ -101,7 +107,12 @@ def _lowdin_refine(v: torch.Tensor):
     the series (I + E)^{-1/2} = I - E/2 + 3 E^2 / 8, the second CholeskyQR pass's job without
     a factorisation; None (one host read, as the Cholesky status would need) when E is too
     large or not finite, and the caller factorises."""
-    g = _hermitian(_gram(v, v))
+    g = _gram(v, v)
+    if 0 < g.shape[0] <= ops.CHOL_MAX:
+        rot, emax = ops.lowdin(g)
+        err = float(emax.cpu().max())
+        return _rotate(rot, v) if err <= _LOWDIN_MAX[v.dtype] else None  # None also for NaN
+    g = _hermitian(g)
     eye = torch.eye(g.shape[0], dtype=g.dtype, device=g.device)
     e = g - eye
     rot = eye - 0.5 * e + 0.375 * (e @ e)
@@ -111,13 +122,20 @@ def _lowdin_refine(v: torch.Tensor):
     return _rotate(rot, v)
 
 
-def _cholesky_keeps_all(g: torch.Tensor, threshold: float):
-    """L^{-1} when the Cholesky factor proves that every singular value of the block
+def _cholesky_keeps_all(gram: torch.Tensor, threshold: float):
+    """L^{-1} of the raw product ``gram`` when the Cholesky factor proves that every singular value of the block
     exceeds ``threshold`` times the largest (then every direction is kept), else None.
 
     With G = B B^H = L L^H the singular values of B are those of L, and
     s_min(L) >= 1 / ||L^{-1}||_F, s_max(L) <= ||L||_F: the test is rigorous, not a guess.
     """
+    if 0 < gram.shape[0] <= ops.CHOL_MAX:
+        linv, stats = ops.chol_inverse(gram)
+        status, trace, *columns = stats.tolist()  # ||L||_F^2 is the trace of G
+        inv = sum(columns)
+        keep = status == 0 and inv > 0.0 and np.isfinite(inv) and inv**-0.5 > threshold * max(trace, 0.0) ** 0.5
+        return linv if keep else None
+    g = _hermitian(gram)
     lower, info = torch.linalg.cholesky_ex(g)
     eye = torch.eye(g.shape[-1], dtype=g.dtype, device=g.device)
     linv = torch.linalg.solve_triangular(lower, eye, upper=False)
@@ -136,15 +154,15 @@ def _gram_orthonormalize(block: torch.Tensor, threshold: float) -> torch.Tensor:
     right singular vectors come from the eigen-decomposition of the Gram matrix
     (descending, as an SVD orders them), followed by one CholeskyQR pass.
     """
-    g = _hermitian(_gram(block, block))
-    linv = _cholesky_keeps_all(g, threshold)
+    gram = _gram(block, block)
+    linv = _cholesky_keeps_all(gram, threshold)
     if linv is not None:
         v = _rotate(linv, block)
         again = _lowdin_refine(v)
         if again is None:
             again = _cholesky_orthonormalize(v)
         return v if again is None else again
-    w, u = torch.linalg.eigh(g)
+    w, u = torch.linalg.eigh(_hermitian(gram))
     w = torch.flip(w, dims=[0])
     u = torch.flip(u, dims=[1])
     s = torch.sqrt(torch.clamp(w, min=0.0))

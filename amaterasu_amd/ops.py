@@ -202,6 +202,49 @@ def precondition(res: torch.Tensor, v: torch.Tensor, kinetic: torch.Tensor, rows
     return out
 
 
+#: Gram matrices of at most this many rows go to the library's Cholesky and Loewdin kernels.
+CHOL_MAX = 512
+
+
+def _require_gram(gram: torch.Tensor):
+    _require(gram, "gram")
+    if gram.dtype not in (torch.complex64, torch.complex128) or gram.shape[-1] != gram.shape[-2]:
+        raise AmtError("gram must be square complex matrices")
+    if not 1 <= gram.shape[-1] <= CHOL_MAX:
+        raise AmtError(f"gram has {gram.shape[-1]} rows, outside 1..{CHOL_MAX}")
+
+
+def chol_inverse(gram: torch.Tensor, used: torch.Tensor | None = None):
+    """(L^{-1}, stats) of the Hermitian part L L^H of a raw product block block^H, or of a batch of
+    them with ``used`` (int32, device) leading rows each. See amt_chol_inverse: stats[..., 0] the
+    status, [..., 1] the trace, [..., 2:] sums of |L^{-1}|^2."""
+    _require_gram(gram)
+    n, batch = gram.shape[-1], gram.numel() // gram.shape[-1] ** 2
+    if used is not None and (used.dtype != torch.int32 or not used.is_cuda or used.numel() != batch):
+        raise AmtError("used must be one int32 per matrix on the device")
+    linv = torch.empty_like(gram)
+    stats = torch.empty((*gram.shape[:-2], (n + 31) // 32 + 2), dtype=torch.float64, device=gram.device)
+    nbytes = int(lib().amt_chol_workspace(n, batch))
+    ws = workspace(nbytes, "chol")
+    check(lib().amt_chol_inverse(precision_of(gram), n, gram.data_ptr(), None if used is None else used.data_ptr(),
+                                 batch, linv.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes, stream_handle()),
+          "chol_inverse")
+    return linv, stats
+
+
+def lowdin(gram: torch.Tensor):
+    """(I - E/2 + 3 E^2/8, largest |component| of E per 32 rows), E = (gram + gram^H)/2 - I."""
+    _require_gram(gram)
+    n = gram.shape[-1]
+    if gram.dim() != 2:
+        raise AmtError("lowdin: one matrix")
+    rot = torch.empty_like(gram)
+    emax = torch.empty((n + 31) // 32, dtype=torch.float64, device=gram.device)
+    check(lib().amt_lowdin(precision_of(gram), n, gram.data_ptr(), rot.data_ptr(), emax.data_ptr(), stream_handle()),
+          "lowdin")
+    return rot, emax
+
+
 def heev_lowest(a: torch.Tensor, nev: int, *, workspace_tag: str = "heev"):
     """Lowest ``nev`` eigenpairs of a Hermitian complex128 matrix on the device: (w, zt) with
     w ascending (float64) and zt[k] the k-th eigenvector (row). See amt_heev_lowest. Calls

@@ -210,6 +210,24 @@ size_t amt_heev_workspace(int n);
 int amt_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws, size_t ws_bytes, void* stream);
 
 /*
+ * Inverse Cholesky factor of the Gram matrices of orthonormalize / orthogonalize_against
+ * (scf/eigen/subspace.py:24-30, 53-60): gram holds `batch` raw n x n products block block^H of
+ * `precision` (1 <= n <= 512), whose Hermitian parts G = L L^H are factored in FP64; linv
+ * receives the n x n L^{-1} (zero above the diagonal). used (device, or null) gives each matrix's
+ * leading rows and columns in use: the others are taken as the identity. stats (device, float64)
+ * has ceil(n / 32) + 2 entries per matrix: 0 or the 1-based row of the first pivot that is not
+ * positive, the trace of the used part (= ||L||_F^2), and the sums of |L^{-1}|^2 over 32 columns
+ * each of the used part.
+ */
+size_t amt_chol_workspace(int n, int batch);
+int amt_chol_inverse(int precision, int n, const void* gram, const int* used, int batch, void* linv, double* stats,
+                     void* ws, size_t ws_bytes, void* stream);
+/* rot = I - E/2 + 3 E^2/8 with E = (gram + gram^H)/2 - I (n x n, 1 <= n <= 512): the rows of a
+ * nearly orthonormal block times rot are orthonormal up to E^3. emax[ceil(n / 32)]: the largest
+ * |component| of E over 32 rows each (float64, device; NaN when there is one). */
+int amt_lowdin(int precision, int n, const void* gram, void* rot, double* emax, void* stream);
+
+/*
  * Learned starting density. No counterpart in the reference: it produces the density=
  * argument of run_scf (scf/driver.py:267-299) as a correction over the atomic superposition
  * of PlaneWaveSystem.initial_density (hamiltonian/system.py:147-190), which stays the

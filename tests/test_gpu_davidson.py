@@ -186,3 +186,63 @@ def test_small_projected_matrices(nb):
         davidson(lambda x: x * float("nan"), guess[0], kin[0], tolerance=1e-8, max_iterations=3)
     with pytest.raises(torch.linalg.LinAlgError):
         solve_batched(lambda x: x * float("nan"), guess, kin, [n] * nk, tolerance=1e-8, max_iterations=3)
+
+
+def _gram_with_spectrum(n, cond, rng):
+    u, _ = np.linalg.qr(rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n)))
+    return (u * np.geomspace(1.0, 1.0 / cond, n)) @ u.conj().T
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 65, 97, 160, 440, 512])
+def test_inverse_cholesky_factor(dtype, n):
+    """L^{-1} of a Gram matrix around the 32-row blocks: lower triangular, X G X^H = I within the
+    factorisation's backward error (n u cond(G), eight of them; FP32 output adds its rounding of X,
+    4 u32 cond(G) sqrt(n) in the Frobenius norm), the trace and the sums of |X|^2; a batch with
+    fewer rows in use each (the rest the identity); the first pivot that is not positive."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    rng = np.random.default_rng(n)
+    cond = 100.0
+    u32 = 2.0**-24 if dtype == "complex64" else 0.0
+    g = torch.from_numpy(_gram_with_spectrum(n, cond, rng)).to(getattr(torch, dtype))
+    h = g.to(torch.complex128).numpy()
+    h = 0.5 * (h + h.conj().T)
+    bound = 8 * n * 2.0**-53 * cond + 4 * u32 * cond * np.sqrt(n)
+    x, stats = ops.chol_inverse(g.cuda())
+    x, stats = x.cpu().to(torch.complex128).numpy(), stats.cpu().numpy()
+    assert stats[0] == 0 and np.abs(np.triu(x, 1)).max(initial=0.0) == 0.0
+    assert np.linalg.norm(x @ h @ x.conj().T - np.eye(n)) <= bound
+    assert abs(stats[1] - np.trace(h).real) <= n * 2.0**-53 * np.trace(h).real
+    assert abs(stats[2:].sum() - np.sum(np.abs(x) ** 2)) <= (bound + 1e-14) * np.sum(np.abs(x) ** 2)
+    used = [max(n // 2, 1), n, max(n - 1, 1)]
+    batch = g.repeat(3, 1, 1).clone()
+    for k, m in enumerate(used):
+        batch[k, m:] = 0
+        batch[k, :, m:] = 0
+    x, stats = ops.chol_inverse(batch.cuda(), torch.tensor(used, dtype=torch.int32, device="cuda"))
+    for k, m in enumerate(used):
+        y = x[k].cpu().to(torch.complex128).numpy()
+        assert float(stats[k, 0]) == 0
+        assert np.linalg.norm(y[:m, :m] @ h[:m, :m] @ y[:m, :m].conj().T - np.eye(m)) <= bound
+        assert np.array_equal(y[m:, m:], np.eye(n - m)) and not y[m:, :m].any()
+        assert abs(float(stats[k, 2:].sum()) - np.sum(np.abs(y[:m, :m]) ** 2)) <= (bound + 1e-14) * np.sum(np.abs(y) ** 2)
+    for bad in {0, n // 2, n - 1}:
+        broken = g.clone()
+        broken[bad, bad] = -1.0
+        assert float(ops.chol_inverse(broken.cuda())[1][0]) == bad + 1
+        broken[bad, bad] = float("nan")
+        assert float(ops.chol_inverse(broken.cuda())[1][0]) == bad + 1
+    # the Loewdin series of I + E
+    e = 1e-3 * _gram_with_spectrum(n, 2.0, rng)
+    v = torch.from_numpy(np.eye(n) + e).to(getattr(torch, dtype))
+    e = v.to(torch.complex128).numpy()
+    e = 0.5 * (e + e.conj().T) - np.eye(n)
+    rot, emax = ops.lowdin(v.cuda())
+    want = np.eye(n) - 0.5 * e + 0.375 * (e @ e)
+    assert np.abs(rot.cpu().to(torch.complex128).numpy() - want).max() <= 2 * u32 + 4 * n * 2.0**-53
+    assert float(emax.max()) == max(np.abs(e.real).max(), np.abs(e.imag).max())
+    v[n // 2, 0] = float("nan")
+    assert np.isnan(float(ops.lowdin(v.cuda())[1].cpu().max()))
