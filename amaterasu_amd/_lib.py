@@ -53,6 +53,11 @@ SIGNATURES = {
     "amt_kb_dij": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_ll, _c_ll, _c_ll, _c_int, _vp]),
     "amt_heev_workspace": (_c_sz, [_c_int]),
     "amt_heev_lowest": (_c_int, [_c_int, _vp, _c_int, _vp, _vp, _vp, _c_sz, _vp]),
+    "amt_heev_batched_workspace": (_c_sz, [_c_int, _c_int]),
+    "amt_heev_lowest_batched": (_c_int, [_c_int, _ip, _vp, _c_ll, _c_ll, _c_int, _vp, _vp, _c_int, _vp, _c_sz, _vp]),
+    "amt_precondition_batched": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp]),
+    "amt_append_rows": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
+    "amt_append_projected": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "amt_chol_workspace": (_c_sz, [_c_int, _c_int]),
     "amt_chol_inverse": (_c_int, [_c_int, _c_int, _vp, _vp, _c_int, _vp, _vp, _vp, _c_sz, _vp]),
     "amt_lowdin": (_c_int, [_c_int, _c_int, _vp, _vp, _vp, _vp]),

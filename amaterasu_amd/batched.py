@@ -29,7 +29,7 @@ import numpy as np
 import torch
 
 from . import ops
-from .eigen import NAN_SILENT, _lowest_eigenpairs, orthonormalize, raise_not_finite
+from .eigen import HEEV_MAX, HEEV_MIN, NAN_SILENT, _lowest_eigenpairs, orthonormalize, raise_not_finite
 
 
 @dataclass
@@ -173,14 +173,19 @@ def _solve_streams(count: int) -> list:
 
 def _lowest(proj: torch.Tensor, used, nbands: int):
     """Lowest ``nbands`` eigenpairs of the leading used[k] x used[k] block of each projected
-    matrix, at its own size with the per-k Davidson's solver (the library's for 96..2048 rows):
+    matrix, at its own size with the per-k Davidson's solver (the library's for 2..2048 rows):
     eigenvalues (nk, nbands) and eigenvector rows (nk, nbands, n), zero on padded coordinates.
 
-    The solves of different k-points are independent chains of small, latency-bound launches,
-    so they run concurrently, one side stream and one workspace per k, ordered against the
+    The solves are independent chains of small, latency-bound launches: matrices the library
+    takes share every launch of one chain (4 matrices of 20 to 80 rows at 8 atoms: 240 -> 143 ms a
+    self-consistent run against one chain per k-point on its own stream, together with the
+    appends and the preconditioner in one launch each, since the host issuing launches was the
+    bound). Sizes it does not take run concurrently, one side stream per k, ordered against the
     caller's stream by events."""
     nk, n = proj.shape[0], proj.shape[-1]
-    used = [int(u) for u in (used.tolist() if isinstance(used, torch.Tensor) else used)]
+    used = [int(u) for u in used]
+    if all(HEEV_MIN <= c <= HEEV_MAX for c in used):
+        return ops.heev_lowest_batched(proj, used, nbands)
     w = torch.empty((nk, nbands), dtype=torch.float64, device=proj.device)
     rot = torch.zeros((nk, nbands, n), dtype=proj.dtype, device=proj.device)
     main = torch.cuda.current_stream()
@@ -249,7 +254,7 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
     # from scratch (subspace.py:72) up to rounding; a collapse recomputes the Ritz block
     proj = torch.zeros((nk, cap, cap), dtype=torch.complex128, device=dev)
     proj[:, :nb, :nb] = _projected(basis[:, :nb], hbasis[:, :nb])
-    eps, vec, hvec = _rayleigh_ritz(proj[:, :nb, :nb], basis[:, :nb], hbasis[:, :nb], full, nb)
+    eps, vec, hvec = _rayleigh_ritz(proj[:, :nb, :nb], basis[:, :nb], hbasis[:, :nb], [nb] * nk, nb)
     # frozen outputs of the k-points that have returned
     out_eps, out_vec = eps, vec
     out_norm = torch.full((nk, nb), float("inf"), dtype=torch.float64, device=dev)
@@ -274,13 +279,10 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
             break
         nnew = active.sum(axis=1)
         width = int(nnew.max())
-        # rows past a k-point's own count stay zero (empty only when every k fills the width)
-        full_width = bool((nnew[running] == width).all()) and running.all()
-        corr = (torch.empty if full_width else torch.zeros)((nk, width, npad), dtype=cdt, device=dev)
+        rows = np.full((nk, width), -1, dtype=np.int32)  # rows past a k-point's own count are zero
         for k in np.flatnonzero(running):
-            rows = torch.as_tensor(np.flatnonzero(active[k]) + k * nb, dtype=torch.int32, device=dev)
-            corr[k, : nnew[k]] = ops.precondition(res, vec.reshape(nk * nb, npad), kin[k], rows,
-                                                  rows_checked=True)  # host-built from this k's bands
+            rows[k, : nnew[k]] = np.flatnonzero(active[k]) + k * nb
+        corr = ops.precondition_batched(res, vec.reshape(nk * nb, npad), kin, torch.as_tensor(rows, device=dev))
         # orthogonalise against the current basis (its padded rows are zero), twice
         cur = int(m.max())
         for _ in range(2):
@@ -303,20 +305,13 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
         kept = np.where(running, kept, 0)
         new = new.contiguous()
         hnew = apply_block(new)
-        for k in np.flatnonzero(running):
-            basis[k, m[k] : m[k] + kept[k]] = new[k, : kept[k]]
-            hbasis[k, m[k] : m[k] + kept[k]] = hnew[k, : kept[k]]
+        grown = torch.as_tensor(np.stack([m, kept]).astype(np.int32), device=dev)
+        ops.append_rows(new, hnew, basis, hbasis, grown)
         cur = int((m + kept).max())
         cols = _bgram(basis[:, :cur], hnew)  # conj of <b_r|H|new_j>, rows of new past kept are zero
-        for k in np.flatnonzero(running):
-            a, b = int(m[k]), int(m[k] + kept[k])
-            ck = cols[k, :b, : kept[k]].conj().to(torch.complex128)
-            proj[k, :a, a:b] = ck[:a]
-            proj[k, a:b, :a] = ck[:a].conj().T
-            proj[k, a:b, a:b] = _herm(ck[a:b])
+        ops.append_projected(cols, proj, grown)
         m = m + kept
-        eps_n, vec_n, hvec_n = _rayleigh_ritz(proj[:, :cur, :cur], basis[:, :cur], hbasis[:, :cur],
-                                              torch.as_tensor(m, device=dev), nb)
+        eps_n, vec_n, hvec_n = _rayleigh_ritz(proj[:, :cur, :cur], basis[:, :cur], hbasis[:, :cur], m, nb)
         if running.all():
             eps, vec, hvec = eps_n, vec_n, hvec_n
             out_eps, out_vec = eps, vec

@@ -19,8 +19,12 @@ void set_error(const std::string& msg) { g_error = msg; }
 
 int launch_residual(int prec, const void* hv, const void* v, const double* eps, void* res, double* norm, int nrow,
                     int npw, hipStream_t s);
+int launch_append(int prec, const void* fresh, const void* hfresh, void* basis, void* hbasis, const int* m,
+                  const int* kept, int nk, int width, int cap, int npw, hipStream_t s);
+int launch_append_projected(int prec, const void* cols, void* proj, const int* m, const int* kept, int nk, int cur,
+                            int width, int cap, hipStream_t s);
 int launch_precondition(int prec, const void* res, const void* v, const void* kin, const int* rows, void* out,
-                        int nout, int npw, hipStream_t s);
+                        int nout, int npw, int per_k, hipStream_t s);
 int launch_dij(int prec, const void* P, const void* D, const int* blk_start, const int* blk_len, void* out,
                int nrow, int nproj, long long sP, long long sD, long long sO, int batch, hipStream_t s);
 
@@ -752,7 +756,46 @@ int amt_precondition(int precision, const void* res, const void* v, const void* 
     set_error("precondition: null argument");
     return 1;
   }
-  return launch_precondition(precision, res, v, kinetic, rows, out, nout, npw, (hipStream_t)stream);
+  return launch_precondition(precision, res, v, kinetic, rows, out, nout, npw, nout > 0 ? nout : 1, (hipStream_t)stream);
+}
+
+int amt_precondition_batched(int precision, const void* res, const void* v, const void* kinetic, const int* rows,
+                             void* out, int nk, int per_k, int npw, void* stream) {
+  if (nk < 1 || per_k < 1 || npw < 1 || (long long)nk * per_k > 0x7fffffff) {
+    set_error("precondition_batched: bad sizes");
+    return 1;
+  }
+  if (!res || !v || !kinetic || !rows || !out) {
+    set_error("precondition_batched: null argument");
+    return 1;
+  }
+  return launch_precondition(precision, res, v, kinetic, rows, out, nk * per_k, npw, per_k, (hipStream_t)stream);
+}
+
+int amt_append_rows(int precision, const void* fresh, const void* hfresh, void* basis, void* hbasis, const int* m,
+                    const int* kept, int nk, int width, int cap, int npw, void* stream) {
+  if (nk < 1 || nk > 65535 || width < 1 || width > 65535 || cap < 1 || npw < 1) {
+    set_error("append_rows: bad sizes");
+    return 1;
+  }
+  if (!fresh || !hfresh || !basis || !hbasis || !m || !kept) {
+    set_error("append_rows: null argument");
+    return 1;
+  }
+  return launch_append(precision, fresh, hfresh, basis, hbasis, m, kept, nk, width, cap, npw, (hipStream_t)stream);
+}
+
+int amt_append_projected(int precision, const void* cols, void* proj, const int* m, const int* kept, int nk, int cur,
+                         int width, int cap, void* stream) {
+  if (nk < 1 || nk > 65535 || cur < 1 || width < 1 || cap < cur || (long long)cur * width > 0x7fffffff - 256) {
+    set_error("append_projected: bad sizes");
+    return 1;
+  }
+  if (!cols || !proj || !m || !kept) {
+    set_error("append_projected: null argument");
+    return 1;
+  }
+  return launch_append_projected(precision, cols, proj, m, kept, nk, cur, width, cap, (hipStream_t)stream);
 }
 
 int amt_kb_dij(int precision, const void* proj, const void* dij, const int* blk_start, const int* blk_len,
@@ -854,5 +897,18 @@ int amt_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws
     set_error("heev: null argument");
     return 1;
   }
-  return launch_heev_lowest(n, a, nev, w, zt, ws, ws_bytes, (hipStream_t)stream);
+  return launch_heev_batched(1, &n, a, n, 0, nev, w, zt, n, ws, ws_bytes, (hipStream_t)stream);
+}
+
+size_t amt_heev_batched_workspace(int nmax, int nmat) {
+  return nmax > 0 && nmat > 0 ? heev_batched_workspace_bytes(nmax, nmat) : 0;
+}
+
+int amt_heev_lowest_batched(int nmat, const int* n, const void* a, long long lda, long long sa, int nev, double* w,
+                            void* zt, int ldz, void* ws, size_t ws_bytes, void* stream) {
+  if (nmat < 1 || !n || !a || !w || !zt || !ws) {
+    set_error("heev_batched: null argument or no matrix");
+    return 1;
+  }
+  return launch_heev_batched(nmat, n, a, lda, sa, nev, w, zt, ldz, ws, ws_bytes, (hipStream_t)stream);
 }

@@ -44,12 +44,32 @@ constexpr double kClusterGap = 2e-4;  // cluster threshold, relative to the Gers
 constexpr int kInverseRounds = 2;
 }  // namespace eig
 
+// The matrices of one launch set: matrix z = blockIdx.z has n[z] rows, and its workspace buffers lie
+// z stride bytes after those of the first. The chains of the matrices are independent and each
+// launch leaves most of the chip idle, so the matrices of a set share every launch. (Four of 20 to
+// 80 rows: one chain of 14 launches where four chains on four streams kept the host busy for
+// 0.5 ms a step.)
+constexpr int kHeevBatch = 16;
+struct HeevBatch {
+  int n[kHeevBatch];
+  long long stride;
+  template <typename T>
+  __device__ __forceinline__ T* at(T* p) const {
+    return (T*)((char*)p + blockIdx.z * stride);
+  }
+};
+
 // Columns per LDS slice of the Rayleigh-Ritz products inside a cluster.
 constexpr int kRRCols = 64;
 
 // Steps of a serial tridiagonal chain whose independent LDS loads are issued together (the
 // chain itself stays in registers, so LDS latency is paid once per chunk).
 constexpr int kTriChunk = 8;
+
+// Eigenvalues worked on for nev wanted ones: a cluster at the end may hold more.
+__host__ __device__ inline int heev_values(int n, int nev) {
+  return nev + eig::kClusterMax < n ? nev + eig::kClusterMax : n;
+}
 
 __device__ __forceinline__ double2 zmul(double2 a, double2 b) { return cmul(a, b); }
 
@@ -145,9 +165,12 @@ extern __shared__ __attribute__((aligned(16))) double tri_dyn[];
   HetrdShared sh{hetrd_dyn, hetrd_dyn + (n), hetrd_dyn + 2 * (n), hetrd_red}
 
 // Prologue: v_0 from row 0, d_0 / e_0 / tau_0, V[0], and p_0 = tau_0 A[1:,1:] v_0 for own rows.
-__global__ __launch_bounds__(eig::NT) void k_hetrd_start(const double2* __restrict__ A, int n, double2* __restrict__ V,
-                                                         double2* __restrict__ taus, double* __restrict__ d,
-                                                         double* __restrict__ e, double2* __restrict__ p) {
+__global__ __launch_bounds__(eig::NT) void k_hetrd_start(const double2* __restrict__ A, const HeevBatch hb,
+                                                         double2* __restrict__ V, double2* __restrict__ taus,
+                                                         double* __restrict__ d, double* __restrict__ e,
+                                                         double2* __restrict__ p) {
+  const int n = hb.n[blockIdx.z];
+  A = hb.at(A), V = hb.at(V), taus = hb.at(taus), d = hb.at(d), e = hb.at(e), p = hb.at(p);
   HETRD_SHARED(n);
   const int len = n - 1;  // length of column 0 below the diagonal
   for (int t = threadIdx.x; t < len; t += eig::NT) sh.v[t] = zconj(A[1 + t]);  // column 0 = conj(row 0)
@@ -215,16 +238,20 @@ __device__ __forceinline__ double2 block_sum2_once(double2 v, double* red) {
 // or 16; longer rows: k_hetrd_step_wide, shorter ones: k_hetrd_step_w64).
 
 template <int kRowRegs>
-__global__ __launch_bounds__(eig::NT) void k_hetrd_step(double2* __restrict__ A, int n, int j,
+__global__ __launch_bounds__(eig::NT) void k_hetrd_step(double2* __restrict__ A, const HeevBatch hb, int len,
                                                         double2* __restrict__ V, double2* __restrict__ taus,
                                                         double* __restrict__ d, double* __restrict__ e,
-                                                        const double2* __restrict__ p_in, double2* __restrict__ p_out) {
+                                                        double2* p0, double2* p1) {
+  const int n = hb.n[blockIdx.z], j = n - 1 - len;
+  if (j < 0) return;
+  const double2* p_in = hb.at(j & 1 ? p1 : p0);
+  double2* p_out = hb.at(j & 1 ? p0 : p1);
+  A = hb.at(A), V = hb.at(V), taus = hb.at(taus), d = hb.at(d), e = hb.at(e);
   constexpr int QV = kRowRegs / 4;  // vector elements per thread (n - j - 1 <= NT * QV)
   double2* sv = hetrd_dyn;          // v_j
   double2* sw = hetrd_dyn + n;      // w_j
   double2* sx = hetrd_dyn + 2 * n;  // column j+1 below the diagonal, unscaled
   __shared__ double red[2][2 * (eig::NT / 64)];
-  const int len = n - j - 1;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const double2 zero = make_double2(0.0, 0.0);
   const int myrow = j + 2 + blockIdx.x + wave * gridDim.x;
@@ -384,11 +411,15 @@ __device__ __forceinline__ double2 w64_element(const double2 (&x)[Q], int idx) {
 #define AMT_W64(x, idx) w64_element<Q>(x, idx)
 
 template <int Q>
-__global__ __launch_bounds__(64) void k_hetrd_step_w64(double2* __restrict__ A, int n, int j,
+__global__ __launch_bounds__(64) void k_hetrd_step_w64(double2* __restrict__ A, const HeevBatch hb, int len,
                                                        double2* __restrict__ V, double2* __restrict__ taus,
                                                        double* __restrict__ d, double* __restrict__ e,
-                                                       const double2* __restrict__ p_in, double2* __restrict__ p_out) {
-  const int len = n - j - 1;
+                                                       double2* p0, double2* p1) {
+  const int n = hb.n[blockIdx.z], j = n - 1 - len;
+  if (j < 0) return;
+  const double2* p_in = hb.at(j & 1 ? p1 : p0);
+  double2* p_out = hb.at(j & 1 ? p0 : p1);
+  A = hb.at(A), V = hb.at(V), taus = hb.at(taus), d = hb.at(d), e = hb.at(e);
   const int lane = threadIdx.x;
   const int myrow = j + 2 + blockIdx.x;
   const bool own = myrow < n;
@@ -520,17 +551,21 @@ __device__ __forceinline__ double2 reg_element(const double2 (&x)[K], int k) {
 }
 
 template <int NW, int RPL>
-__global__ __launch_bounds__(64 * NW) void k_hetrd_tail(double2* __restrict__ A, int n, int j0,
+__global__ __launch_bounds__(64 * NW) void k_hetrd_tail(double2* __restrict__ A, const HeevBatch hb,
                                                         double2* __restrict__ V, double2* __restrict__ taus,
                                                         double* __restrict__ d, double* __restrict__ e,
-                                                        const double2* __restrict__ p_in) {
+                                                        const double2* __restrict__ p0,
+                                                        const double2* __restrict__ p1) {
   constexpr int TL = 64 * RPL;  // rows (and columns) held
   constexpr int CW = TL / NW;   // columns per wavefront
   __shared__ double2 vw[NW][2][TL];    // per-wavefront copies of v and w
   __shared__ double2 col[2][TL];       // the next pivot column before its update, by step parity
   __shared__ double2 part[2][NW][TL];  // per-wavefront partial products M v, by step parity
   const int lane = threadIdx.x & 63, wq = threadIdx.x >> 6;
-  const int L0 = n - j0 - 1;  // trailing length at step j0, <= TL (checked by the host)
+  const int n = hb.n[blockIdx.z], j0 = max(n - 1 - TL, 0);
+  const double2* p_in = hb.at(j0 & 1 ? p1 : p0);
+  A = hb.at(A), V = hb.at(V), taus = hb.at(taus), d = hb.at(d), e = hb.at(e);
+  const int L0 = n - j0 - 1;  // trailing length at step j0, <= TL
   const int c0 = CW * wq;
   const double2 zero = make_double2(0.0, 0.0);
   double2 m[RPL][CW];  // rows lane + 64 q, columns c0 ..
@@ -669,17 +704,20 @@ __global__ __launch_bounds__(64 * NW) void k_hetrd_tail(double2* __restrict__ A,
 // barrier: at most 256 registers and 2n elements of LDS per workgroup (56 KB at n = 1760),
 // which lets two workgroups share a CU. With three vectors in LDS and in registers (the
 // n <= 1024 form) one workgroup per CU fit, and a 440-workgroup launch ran in two rounds.
-__global__ __launch_bounds__(eig::NT, 2) void k_hetrd_step_wide(double2* __restrict__ A, int n, int j,
-                                                               double2* __restrict__ V, double2* __restrict__ taus,
-                                                               double* __restrict__ d, double* __restrict__ e,
-                                                               const double2* __restrict__ p_in,
-                                                               double2* __restrict__ p_out) {
+__global__ __launch_bounds__(eig::NT, 2) void k_hetrd_step_wide(double2* __restrict__ A, const HeevBatch hb, int len,
+                                                                double2* __restrict__ V, double2* __restrict__ taus,
+                                                                double* __restrict__ d, double* __restrict__ e,
+                                                                double2* p0, double2* p1) {
+  const int n = hb.n[blockIdx.z], j = n - 1 - len;
+  if (j < 0) return;
+  const double2* p_in = hb.at(j & 1 ? p1 : p0);
+  double2* p_out = hb.at(j & 1 ? p0 : p1);
+  A = hb.at(A), V = hb.at(V), taus = hb.at(taus), d = hb.at(d), e = hb.at(e);
   constexpr int RR = eig::MAXN / 64;      // row elements per lane
   constexpr int QV = eig::MAXN / eig::NT;  // vector elements per thread
   double2* sv = hetrd_dyn;      // v_j, then the column j+1 below the diagonal (unscaled)
   double2* sw = hetrd_dyn + n;  // p_j, then w_j
   __shared__ double red[2][2 * (eig::NT / 64)];
-  const int len = n - j - 1;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const double2 zero = make_double2(0.0, 0.0);
   const int myrow = j + 2 + blockIdx.x + wave * gridDim.x;
@@ -836,8 +874,10 @@ __host__ __device__ inline int bt_chunks(int n) { return (n - 1 + kBtRows - 1) /
 
 // Partial Gram matrices of the blocks: Gp[b][ch][a][c] = sum over rows r in chunk ch of
 // block b (r = j0 + 1 + ch kBtRows + rr) of conj(v_a[r]) v_c[r], grid (chunks, blocks).
-__global__ __launch_bounds__(eig::NT) void k_bt_gram(const double2* __restrict__ V, int n,
+__global__ __launch_bounds__(eig::NT) void k_bt_gram(const double2* __restrict__ V, const HeevBatch hb,
                                                      double2* __restrict__ Gp) {
+  const int n = hb.n[blockIdx.z];
+  V = hb.at(V), Gp = hb.at(Gp);
   constexpr int B = kBtBlock, RC = kBtRows;
   __shared__ double2 tile[RC][B + 1];
   const int ch = blockIdx.x, b = blockIdx.y, j0 = b * B;
@@ -869,8 +909,11 @@ __global__ __launch_bounds__(eig::NT) void k_bt_gram(const double2* __restrict__
 // recursion runs on one wave with lane a holding row a of T in registers (both loops
 // unrolled), reading column i of the Gram matrix from LDS.
 __global__ __launch_bounds__(eig::NT) void k_bt_tfactor(const double2* __restrict__ Gp,
-                                                        const double2* __restrict__ taus, int n,
+                                                        const double2* __restrict__ taus, const HeevBatch hb,
                                                         double2* __restrict__ Tf) {
+  const int n = hb.n[blockIdx.z];
+  if ((int)blockIdx.x >= bt_blocks(n)) return;
+  Gp = hb.at(Gp), taus = hb.at(taus), Tf = hb.at(Tf);
   constexpr int B = kBtBlock;
   __shared__ double2 G[B][B + 1];
   const int b = blockIdx.x, j0 = b * B;
@@ -915,8 +958,11 @@ constexpr int kBtBatchW = 16;  // and in the sums w = V^H z
 
 __global__ __launch_bounds__(kBtThreads) void k_bt_apply(const double2* __restrict__ V,
                                                          const double2* __restrict__ Tf,
-                                                         const double* __restrict__ S, int n, int nev,
-                                                         double2* __restrict__ Zt) {
+                                                         const double* __restrict__ S, const HeevBatch hb, int nev,
+                                                         double2* __restrict__ Zt, int ldz) {
+  const int n = hb.n[blockIdx.z];
+  V = hb.at(V), Tf = hb.at(Tf), S = hb.at(S);
+  Zt += (long long)blockIdx.z * nev * ldz;
   constexpr int B = kBtBlock, E = kBtVecs, NT = kBtThreads, SL = kBtSlices;
   double2* z = hetrd_dyn;  // E x n
   __shared__ double2 w[E][B], u[E][B];
@@ -999,9 +1045,9 @@ __global__ __launch_bounds__(kBtThreads) void k_bt_apply(const double2* __restri
     }
     __syncthreads();
   }
-  for (int i = tid; i < E * n; i += NT) {
-    const int e = i / n;
-    if (e0 + e < nev) Zt[(long long)(e0 + e) * n + i % n] = z[i];
+  for (int i = tid; i < E * ldz; i += NT) {  // zeros past a smaller matrix of the set
+    const int e = i / ldz, r = i % ldz;
+    if (e0 + e < nev) Zt[(long long)(e0 + e) * ldz + r] = r < n ? z[e * n + r] : make_double2(0.0, 0.0);
   }
 }
 
@@ -1024,8 +1070,10 @@ __device__ __forceinline__ double recip(double q) {
 }
 
 __global__ __launch_bounds__(eig::NT) void k_tri_bisect(const double* __restrict__ d, const double* __restrict__ e,
-                                                        int n, int m, double* __restrict__ wb,
+                                                        const HeevBatch hb, int nev, double* __restrict__ wb,
                                                         double* __restrict__ scal) {
+  const int n = hb.n[blockIdx.z], m = heev_values(n, nev);
+  d = hb.at(d), e = hb.at(e), wb = hb.at(wb), scal = hb.at(scal);
   double* dl = tri_dyn;  // n entries each
   double* e2 = tri_dyn + n;
   __shared__ double red[3 * (eig::NT / 64)];
@@ -1250,9 +1298,11 @@ __device__ void tri_solve(const TriLU& f, int n, double* __restrict__ x) {
 // and factors T - w_r I (factors kept in work + 5 n r for the later rounds); every round
 // scales the row by tiny (it is unit-norm from the previous round) and solves once.
 __global__ __launch_bounds__(64) void k_tri_inverse(const double* __restrict__ d, const double* __restrict__ e,
-                                                    int n, int m, int round, const double* __restrict__ wb,
-                                                    const double* __restrict__ scal, double* __restrict__ S,
-                                                    double* __restrict__ work) {
+                                                    const HeevBatch hb, int nev, int round,
+                                                    const double* __restrict__ wb, const double* __restrict__ scal,
+                                                    double* __restrict__ S, double* __restrict__ work) {
+  const int n = hb.n[blockIdx.z], m = heev_values(n, nev);
+  d = hb.at(d), e = hb.at(e), wb = hb.at(wb), scal = hb.at(scal), S = hb.at(S), work = hb.at(work);
   // dynamic LDS of 8 n doubles: the factors, the vector and T
   const TriLU f{tri_dyn, tri_dyn + n, tri_dyn + 2 * n, tri_dyn + 3 * n, tri_dyn + 4 * n};
   double* x = tri_dyn + 5 * n;
@@ -1636,10 +1686,13 @@ __device__ void solve_piece(const double* __restrict__ d, const double* __restri
 // solved in order by this workgroup, each orthogonalised against the piece before it, so
 // (near-)degenerate eigenvalues never straddle a cut and neighbouring pieces stay orthogonal.
 __global__ __launch_bounds__(eig::NT) void k_tri_cluster(const double* __restrict__ d, const double* __restrict__ e,
-                                                         int n, int m, int nev, int round, int last,
+                                                         const HeevBatch hb, int nev, int round, int last,
                                                          const double* __restrict__ wb,
                                                          const double* __restrict__ scal, double* __restrict__ w,
                                                          double* __restrict__ S, double* __restrict__ work) {
+  const int n = hb.n[blockIdx.z], m = heev_values(n, nev);
+  d = hb.at(d), e = hb.at(e), wb = hb.at(wb), scal = hb.at(scal), S = hb.at(S), work = hb.at(work);
+  w += blockIdx.z * nev;
   __shared__ TriShared sh;
   const int k = blockIdx.x;
   if (k >= nev) return;
@@ -1678,40 +1731,43 @@ static int hetrd_groups(int n) {
   return g;
 }
 
-static void enqueue_tridiag(hipStream_t s, int n, double2* A, double2* V, double2* taus, double* d, double* e,
-                            double2* p0, double2* p1) {
-  const int G = hetrd_groups(n);
-  hipLaunchKernelGGL(k_hetrd_start, dim3(G), dim3(eig::NT), 3 * (size_t)n * sizeof(double2), s, A, n, V, taus,
-                     d, e, p0);
-  // Step j touches the trailing rows j+2 .. n-1 and columns j+1 .. n-1 only: its grid covers
+// Row-major A (leading dimension lda) into the workspace copy, rows back to back.
+__global__ __launch_bounds__(eig::NT) void k_heev_load(const double2* __restrict__ a, long long lda, long long sa,
+                                                       const HeevBatch hb, double2* __restrict__ A) {
+  const int n = hb.n[blockIdx.z];
+  A = hb.at(A);
+  a += blockIdx.z * sa;
+  for (long long i = (long long)blockIdx.x * eig::NT + threadIdx.x; i < (long long)n * n; i += (long long)gridDim.x * eig::NT)
+    A[i] = a[i / n * lda + i % n];
+}
+
+// nmax: the most rows of the set's nz matrices.
+static void enqueue_tridiag(hipStream_t s, const HeevBatch& hb, int nmax, int nz, double2* A, double2* V, double2* taus,
+                            double* d, double* e, double2* p0, double2* p1) {
+  const int n = nmax;
+  hipLaunchKernelGGL(k_hetrd_start, dim3(hetrd_groups(n), 1, nz), dim3(eig::NT), 3 * (size_t)n * sizeof(double2), s, A,
+                     hb, V, taus, d, e, p0);
+  // The step with trailing length len touches len - 1 rows and len columns only: its grid covers
   // those rows (one per wave) and its row template the trailing length, so the late, short
-  // steps launch few workgroups with short loops.
+  // steps launch few workgroups with short loops. A matrix with fewer rows joins at its own length.
   const size_t lds3 = 3 * (size_t)n * sizeof(double2), lds2 = 2 * (size_t)n * sizeof(double2);
-  for (int j = 0; j <= n - 2; ++j) {
-    const double2* pin = (j & 1) ? p1 : p0;
-    double2* pout = (j & 1) ? p0 : p1;
-    const int len = n - j - 1, rows = n - j - 2;
-    if (len <= kTailLen) {  // steps j .. n-2 in one launch
-      hipLaunchKernelGGL((k_hetrd_tail<kTailWaves, kTailLen / 64>), dim3(1), dim3(64 * kTailWaves), 0, s, A, n, j, V,
-                         taus, d, e, pin);
-      break;
-    }
-    const dim3 grid(rows > 0 ? (rows + 3) / 4 : 1);
+  for (int len = n - 1; len > kTailLen; --len) {
+    const dim3 grid((len + 2) / 4, 1, nz), rows(len - 1, 1, nz);
     if (len > eig::MAXN / 2)
-      hipLaunchKernelGGL(k_hetrd_step_wide, grid, dim3(eig::NT), lds2, s, A, n, j, V, taus, d, e, pin, pout);
+      hipLaunchKernelGGL(k_hetrd_step_wide, grid, dim3(eig::NT), lds2, s, A, hb, len, V, taus, d, e, p0, p1);
     else if (len > 768)
-      hipLaunchKernelGGL(k_hetrd_step<16>, grid, dim3(eig::NT), lds3, s, A, n, j, V, taus, d, e, pin, pout);
+      hipLaunchKernelGGL(k_hetrd_step<16>, grid, dim3(eig::NT), lds3, s, A, hb, len, V, taus, d, e, p0, p1);
     else if (len > 512)
-      hipLaunchKernelGGL(k_hetrd_step<12>, grid, dim3(eig::NT), lds3, s, A, n, j, V, taus, d, e, pin, pout);
+      hipLaunchKernelGGL(k_hetrd_step<12>, grid, dim3(eig::NT), lds3, s, A, hb, len, V, taus, d, e, p0, p1);
     else if (len > 64 * kW64Max)
-      hipLaunchKernelGGL(k_hetrd_step<8>, grid, dim3(eig::NT), lds3, s, A, n, j, V, taus, d, e, pin, pout);
+      hipLaunchKernelGGL(k_hetrd_step<8>, grid, dim3(eig::NT), lds3, s, A, hb, len, V, taus, d, e, p0, p1);
     else if (len > 256)
-      hipLaunchKernelGGL(k_hetrd_step_w64<kW64Max>, dim3(rows > 0 ? rows : 1), dim3(64), 0, s, A, n, j, V, taus, d,
-                         e, pin, pout);
+      hipLaunchKernelGGL(k_hetrd_step_w64<kW64Max>, rows, dim3(64), 0, s, A, hb, len, V, taus, d, e, p0, p1);
     else
-      hipLaunchKernelGGL(k_hetrd_step_w64<4>, dim3(rows > 0 ? rows : 1), dim3(64), 0, s, A, n, j, V, taus, d, e,
-                         pin, pout);
+      hipLaunchKernelGGL(k_hetrd_step_w64<4>, rows, dim3(64), 0, s, A, hb, len, V, taus, d, e, p0, p1);
   }
+  hipLaunchKernelGGL((k_hetrd_tail<kTailWaves, kTailLen / 64>), dim3(1, 1, nz), dim3(64 * kTailWaves), 0, s, A, hb, V,
+                     taus, d, e, p0, p1);  // the steps from trailing length kTailLen on
 }
 
 size_t heev_workspace_bytes(int n) {
@@ -1721,19 +1777,15 @@ size_t heev_workspace_bytes(int n) {
   return (size_t)n * n * 16 * 2 + (size_t)2 * n * 16 + (size_t)n * 16 + (size_t)n * n * 8 + (size_t)3 * n * 8 + 32 +
          (size_t)5 * n * n * 8 + 16 + bb * (bc + 1) * kBtBlock * kBtBlock * 16;
 }
+// One set of at most kHeevBatch matrices is worked on at a time.
+static size_t heev_stride(int nmax) { return (heev_workspace_bytes(nmax) + 255) & ~(size_t)255; }
+size_t heev_batched_workspace_bytes(int nmax, int nmat) {
+  return nmat > 1 ? heev_stride(nmax) * (nmat < kHeevBatch ? nmat : kHeevBatch) : heev_workspace_bytes(nmax);
+}
 
-int launch_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws, size_t ws_bytes,
-                       hipStream_t s) {
-  if (n < 2 || n > eig::MAXN || nev < 1 || nev > n) {
-    set_error("heev: need 2 <= n <= 2048 and 1 <= nev <= n");
-    return 1;
-  }
-  if (ws_bytes < heev_workspace_bytes(n)) {
-    set_error("heev: workspace smaller than amt_heev_workspace(n)");
-    return 1;
-  }
-  char* base = static_cast<char*>(ws);
-  double2* A = reinterpret_cast<double2*>(base);
+static int heev_set(const HeevBatch& hb, int n, int nz, const double2* a, long long lda, long long sa, int nev, double* w,
+                    double2* zt, int ldz, void* ws, hipStream_t s) {
+  double2* A = static_cast<double2*>(ws);
   double2* V = A + (size_t)n * n;
   double2* p0 = V + (size_t)n * n;
   double2* p1 = p0 + n;
@@ -1744,23 +1796,21 @@ int launch_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void*
   double* wb = e + n;
   double* scal = wb + n;
   double* lu = scal + 4;
-  if (hipMemcpyAsync(A, a, (size_t)n * n * 16, hipMemcpyDeviceToDevice, s) != hipSuccess) {
-    set_error("heev: copy of the input failed");
-    return 1;
-  }
-  enqueue_tridiag(s, n, A, V, taus, d, e, p0, p1);
+  const int fill = (n * n + eig::NT - 1) / eig::NT;
+  hipLaunchKernelGGL(k_heev_load, dim3(fill < 1024 ? fill : 1024, 1, nz), dim3(eig::NT), 0, s, a, lda, sa, hb, A);
+  enqueue_tridiag(s, hb, n, nz, A, V, taus, d, e, p0, p1);
   if (hipGetLastError() != hipSuccess) {
     set_error("heev: tridiagonalisation launch failed");
     return 1;
   }
-  const int m = nev + eig::kClusterMax < n ? nev + eig::kClusterMax : n;
-  hipLaunchKernelGGL(k_tri_bisect, dim3(m), dim3(eig::NT), 2 * (size_t)n * sizeof(double), s, d, e, n, m, wb,
+  const int m = heev_values(n, nev);
+  hipLaunchKernelGGL(k_tri_bisect, dim3(m, 1, nz), dim3(eig::NT), 2 * (size_t)n * sizeof(double), s, d, e, hb, nev, wb,
                      scal);
   for (int round = 0; round < eig::kInverseRounds; ++round) {
-    hipLaunchKernelGGL(k_tri_inverse, dim3(m), dim3(64), 8 * (size_t)n * sizeof(double), s, d, e, n, m, round,
+    hipLaunchKernelGGL(k_tri_inverse, dim3(m, 1, nz), dim3(64), 8 * (size_t)n * sizeof(double), s, d, e, hb, nev, round,
                        wb, scal, S, lu);
-    hipLaunchKernelGGL(k_tri_cluster, dim3(nev), dim3(eig::NT), 2 * eig::kClusterMax * (kRRCols + 1) * sizeof(double),
-                       s, d, e, n, m, nev, round,
+    hipLaunchKernelGGL(k_tri_cluster, dim3(nev, 1, nz), dim3(eig::NT),
+                       2 * eig::kClusterMax * (kRRCols + 1) * sizeof(double), s, d, e, hb, nev, round,
                        round + 1 == eig::kInverseRounds ? 1 : 0, wb, scal, w, S, lu);
   }
   if (hipGetLastError() != hipSuccess) {
@@ -1769,13 +1819,39 @@ int launch_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void*
   }
   double2* Gp = reinterpret_cast<double2*>((reinterpret_cast<uintptr_t>(lu + (size_t)5 * n * n) + 15) & ~uintptr_t(15));
   double2* Tf = Gp + (size_t)bt_blocks(n) * bt_chunks(n) * kBtBlock * kBtBlock;
-  hipLaunchKernelGGL(k_bt_gram, dim3(bt_chunks(n), bt_blocks(n)), dim3(eig::NT), 0, s, V, n, Gp);
-  hipLaunchKernelGGL(k_bt_tfactor, dim3(bt_blocks(n)), dim3(eig::NT), 0, s, Gp, taus, n, Tf);
-  hipLaunchKernelGGL(k_bt_apply, dim3((nev + kBtVecs - 1) / kBtVecs), dim3(kBtThreads),
-                     (size_t)kBtVecs * n * sizeof(double2), s, V, Tf, S, n, nev, static_cast<double2*>(zt));
+  hipLaunchKernelGGL(k_bt_gram, dim3(bt_chunks(n), bt_blocks(n), nz), dim3(eig::NT), 0, s, V, hb, Gp);
+  hipLaunchKernelGGL(k_bt_tfactor, dim3(bt_blocks(n), 1, nz), dim3(eig::NT), 0, s, Gp, taus, hb, Tf);
+  hipLaunchKernelGGL(k_bt_apply, dim3((nev + kBtVecs - 1) / kBtVecs, 1, nz), dim3(kBtThreads),
+                     (size_t)kBtVecs * n * sizeof(double2), s, V, Tf, S, hb, nev, zt, ldz);
   if (hipGetLastError() != hipSuccess) {
     set_error("heev: back-transformation launch failed");
     return 1;
+  }
+  return 0;
+}
+
+int launch_heev_batched(int nmat, const int* n, const void* a, long long lda, long long sa, int nev, double* w, void* zt,
+                        int ldz, void* ws, size_t ws_bytes, hipStream_t s) {
+  int nmax = 0;
+  for (int z = 0; z < nmat; ++z) {
+    if (n[z] < 2 || n[z] > eig::MAXN || nev < 1 || nev > n[z] || n[z] > lda || n[z] > ldz) {
+      set_error("heev: need 2 <= n <= 2048 and 1 <= nev <= n");
+      return 1;
+    }
+    nmax = n[z] > nmax ? n[z] : nmax;
+  }
+  if (ws_bytes < heev_batched_workspace_bytes(nmax, nmat)) {
+    set_error("heev: workspace smaller than amt_heev_workspace(n)");
+    return 1;
+  }
+  for (int z0 = 0; z0 < nmat; z0 += kHeevBatch) {
+    HeevBatch hb{};
+    const int nz = nmat - z0 < kHeevBatch ? nmat - z0 : kHeevBatch;
+    for (int z = 0; z < nz; ++z) hb.n[z] = n[z0 + z];
+    hb.stride = (long long)heev_stride(nmax);
+    if (heev_set(hb, nmax, nz, static_cast<const double2*>(a) + z0 * sa, lda, sa, nev, w + (size_t)z0 * nev,
+                 static_cast<double2*>(zt) + (size_t)z0 * nev * ldz, ldz, ws, s))
+      return 1;
   }
   return 0;
 }

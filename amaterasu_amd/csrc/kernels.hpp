@@ -138,7 +138,9 @@ int set_zgemm_split(int prec, int op, int m, int n, int k, int batch, int split)
 
 // Lowest eigenpairs of a dense Hermitian FP64 matrix (eig.hip).
 size_t heev_workspace_bytes(int n);
-int launch_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws, size_t ws_bytes, hipStream_t s);
+size_t heev_batched_workspace_bytes(int nmax, int nmat);
+int launch_heev_batched(int nmat, const int* n, const void* a, long long lda, long long sa, int nev, double* w, void* zt,
+                        int ldz, void* ws, size_t ws_bytes, hipStream_t s);
 
 // Inverse Cholesky factor of Gram matrices and the Loewdin series (chol.hip).
 int chol_blocks(int n);

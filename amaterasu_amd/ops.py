@@ -17,7 +17,7 @@ _WORKSPACES: dict = {}
 
 
 def stream_handle() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def precision_of(t: torch.Tensor) -> int:
@@ -202,6 +202,59 @@ def precondition(res: torch.Tensor, v: torch.Tensor, kinetic: torch.Tensor, rows
     return out
 
 
+def precondition_batched(res: torch.Tensor, v: torch.Tensor, kinetic: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
+    """:func:`precondition` for all k-points in one launch: ``kinetic`` is ``[nk][npw]``, ``rows``
+    ``[nk][width]`` (int32, device) holds row indices of ``res`` and ``v``, negative for a row of
+    zeros, checked by the caller. Returns ``[nk][width][npw]``."""
+    _require(res, "res")
+    _require(v, "v")
+    _require(kinetic, "kinetic")
+    _require(rows, "rows")
+    prec = precision_of(v)
+    if res.shape != v.shape or res.dtype != v.dtype or v.dim() != 2:
+        raise AmtError("precondition: res and v must be equal 2-D blocks")
+    nk, width = rows.shape
+    if rows.dtype != torch.int32 or kinetic.dtype != real_dtype(prec) or tuple(kinetic.shape) != (nk, v.shape[1]):
+        raise AmtError("precondition: kinetic must have one entry per k-point and plane wave, rows one list per k-point")
+    out = torch.empty((nk, width, v.shape[1]), dtype=v.dtype, device=v.device)
+    check(lib().amt_precondition_batched(prec, res.data_ptr(), v.data_ptr(), kinetic.data_ptr(), rows.data_ptr(),
+                                         out.data_ptr(), nk, width, v.shape[1], stream_handle()), "precondition_batched")
+    return out
+
+
+def append_rows(fresh: torch.Tensor, hfresh: torch.Tensor, basis: torch.Tensor, hbasis: torch.Tensor,
+                grown: torch.Tensor):
+    """Rows ``j < grown[1, k]`` of ``fresh`` and ``hfresh`` ``[nk][width][npw]`` become rows
+    ``grown[0, k] + j`` of ``basis`` and ``hbasis`` ``[nk][cap][npw]`` (``grown`` int32, device)."""
+    for t, name in ((fresh, "fresh"), (hfresh, "hfresh"), (basis, "basis"), (hbasis, "hbasis"), (grown, "grown")):
+        _require(t, name)
+    nk, width, npw = fresh.shape
+    cap = basis.shape[1]
+    if (hfresh.shape != fresh.shape or hbasis.shape != basis.shape or tuple(basis.shape) != (nk, cap, npw)
+            or not fresh.dtype == hfresh.dtype == basis.dtype == hbasis.dtype):
+        raise AmtError("append_rows: blocks of one dtype, [nk][width][npw] into [nk][cap][npw]")
+    if grown.dtype != torch.int32 or tuple(grown.shape) != (2, nk):
+        raise AmtError("append_rows: grown must be int32 [2][nk]")
+    check(lib().amt_append_rows(precision_of(fresh), fresh.data_ptr(), hfresh.data_ptr(), basis.data_ptr(),
+                                hbasis.data_ptr(), grown[0].data_ptr(), grown[1].data_ptr(), nk, width, cap, npw,
+                                stream_handle()), "append_rows")
+
+
+def append_projected(cols: torch.Tensor, proj: torch.Tensor, grown: torch.Tensor):
+    """New rows and columns of the projected matrices ``proj`` ``[nk][cap][cap]`` from ``cols``
+    ``[nk][cur][width]`` = basis (H fresh)^H; ``grown`` as in :func:`append_rows`."""
+    for t, name in ((cols, "cols"), (proj, "proj"), (grown, "grown")):
+        _require(t, name)
+    nk, cur, width = cols.shape
+    cap = proj.shape[1]
+    if proj.dtype != torch.complex128 or tuple(proj.shape) != (nk, cap, cap) or cur > cap:
+        raise AmtError("append_projected: proj must be complex128 [nk][cap][cap]")
+    if grown.dtype != torch.int32 or tuple(grown.shape) != (2, nk):
+        raise AmtError("append_projected: grown must be int32 [2][nk]")
+    check(lib().amt_append_projected(precision_of(cols), cols.data_ptr(), proj.data_ptr(), grown[0].data_ptr(),
+                                     grown[1].data_ptr(), nk, cur, width, cap, stream_handle()), "append_projected")
+
+
 #: Gram matrices of at most this many rows go to the library's Cholesky and Loewdin kernels.
 CHOL_MAX = 512
 
@@ -261,5 +314,26 @@ def heev_lowest(a: torch.Tensor, nev: int, *, workspace_tag: str = "heev"):
     ws = workspace(nbytes, workspace_tag)
     check(lib().amt_heev_lowest(n, a.data_ptr(), nev, w.data_ptr(), zt.data_ptr(), ws.data_ptr(), nbytes,
                                 stream_handle()), "heev")
+    return w, zt
+
+
+def heev_lowest_batched(a: torch.Tensor, sizes, nev: int):
+    """:func:`heev_lowest` of the leading ``sizes[k]`` rows of every matrix of ``a`` ``[nk][n][n]``
+    (rows contiguous) in one set of launches: ``w`` ``[nk][nev]`` and ``zt`` ``[nk][nev][n]``, zero
+    past ``sizes[k]``."""
+    _require_rows(a, "a")
+    if a.dtype != torch.complex128 or a.dim() != 3 or a.shape[1] != a.shape[2]:
+        raise AmtError("heev: a must be square complex128 device matrices")
+    nk, n = a.shape[0], a.shape[-1]
+    sizes = [int(s) for s in sizes]
+    if len(sizes) != nk or not all(1 <= nev <= s <= n for s in sizes):
+        raise AmtError(f"heev: sizes {sizes} outside {nev}..{n}")
+    w = torch.empty((nk, nev), dtype=torch.float64, device=a.device)
+    zt = torch.empty((nk, nev, n), dtype=torch.complex128, device=a.device)
+    nbytes = int(lib().amt_heev_batched_workspace(max(sizes), nk))
+    ws = workspace(nbytes, "heev_batched")
+    check(lib().amt_heev_lowest_batched(nk, (ctypes.c_int * nk)(*sizes), a.data_ptr(), a.stride(1), a.stride(0), nev,
+                                        w.data_ptr(), zt.data_ptr(), n, ws.data_ptr(), nbytes, stream_handle()),
+          "heev_batched")
     return w, zt
 

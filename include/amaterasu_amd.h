@@ -193,6 +193,23 @@ int amt_residual(int precision, const void* hv, const void* v, const double* eps
  */
 int amt_precondition(int precision, const void* res, const void* v, const void* kinetic, const int* rows,
                      void* out, int nout, int npw, void* stream);
+/*
+ * The same over k-points in one launch: out is [nk][per_k][npw], rows holds nk per_k source rows
+ * (negative: a row of zeros), kinetic is [nk][npw].
+ */
+int amt_precondition_batched(int precision, const void* res, const void* v, const void* kinetic, const int* rows,
+                             void* out, int nk, int per_k, int npw, void* stream);
+/*
+ * Growth of the subspaces of all k-points (scf/eigen/davidson.py:97-104). m and kept are device
+ * arrays of nk entries, m[k] + kept[k] <= cap. amt_append_rows: rows j < kept[k] of fresh and hfresh
+ * [nk][width][npw] become rows m[k] + j of basis and hbasis [nk][cap][npw]. amt_append_projected:
+ * cols [nk][cur][width] = basis (H fresh)^H gives the new rows and columns of the projected matrices
+ * proj [nk][cap][cap] (complex128).
+ */
+int amt_append_rows(int precision, const void* fresh, const void* hfresh, void* basis, void* hbasis, const int* m,
+                    const int* kept, int nk, int width, int cap, int npw, void* stream);
+int amt_append_projected(int precision, const void* cols, void* proj, const int* m, const int* kept, int nk, int cur,
+                         int width, int cap, void* stream);
 /* (P D) of KBProjectors.apply (pseudo/kb.py:230) for block-diagonal D (real, nproj x nproj). */
 int amt_kb_dij(int precision, const void* proj, const void* dij, const int* blk_start, const int* blk_len,
                void* out, int nrow, int nproj, long long sp, long long sd, long long so, int batch, void* stream);
@@ -208,6 +225,14 @@ int amt_kb_dij(int precision, const void* proj, const void* dij, const int* blk_
  */
 size_t amt_heev_workspace(int n);
 int amt_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws, size_t ws_bytes, void* stream);
+/*
+ * The same for nmat matrices of n[z] rows each (host array) that share every launch: matrix z at a +
+ * z sa (row stride lda, complex128 elements), w [nmat][nev], zt [nmat][nev][ldz] with zeros past
+ * n[z]. nev <= every n[z] <= lda, ldz. ws must hold amt_heev_batched_workspace(max n, nmat) bytes.
+ */
+size_t amt_heev_batched_workspace(int nmax, int nmat);
+int amt_heev_lowest_batched(int nmat, const int* n, const void* a, long long lda, long long sa, int nev, double* w,
+                            void* zt, int ldz, void* ws, size_t ws_bytes, void* stream);
 
 /*
  * Inverse Cholesky factor of the Gram matrices of orthonormalize / orthogonalize_against

@@ -119,3 +119,84 @@ def test_library_eigensolver_inside_davidson(monkeypatch):
         for c in (one.coefficients, res.coefficients[k][:, :n]):
             ov = c @ c.conj().T
             assert torch.abs(ov - torch.eye(nb, dtype=ov.dtype, device=ov.device)).max().item() < 1e-11
+
+
+@pytest.mark.parametrize("sizes,nev", [([2, 2], 1), ([3, 9, 5, 9], 3), ([64, 65, 66, 33], 20), ([200, 66, 130], 40),
+                                       ([300, 280], 16), ([20] * 17 + [24] * 2, 8)])
+def test_heev_batched_matches_single(sizes, nev):
+    """The batched eigensolver runs every matrix's own chain: against the one-matrix entry point
+    (equal eigenvalues to 8 n eps ||A||, vectors with the same residual bound, zeros past a
+    smaller matrix), from strided views whose other entries are NaN."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    rng = np.random.default_rng(sum(sizes) + nev)
+    cap = max(sizes) + 3
+    a = torch.full((len(sizes), cap, cap), float("nan"), dtype=torch.complex128, device="cuda")
+    mats = []
+    for k, n in enumerate(sizes):
+        x = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+        mats.append(torch.from_numpy(x + x.conj().T).cuda())
+        a[k, :n, :n] = mats[-1]
+    cur = max(sizes)
+    w, zt = ops.heev_lowest_batched(a[:, :cur, :cur], sizes, nev)
+    for k, n in enumerate(sizes):
+        ws, zs = ops.heev_lowest(mats[k], nev)
+        norm = float(torch.linalg.matrix_norm(mats[k], 2))
+        tol = 8 * n * 2.2e-16 * norm
+        assert float((w[k] - ws).abs().max()) <= tol
+        z = zt[k]
+        assert not z[:, n:].any()
+        z = z[:, :n]
+        single = (zs @ mats[k].T - ws[:, None] * zs).abs().max().item()
+        assert (z @ mats[k].T - w[k][:, None] * z).abs().max().item() <= max(tol, 2 * single)
+        eye = torch.eye(nev, dtype=z.dtype, device="cuda")
+        assert (z.conj() @ z.T - eye).abs().max().item() <= max(tol / norm, 2 * (zs.conj() @ zs.T - eye).abs().max().item())
+
+
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+@pytest.mark.parametrize("npw,width", [(1, 1), (255, 3), (257, 5), (5000, 2)])
+def test_subspace_growth_kernels(dtype, npw, width):
+    """Appended rows are copies; projected entries those of the formula (FP64 of the given
+    numbers: exact for conj and to one rounding for the Hermitian part); a list with negative
+    entries gives zero rows and the others those of the one-k-point entry."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    dt = getattr(torch, dtype)
+    rdt = torch.float64 if dt == torch.complex128 else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(npw)
+    rand = lambda *s: torch.randn(*s, dtype=dt, device="cuda", generator=gen)  # noqa: E731
+    nk, cap = 3, 2 * width + 4
+    m, kept = np.array([2, 0, 4]), np.array([width, 0, max(width - 1, 0)])
+    grown = torch.as_tensor(np.stack([m, kept]).astype(np.int32), device="cuda")
+    new, hnew, basis, hbasis = rand(nk, width, npw), rand(nk, width, npw), rand(nk, cap, npw), rand(nk, cap, npw)
+    want, hwant = basis.clone(), hbasis.clone()
+    cur = int((m + kept).max())
+    cols = rand(nk, cur, width)
+    proj = torch.randn(nk, cap, cap, dtype=torch.complex128, device="cuda", generator=gen)
+    pwant = proj.clone()
+    for k in range(nk):
+        a, b = m[k], m[k] + kept[k]
+        want[k, a:b], hwant[k, a:b] = new[k, : kept[k]], hnew[k, : kept[k]]
+        ck = cols[k, :b, : kept[k]].conj().to(torch.complex128)
+        pwant[k, :a, a:b], pwant[k, a:b, :a] = ck[:a], ck[:a].conj().T
+        pwant[k, a:b, a:b] = 0.5 * (ck[a:b] + ck[a:b].conj().T)
+    ops.append_rows(new, hnew, basis, hbasis, grown)
+    ops.append_projected(cols, proj, grown)
+    assert torch.equal(basis, want) and torch.equal(hbasis, hwant)
+    assert (proj - pwant).abs().max().item() <= 4 * 2.0**-53 * pwant.abs().max().item()
+    res, vec = rand(2 * nk, npw), rand(2 * nk, npw)
+    kin = torch.rand(nk, npw, dtype=rdt, device="cuda", generator=gen)
+    rows = np.full((nk, width), -1, dtype=np.int32)
+    rows[0, 0], rows[2, :2] = 1, [4, 5][:width]
+    out = ops.precondition_batched(res, vec, kin, torch.as_tensor(rows, device="cuda"))
+    for k in range(nk):
+        for i in range(width):
+            if rows[k, i] < 0:
+                assert not out[k, i].any()
+            else:
+                one = ops.precondition(res, vec, kin[k], torch.tensor([rows[k, i]], device="cuda"))
+                assert torch.equal(out[k, i], one[0])
