@@ -260,7 +260,7 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
     out_norm = torch.full((nk, nb), float("inf"), dtype=torch.float64, device=dev)
     running = np.ones(nk, dtype=bool)
     iters = np.zeros(nk, dtype=int)
-    kin = kinetic.to(dev).contiguous()
+    kin = kinetic.to(device=dev, dtype=ops.real_dtype(ops.precision_of(guess))).contiguous()
     for step in range(1, max_iterations + 1):
         iters[running] = step
         res, norms = ops.residual(hvec.reshape(nk * nb, npad), vec.reshape(nk * nb, npad), eps.reshape(-1))
@@ -306,7 +306,7 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
         new = new.contiguous()
         hnew = apply_block(new)
         grown = torch.as_tensor(np.stack([m, kept]).astype(np.int32), device=dev)
-        ops.append_rows(new, hnew, basis, hbasis, grown)
+        ops.append_rows(new, hnew.to(cdt).contiguous(), basis, hbasis, grown)
         cur = int((m + kept).max())
         cols = _bgram(basis[:, :cur], hnew)  # conj of <b_r|H|new_j>, rows of new past kept are zero
         ops.append_projected(cols, proj, grown)

@@ -500,8 +500,8 @@ int amt_hpsi(const amt_plan_t* h, int precision, const void* psi, void* hpsi, in
   hipStream_t s = (hipStream_t)stream;
   unsigned char* base = static_cast<unsigned char*>(ws);
   if (p.plane_threads[precision] == 0) {
-    if (launch_hpsi_full_grid(p, precision, psi, hpsi, nb, k0, nkk, veff, base, l.sticks, s)) return 1;
-  } else if (launch_hpsi_local(p, precision, psi, hpsi, nb, k0, nkk, veff, base, s)) {
+    if (launch_hpsi_full_grid(p, precision, psi, hpsi, nb, k0, nkk, veff, base, l.sticks, s, true)) return 1;
+  } else if (launch_hpsi_local(p, precision, psi, hpsi, nb, k0, nkk, veff, base, s, 0, true)) {
     return 1;
   }
   const int np = p.nproj[precision];
@@ -515,11 +515,9 @@ int amt_hpsi(const amt_plan_t* h, int precision, const void* psi, void* hpsi, in
   void* pd = base + l.sticks + l.proj;
   void* gws = base + l.sticks + l.proj + l.pd;
   const long long spsi = (long long)nb * p.npw_pad, smat = (long long)np * p.npw_pad, sp = (long long)nb * np;
-  if (launch_zgemm(precision, 1, nb, np, p.npw_pad, 1.0, psi, p.npw_pad, spsi, mat, p.npw_pad, smat, 0.0, proj, np,
-                   sp, nkk, gws, l.gemm, s))
-    return 1;
-  if (launch_dij(precision, proj, dij, p.kb_blk_start[precision], p.kb_blk_len[precision], pd, nb, np, sp,
-                 (long long)np * np, sp, nkk, s))
+  const DijArgs contract{dij, (long long)np * np, p.kb_blk_start[precision], p.kb_blk_len[precision], pd, sp};
+  if (launch_zgemm_dij(precision, nb, np, p.npw_pad, psi, p.npw_pad, spsi, mat, p.npw_pad, smat, proj, contract, nkk,
+                       gws, l.gemm, s))
     return 1;
   return launch_zgemm(precision, 0, nb, p.npw_pad, np, 1.0, pd, np, sp, mat, p.npw_pad, smat, 1.0, hpsi, p.npw_pad,
                       spsi, nkk, gws, l.gemm, s);

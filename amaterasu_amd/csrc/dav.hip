@@ -148,6 +148,7 @@ __global__ void k_dij(const typename Cplx<R>::T* __restrict__ P, const R* __rest
   const R* d = D + batch * sD;
   const int j0 = blk_start[i], j1 = j0 + blk_len[i];
   R sr = 0, si = 0;
+#pragma unroll 4
   for (int j = j0; j < j1; ++j) {
     const R dj = d[(long long)j * nproj + i];
     sr += p[j].x * dj;

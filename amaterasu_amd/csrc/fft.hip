@@ -213,9 +213,9 @@ __global__ void k_plane_vloc(C* __restrict__ sticks, const int* __restrict__ sti
 // Forward transform along i, then out[g] = T_g psi[g] + (1/N) sticks at g.
 template <int TPT, typename C, typename R>
 __global__ void k_stick_forward(const C* __restrict__ sticks, const C* __restrict__ psi, C* __restrict__ out,
-                                const int* __restrict__ stick_map, const R* __restrict__ kin, int n1, int smax,
-                                int npw_pad, int nb, int k0, AxisPlan ap1, const C* __restrict__ tw1, int W,
-                                R scale) {
+                                const int* __restrict__ stick_map, const R* __restrict__ kin,
+                                const int* __restrict__ npw, int n1, int smax, int npw_pad, int nb, int k0,
+                                AxisPlan ap1, const C* __restrict__ tw1, int W, R scale) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   C* lds = reinterpret_cast<C*>(smem_raw);
   const int tid = threadIdx.x, nth = blockDim.x;
@@ -233,6 +233,8 @@ __global__ void k_stick_forward(const C* __restrict__ sticks, const C* __restric
   const C* c = psi + (long long)kb * npw_pad;
   C* o = out + (long long)kb * npw_pad;
   const R* t = kin + (long long)k * npw_pad;
+  if (npw && blockIdx.x == 0)  // the row's padding
+    for (int g = npw[k] + tid; g < npw_pad; g += nth) o[g] = cmake<C>(0, 0);
   for (int e = tid; e < n1 * W; e += nth) {
     const int i = e / W, w = e % W, s = s0 + w;
     if (s < smax) {
@@ -332,14 +334,17 @@ __global__ void k_grid_vmul(C* __restrict__ grids, const R* __restrict__ v, long
   for (int b = 0; b < nbc; ++b) grids[(long long)b * ngrid + e] = cscale(grids[(long long)b * ngrid + e], ve);
 }
 
-// out[b][g] = kin[g] psi[b][g] + scale grid[b][flatmap[g]] for g < npw (padding not written)
+// out[b][g] = kin[g] psi[b][g] + scale grid[b][flatmap[g]] for g < npw, 0 for npw <= g < end
 template <typename C, typename R>
 __global__ void k_gather_kinetic(const C* __restrict__ grid, const C* __restrict__ psi, C* __restrict__ out,
-                                 const int* __restrict__ flatmap, const R* __restrict__ kin, int npw, int npw_pad,
-                                 long long ngrid, R scale) {
+                                 const int* __restrict__ flatmap, const R* __restrict__ kin, int npw, int end,
+                                 int npw_pad, long long ngrid, R scale) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int b = blockIdx.y;
-  if (g >= npw) return;
+  if (g >= npw) {
+    if (g < end) out[(long long)b * npw_pad + g] = cmake<C>(0, 0);
+    return;
+  }
   const C x = psi[(long long)b * npw_pad + g];
   const C y = grid[(long long)b * ngrid + flatmap[g]];
   out[(long long)b * npw_pad + g] = cmake<C>(kin[g] * x.x + scale * y.x, kin[g] * x.y + scale * y.y);
@@ -384,7 +389,7 @@ static int check(hipError_t e, const char* what) {
 
 template <typename R>
 static int hpsi_local_t(const Plan& p, const void* psi_, void* hpsi_, int nb, int k0, int nkk, const void* veff_,
-                        void* sticks_, hipStream_t s, int stage) {
+                        void* sticks_, hipStream_t s, int stage, bool pad) {
   using C = typename Cplx<R>::T;
   constexpr int prec = sizeof(R) == 8 ? kFP64 : kFP32;
   constexpr int TPT = sizeof(R) == 8 ? kTptF64 : kTptF32;
@@ -415,23 +420,24 @@ static int hpsi_local_t(const Plan& p, const void* psi_, void* hpsi_, int nb, in
   }
   if (stage == 0 || stage == 3) {
     hipLaunchKernelGGL((k_stick_forward<TPT, C, R>), sgrid, dim3(p.stick_threads[prec]), slds, s, sticks, psi,
-                       hpsi, p.d_stick_map, kin, p.n1, p.smax, p.npw_pad, nb, k0, p.ap[0], tw[0], W, scale);
+                       hpsi, p.d_stick_map, kin, pad ? p.d_npw : nullptr, p.n1, p.smax, p.npw_pad, nb, k0, p.ap[0],
+                       tw[0], W, scale);
     if (check(hipGetLastError(), "stick_forward launch")) return 1;
   }
   return 0;
 }
 
 int launch_hpsi_local(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                      const void* veff, void* sticks, hipStream_t s, int stage) {
+                      const void* veff, void* sticks, hipStream_t s, int stage, bool pad) {
   if (p.fast) {
-    if (launch_hpsi_fast(p, prec, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage)) {
+    if (launch_hpsi_fast(p, prec, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage, pad)) {
       set_error(std::string("hpsi (compile-time length) launch: ") + hipGetErrorString(hipGetLastError()));
       return 1;
     }
     return 0;
   }
-  return prec == kFP64 ? hpsi_local_t<double>(p, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage)
-                       : hpsi_local_t<float>(p, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage);
+  return prec == kFP64 ? hpsi_local_t<double>(p, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage, pad)
+                       : hpsi_local_t<float>(p, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage, pad);
 }
 
 template <typename R>
@@ -585,7 +591,7 @@ long long full_grid_rows(const Plan& p, int prec, size_t ws_bytes) {
 
 template <typename R>
 static int hpsi_full_grid_t(const Plan& p, const void* psi_, void* hpsi_, int nb, int k0, int nkk, const void* veff_,
-                            void* ws, size_t ws_bytes, hipStream_t s) {
+                            void* ws, size_t ws_bytes, hipStream_t s, bool pad) {
   using C = typename Cplx<R>::T;
   constexpr int prec = sizeof(R) == 8 ? kFP64 : kFP32;
   const long long ngrid = (long long)p.n1 * p.n2 * p.n3;
@@ -601,7 +607,7 @@ static int hpsi_full_grid_t(const Plan& p, const void* psi_, void* hpsi_, int nb
   const R* veff = static_cast<const R*>(veff_);
   const R* kin = prec == kFP64 ? (const R*)p.d_kin64 : (const R*)p.d_kin32;
   for (int kk = 0; kk < nkk; ++kk) {
-    const int k = k0 + kk;
+    const int k = k0 + kk, end = pad ? p.npw_pad : p.npw[k];
     for (int b0 = 0; b0 < nb; b0 += (int)cap) {
       const int nbc = (int)(nb - b0 < cap ? nb - b0 : cap);
       const C* in = psi + ((long long)kk * nb + b0) * p.npw_pad;
@@ -616,9 +622,9 @@ static int hpsi_full_grid_t(const Plan& p, const void* psi_, void* hpsi_, int nb
                          ngrid, nbc);
       if (check(hipGetLastError(), "full-grid V_eff launch")) return 1;
       if (launch_fft3d(f, prec, nbc, grids, -1, 1.0, s)) return 1;
-      hipLaunchKernelGGL((k_gather_kinetic<C, R>), dim3((p.npw[k] + 255) / 256, nbc), dim3(256), 0, s, grids, in,
+      hipLaunchKernelGGL((k_gather_kinetic<C, R>), dim3((end + 255) / 256, nbc), dim3(256), 0, s, grids, in,
                          out, p.d_flatmap + (long long)k * p.npw_pad, kin + (long long)k * p.npw_pad, p.npw[k],
-                         p.npw_pad, ngrid, (R)(1.0 / (double)ngrid));
+                         end, p.npw_pad, ngrid, (R)(1.0 / (double)ngrid));
       if (check(hipGetLastError(), "full-grid gather launch")) return 1;
     }
   }
@@ -626,9 +632,9 @@ static int hpsi_full_grid_t(const Plan& p, const void* psi_, void* hpsi_, int nb
 }
 
 int launch_hpsi_full_grid(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                          const void* veff, void* ws, size_t ws_bytes, hipStream_t s) {
-  return prec == kFP64 ? hpsi_full_grid_t<double>(p, psi, hpsi, nb, k0, nkk, veff, ws, ws_bytes, s)
-                       : hpsi_full_grid_t<float>(p, psi, hpsi, nb, k0, nkk, veff, ws, ws_bytes, s);
+                          const void* veff, void* ws, size_t ws_bytes, hipStream_t s, bool pad) {
+  return prec == kFP64 ? hpsi_full_grid_t<double>(p, psi, hpsi, nb, k0, nkk, veff, ws, ws_bytes, s, pad)
+                       : hpsi_full_grid_t<float>(p, psi, hpsi, nb, k0, nkk, veff, ws, ws_bytes, s, pad);
 }
 
 // rho = beta rho + scale sum_l w_l |u_l|^2 through whole grids; `acc` is one FP64 grid.

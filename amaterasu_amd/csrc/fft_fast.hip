@@ -25,9 +25,9 @@ int lane_plane_half_width(int n) { return lane_half_width(n); }
   if (rc < 0) rc = fn##_d(__VA_ARGS__);            \
   return rc
 
-static int stick(const Plan& p, int prec, int inverse, const void* psi, void* hpsi, void* sticks, int nb, int k0,
+static int stick(const Plan& p, int prec, int pass, const void* psi, void* hpsi, void* sticks, int nb, int k0,
                  int nkb, hipStream_t s) {
-  AMT_FIRST_PART(fast_stick, p, prec, inverse, psi, hpsi, sticks, nb, k0, nkb, s);
+  AMT_FIRST_PART(fast_stick, p, prec, pass, psi, hpsi, sticks, nb, k0, nkb, s);
 }
 static int plane(const Plan& p, int prec, void* sticks, const void* veff, int nb, int k0, int nkb, hipStream_t s) {
   AMT_FIRST_PART(fast_plane, p, prec, sticks, veff, nb, k0, nkb, s);
@@ -49,11 +49,11 @@ __global__ void k_permute_field(const R* __restrict__ src, R* __restrict__ dst, 
 }
 
 int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                     const void* veff, void* ws, hipStream_t s, int stage) {
+                     const void* veff, void* ws, hipStream_t s, int stage, bool pad) {
   const int nkb = nb * nkk;
   void* sticks = static_cast<unsigned char*>(ws) + p.field_bytes(prec);
   if (stage == 0 || stage == 1)
-    if (stick(p, prec, 1, psi, nullptr, sticks, nb, k0, nkb, s)) return 1;
+    if (stick(p, prec, kStickInverse, psi, nullptr, sticks, nb, k0, nkb, s)) return 1;
   if (stage == 0 || stage == 2) {
     const void* v = veff;
     if (p.permuted) {
@@ -71,13 +71,13 @@ int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int n
     if (plane(p, prec, sticks, v, nb, k0, nkb, s)) return 1;
   }
   if (stage == 0 || stage == 3)
-    if (stick(p, prec, 0, psi, hpsi, sticks, nb, k0, nkb, s)) return 1;
+    if (stick(p, prec, pad ? kStickForwardPad : kStickForward, psi, hpsi, sticks, nb, k0, nkb, s)) return 1;
   return 0;
 }
 
 int launch_density_fast(const Plan& p, int prec, const void* psi, int nb, int k0, int nkk, const int* list,
                         const double* weight, int nlist, int chunk, void* sticks, double* part, hipStream_t s) {
-  if (stick(p, prec, 1, psi, nullptr, sticks, nb, k0, nb * nkk, s)) return 1;
+  if (stick(p, prec, kStickInverse, psi, nullptr, sticks, nb, k0, nb * nkk, s)) return 1;
   return density(p, prec, sticks, nb, k0, list, weight, nlist, chunk, part, s) ? 1 : 0;
 }
 

@@ -34,7 +34,7 @@ constexpr int lane_count(int n, bool fp64) {
 }
 
 #define AMT_DECLARE_PART(S)                                                                                            \
-  int fast_stick_##S(const Plan& p, int prec, int inverse, const void* psi, void* hpsi, void* sticks, int nb, int k0, \
+  int fast_stick_##S(const Plan& p, int prec, int pass, const void* psi, void* hpsi, void* sticks, int nb, int k0, \
                      int nkb, hipStream_t s);                                                                          \
   int fast_plane_##S(const Plan& p, int prec, void* sticks, const void* veff, int nb, int k0, int nkb,               \
                      hipStream_t s);                                                                                   \

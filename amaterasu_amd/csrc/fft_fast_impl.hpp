@@ -70,8 +70,9 @@ __global__ __launch_bounds__(256) void k_stick_inverse_n(const C* __restrict__ p
 template <int N, typename C, typename R, int W>
 __global__ __launch_bounds__(256) void k_stick_forward_n(const C* __restrict__ sticks, const C* __restrict__ psi,
                                                          C* __restrict__ out, const int* __restrict__ stick_map,
-                                                         const R* __restrict__ kin, int smax, int npw_pad, int nb,
-                                                         int k0, const C* __restrict__ tw, R scale, int nch, int nkb) {
+                                                         const R* __restrict__ kin, const int* __restrict__ npw,
+                                                         int smax, int npw_pad, int nb, int k0,
+                                                         const C* __restrict__ tw, R scale, int nch, int nkb) {
   constexpr int T2 = ceil_div(W * Split<N>::N1, 256);
   __shared__ C tile[N * W];
   const int tid = threadIdx.x;
@@ -90,6 +91,8 @@ __global__ __launch_bounds__(256) void k_stick_forward_n(const C* __restrict__ s
   const C* cc = psi + (long long)kb * npw_pad;
   C* o = out + (long long)kb * npw_pad;
   const R* t = kin + (long long)k * npw_pad;
+  if (npw && chunk == 0)  // the row's padding
+    for (int g = npw[k] + tid; g < npw_pad; g += 256) o[g] = cmake<C>(0, 0);
   for (int e = tid; e < N * W; e += 256) {
     const int i = e / W, w = e % W, s = s0 + w;
     if (s < smax) {
@@ -689,7 +692,7 @@ struct LanePlane {
 };
 
 template <int N, typename R, int W>
-int stick_pass(const Plan& p, int inverse, const void* psi_, void* hpsi_, void* sticks_, int nb, int k0, int nkb,
+int stick_pass(const Plan& p, int pass, const void* psi_, void* hpsi_, void* sticks_, int nb, int k0, int nkb,
                hipStream_t s) {
   using C = typename Cplx<R>::T;
   constexpr int prec = sizeof(R) == 8 ? kFP64 : kFP32;
@@ -698,24 +701,25 @@ int stick_pass(const Plan& p, int inverse, const void* psi_, void* hpsi_, void* 
   const R* kin = prec == kFP64 ? (const R*)p.d_kin64 : (const R*)p.d_kin32;
   const int nch = (p.smax + W - 1) / W;
   const dim3 grid(stick_grid(nch, nkb));
-  if (inverse)
+  if (pass == kStickInverse)
     hipLaunchKernelGGL((k_stick_inverse_n<N, C, W>), grid, dim3(256), 0, s, static_cast<const C*>(psi_),
                        static_cast<C*>(sticks_), p.d_stick_map, p.smax, p.npw_pad, nb, k0, tw, nch, nkb);
   else
     hipLaunchKernelGGL((k_stick_forward_n<N, C, R, W>), grid, dim3(256), 0, s, static_cast<const C*>(sticks_),
-                       static_cast<const C*>(psi_), static_cast<C*>(hpsi_), p.d_stick_map, kin, p.smax, p.npw_pad,
+                       static_cast<const C*>(psi_), static_cast<C*>(hpsi_), p.d_stick_map, kin,
+                       pass == kStickForwardPad ? p.d_npw : nullptr, p.smax, p.npw_pad,
                        nb, k0, tw, (R)(1.0 / ((double)p.n1 * p.n2 * p.n3)), nch, nkb);
   return hipGetLastError() != hipSuccess ? 1 : 0;
 }
 
 template <int N, typename R>
-int stick_t(const Plan& p, int inverse, const void* psi, void* hpsi, void* sticks, int nb, int k0, int nkb,
+int stick_t(const Plan& p, int pass, const void* psi, void* hpsi, void* sticks, int nb, int k0, int nkb,
             hipStream_t s) {
   constexpr int prec = sizeof(R) == 8 ? kFP64 : kFP32;
   constexpr int W = stick_width<typename Cplx<R>::T>();
   return p.fast_stick_w[prec] == W / 2  // the launch shape the plan holds (autotuner)
-             ? stick_pass<N, R, W / 2>(p, inverse, psi, hpsi, sticks, nb, k0, nkb, s)
-             : stick_pass<N, R, W>(p, inverse, psi, hpsi, sticks, nb, k0, nkb, s);
+             ? stick_pass<N, R, W / 2>(p, pass, psi, hpsi, sticks, nb, k0, nkb, s)
+             : stick_pass<N, R, W>(p, pass, psi, hpsi, sticks, nb, k0, nkb, s);
 }
 
 template <int N, typename R>
@@ -767,13 +771,13 @@ int density_t(const Plan& p, const void* sticks, int nb, int k0, const int* list
 }  // namespace
 
 // The part's lengths: -1 for any other.
-int AMT_PART_FN(fast_stick)(const Plan& p, int prec, int inverse, const void* psi, void* hpsi, void* sticks, int nb,
+int AMT_PART_FN(fast_stick)(const Plan& p, int prec, int pass, const void* psi, void* hpsi, void* sticks, int nb,
                             int k0, int nkb, hipStream_t s) {
   switch (p.dim(0)) {
 #define AMT_CASE(N)                                                                     \
   case N:                                                                               \
-    return prec == kFP64 ? stick_t<N, double>(p, inverse, psi, hpsi, sticks, nb, k0, nkb, s) \
-                         : stick_t<N, float>(p, inverse, psi, hpsi, sticks, nb, k0, nkb, s);
+    return prec == kFP64 ? stick_t<N, double>(p, pass, psi, hpsi, sticks, nb, k0, nkb, s) \
+                         : stick_t<N, float>(p, pass, psi, hpsi, sticks, nb, k0, nkb, s);
     AMT_PART(AMT_CASE)
 #undef AMT_CASE
     default:

@@ -510,10 +510,91 @@ size_t zgemm_workspace_bytes(int prec, int op, int m, int n, int k, int batch) {
   return (size_t)batch * g.ns * m * n * c;
 }
 
+// Splits summed and contracted in one launch, for small products: out = P D with P the sum of the
+// partials (FP64 sums rounded to R, as k_splitk_reduce stores them) and D real, block-diagonal
+// over atoms. A workgroup takes, of one row, the columns whose atom block starts in its
+// kDijCols: with blocks of up to 33 columns it sums at most kDijPass columns, each summed by one
+// workgroup only, and keeps them in LDS. Bound by the launch and one chain of loads: 5.9 us for
+// 8 x 36 in 12 splits, where k_splitk_reduce and k_dij take 4 and 5.4 and a gap between them (H.psi
+// of 2 atoms 37 -> 31 us with the fill of H.psi gone as well). Past one workgroup per CU the two
+// kernels, with more wavefronts in flight, win: 7.7 + 6.1 us against 35-44 for 16 x 64 x 144, 17.3 +
+// 6.2 against 45 for 160 x 1152.
+constexpr long long kDijFuse = 256;  // workgroups
+constexpr int kDijCols = 96, kDijPass = 128, kDijGroups = kReduceGroups / 2;
+
+template <typename R>
+__global__ __launch_bounds__(kDijGroups * kDijPass) void k_splitk_dij(
+    int M, int N, int nsplit, const typename Cplx<R>::T* __restrict__ part, const R* __restrict__ D, long long sD,
+    const int* __restrict__ blk_start, const int* __restrict__ blk_len, typename Cplx<R>::T* __restrict__ out,
+    long long sO) {
+  using C = typename Cplx<R>::T;
+  __shared__ double red[kReduceGroups][kDijPass][2];
+  __shared__ C sum[kDijPass];
+  __shared__ int reach[kDijPass / 64];
+  const int g = threadIdx.x / kDijPass, el = threadIdx.x % kDijPass;
+  const int row = blockIdx.y, batch = blockIdx.z, first = blockIdx.x * kDijCols;
+  const long long mn = (long long)M * N;
+  const C* p = part + (long long)batch * nsplit * mn + (long long)row * N;
+  for (int w0 = first; w0 < N; w0 += kDijPass) {  // a second window for longer blocks only
+    if (w0 > first && blk_start[w0] >= first + kDijCols) break;
+    const int col = w0 + el;
+    const int j0 = col < N ? blk_start[col] : N;
+    const bool own = col < N && j0 >= first && j0 < first + kDijCols;
+    const int j1 = own ? j0 + blk_len[col] : 0;
+    int hi = j1;
+    for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
+    if (g == 0 && (el & 63) == 0) reach[el >> 6] = hi;
+    __syncthreads();
+    for (int q = 0; q < kDijPass / 64; ++q) hi = max(hi, reach[q]);
+    const R* d = D + batch * sD + col;
+    R sr = 0, si = 0;
+    for (int base = first; base < hi; base += kDijPass) {  // columns any owned block may hold
+      const int c = base + el;
+      double xr = 0, xi = 0, yr = 0, yi = 0;  // k_splitk_reduce's groups g and g + kDijGroups
+      if (c < hi)
+#pragma unroll 4
+        for (int s = g; s < nsplit; s += kReduceGroups) {
+          const C v = p[(long long)s * mn + c];
+          const C u = s + kDijGroups < nsplit ? p[(long long)(s + kDijGroups) * mn + c] : cmake<C>(0, 0);
+          xr += v.x;
+          xi += v.y;
+          yr += u.x;
+          yi += u.y;
+        }
+      red[g][el][0] = xr;
+      red[g][el][1] = xi;
+      red[g + kDijGroups][el][0] = yr;
+      red[g + kDijGroups][el][1] = yi;
+      __syncthreads();
+      if (g == 0) {
+        for (int q = 1; q < kReduceGroups; ++q) {
+          xr += red[q][el][0];
+          xi += red[q][el][1];
+        }
+        sum[el] = cmake<C>((R)xr, (R)xi);
+      }
+      __syncthreads();
+      if (g == 0 && own)
+#pragma unroll 4
+        for (int j = max(j0, base); j < min(j1, base + kDijPass); ++j) {
+          const R dj = d[(long long)j * N];
+          sr += sum[j - base].x * dj;
+          si += sum[j - base].y * dj;
+        }
+      __syncthreads();
+    }
+    if (g == 0 && own) out[batch * sO + (long long)row * N + col] = cmake<C>(sr, si);
+    __syncthreads();
+  }
+}
+
+int launch_dij(int prec, const void* P, const void* D, const int* blk_start, const int* blk_len, void* out, int nrow,
+               int nproj, long long sP, long long sD, long long sO, int batch, hipStream_t s);
+
 template <typename R>
 static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, long long lda, long long sa,
                    const void* b, long long ldb, long long sb, double beta, void* c, long long ldc, long long sc,
-                   int batch, void* ws, size_t ws_bytes, hipStream_t s) {
+                   int batch, void* ws, size_t ws_bytes, hipStream_t s, const DijArgs* dij = nullptr) {
   using C = typename Cplx<R>::T;
   if (m <= 0 || n <= 0 || batch <= 0) return 0;
   const GemmPlan g = plan_gemm(std::is_same<R, double>::value ? kFP64 : kFP32, op, m, n, k, batch);
@@ -564,7 +645,17 @@ static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, lon
     set_error(std::string("zgemm launch: ") + hipGetErrorString(e));
     return 1;
   }
-  if (ns > 1) {
+  const bool fuse = dij && ns > 1 && (long long)((n + kDijCols - 1) / kDijCols) * m * batch <= kDijFuse;
+  if (fuse) {
+    hipLaunchKernelGGL((k_splitk_dij<R>), dim3((n + kDijCols - 1) / kDijCols, m, batch),
+                       dim3(kDijGroups * kDijPass), 0, s, m, n, ns, (const C*)part, (const R*)dij->d, dij->sd,
+                       dij->blk_start, dij->blk_len, (C*)dij->out, dij->so);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
+      set_error(std::string("zgemm contraction launch: ") + hipGetErrorString(e));
+      return 1;
+    }
+  } else if (ns > 1) {
     const long long mn = (long long)m * n;
     hipLaunchKernelGGL((k_splitk_reduce<R>), dim3((unsigned)((mn + kReduceCols - 1) / kReduceCols), batch),
                        dim3(kReduceGroups * kReduceCols), 0, s, m, n, ns, (const C*)part, (C*)c, ldc, sc, (R)alpha,
@@ -575,6 +666,9 @@ static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, lon
       return 1;
     }
   }
+  if (dij && !fuse)
+    return launch_dij(std::is_same<R, double>::value ? kFP64 : kFP32, c, dij->d, dij->blk_start, dij->blk_len, dij->out,
+                      m, n, sc, dij->sd, dij->so, batch, s);
   return 0;
 }
 
@@ -585,6 +679,15 @@ int launch_zgemm(int prec, int op, int m, int n, int k, double alpha, const void
                                          ws_bytes, s)
                        : zgemm_t<float>(op, m, n, k, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, batch, ws,
                                         ws_bytes, s);
+}
+
+int launch_zgemm_dij(int prec, int m, int n, int k, const void* a, long long lda, long long sa, const void* b,
+                     long long ldb, long long sb, void* proj, const DijArgs& dij, int batch, void* ws, size_t ws_bytes,
+                     hipStream_t s) {
+  return prec == kFP64 ? zgemm_t<double>(1, m, n, k, 1.0, a, lda, sa, b, ldb, sb, 0.0, proj, n, (long long)m * n, batch,
+                                         ws, ws_bytes, s, &dij)
+                       : zgemm_t<float>(1, m, n, k, 1.0, a, lda, sa, b, ldb, sb, 0.0, proj, n, (long long)m * n, batch,
+                                        ws, ws_bytes, s, &dij);
 }
 
 }  // namespace amt

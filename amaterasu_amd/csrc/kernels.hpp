@@ -86,19 +86,23 @@ struct Plan {
 
 void set_error(const std::string& msg);
 
+// The passes of the stick kernels, and `pad` of the H.psi launchers: the forward pass also writes
+// zeros to the columns past each k-point's plane waves (amt_hpsi; amt_hpsi_local leaves them).
+enum StickPass { kStickForward = 0, kStickInverse = 1, kStickForwardPad = 2 };
+
 // Compile-time-length kernels (fft_fast.hip) for grids with two axes of one listed length.
 bool fast_length_supported(int n);
 bool lane_plane_supported(int n, int prec);
 int lane_plane_half_width(int n);
 int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                     const void* veff, void* sticks, hipStream_t s, int stage);
+                     const void* veff, void* sticks, hipStream_t s, int stage, bool pad = false);
 int launch_density_fast(const Plan& p, int prec, const void* psi, int nb, int k0, int nkk, const int* list,
                         const double* weight, int nlist, int chunk, void* sticks, double* part, hipStream_t s);
 
 // Local part of H.psi (kinetic + V_eff) for nbk = nkb bands laid out [kb][npw_pad],
 // kb = k * nb + b for k in [k0, k0 + nkb / nb). `sticks` is nkb * n1 * smax complex.
 int launch_hpsi_local(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                      const void* veff, void* sticks, hipStream_t s, int stage = 0);
+                      const void* veff, void* sticks, hipStream_t s, int stage = 0, bool pad = false);
 // launch_hpsi_local over the library's fixed scratch array (noalloc.hip).
 long long noalloc_rows_per_launch(const Plan& p, int prec);
 int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
@@ -112,7 +116,7 @@ int launch_density(const Plan& p, int prec, const void* psi, int nb, int k0, int
 // fit one workgroup's LDS; full_grid_rows = grids the workspace holds.
 long long full_grid_rows(const Plan& p, int prec, size_t ws_bytes);
 int launch_hpsi_full_grid(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                          const void* veff, void* ws, size_t ws_bytes, hipStream_t s);
+                          const void* veff, void* ws, size_t ws_bytes, hipStream_t s, bool pad = false);
 int launch_density_full_grid(const Plan& p, int prec, const void* psi, int nb, int k0, const int* list,
                              const double* weight, int nlist, void* ws, size_t ws_bytes, double* acc, double* rho,
                              double beta, double scale, hipStream_t s);
@@ -133,6 +137,19 @@ int launch_fft3d(const FftPlan& fp, int prec, int batch, void* data, int sign, d
 int launch_zgemm(int prec, int op, int m, int n, int k, double alpha, const void* a, long long lda,
                  long long sa, const void* b, long long ldb, long long sb, double beta, void* c, long long ldc,
                  long long sc, int batch, void* ws, size_t ws_bytes, hipStream_t s);
+// P = a b^H [m][n] followed by out = P D (D real [n][n], block-diagonal: blk_start/blk_len per
+// column); `proj` holds P where the product is not split along K.
+struct DijArgs {
+  const void* d;
+  long long sd;
+  const int *blk_start, *blk_len;
+  void* out;
+  long long so;
+};
+int launch_zgemm_dij(int prec, int m, int n, int k, const void* a, long long lda, long long sa, const void* b,
+                     long long ldb, long long sb, void* proj, const DijArgs& dij, int batch, void* ws, size_t ws_bytes,
+                     hipStream_t s);
+
 size_t zgemm_workspace_bytes(int prec, int op, int m, int n, int k, int batch);
 int set_zgemm_split(int prec, int op, int m, int n, int k, int batch, int split);
 

@@ -206,7 +206,8 @@ class DevicePlan:
         if v.numel() != self.shape[0] * self.shape[1] * self.shape[2]:
             raise AmtError("effective potential does not match the grid")
         if out is None:
-            h = torch.zeros_like(p3)
+            # amt_hpsi writes every element, zeros on the padding
+            h = torch.empty_like(p3) if coupling is None else torch.zeros_like(p3)
         else:
             h = out.unsqueeze(0) if out.dim() == 2 else out
             if tuple(h.shape) != tuple(p3.shape) or h.dtype != p3.dtype or not h.is_contiguous():

@@ -103,7 +103,8 @@ size_t amt_hpsi_workspace(const amt_plan_t* plan, int precision, int nb, int nk)
  *   hpsi = T_G psi + gather(FFT(V_eff . IFFT(scatter psi))) + (psi beta^H) D beta
  * for nb bands at each of the k-points k0..k0+nk-1 ([nk][nb][npw_pad], the projector term of
  * KBProjectors.apply, pseudo/kb.py:216-230, with the tables of amt_plan_set_projectors; no
- * projector term when none are attached). `ws` holds amt_hpsi_workspace(...) bytes.
+ * projector term when none are attached). Every element of hpsi is written, zeros on the padded
+ * columns. `ws` holds amt_hpsi_workspace(...) bytes.
  */
 int amt_hpsi(const amt_plan_t* plan, int precision, const void* psi, void* hpsi, int nb, int k0, int nk,
              const void* veff, void* ws, size_t ws_bytes, void* stream);

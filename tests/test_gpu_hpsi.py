@@ -346,3 +346,70 @@ def test_plane_kernels_match_full_grid_route(shape):
             bound = 64 * u * np.log2(np.prod(shape))
             assert float((got - want).abs().max() / want.abs().max()) < bound, (half, prec)
             assert float((rho - rho_want).abs().max() / rho_want.abs().max()) < bound, (half, prec)
+
+
+@pytest.mark.parametrize("route", ["plane", "full grid"])
+@pytest.mark.parametrize("split", [1, 7])
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+@pytest.mark.parametrize("blocks", [[1], [8, 8, 8, 8], [1, 5, 18, 40, 130, 7], [31, 33, 97]])
+def test_projector_contraction_and_padding(si2_system, blocks, dtype, split, route):
+    """amt_hpsi with projector tables of any block lengths, with the first product split along the
+    plane waves (splits summed and contracted in one launch) and not, against the local part plus
+    the dense (psi beta^H) D beta in FP64: within the rounding of sums of npw, block and nproj
+    terms. The output starts as NaN, so every element, padding included, has to be written."""
+    import torch
+
+    from amaterasu_amd import ops
+    from amaterasu_amd._lib import check, lib
+    from amaterasu_amd.hamiltonian import Hamiltonian
+
+    dt = getattr(torch, dtype)
+    rng = np.random.default_rng(len(blocks))
+    v = rng.normal(size=(1, *si2_system.grid.shape))
+    ham = Hamiltonian(si2_system, v, precision="fp64" if dtype == "complex128" else "fp32")
+    plan = ham.plan
+    plan.set_projectors(None)
+    prec, nk, nb, np_, npw = ops.precision_of(torch.empty(0, dtype=dt)), plan.nk, 5, sum(blocks), plan.npw_pad
+    rdt = ops.real_dtype(prec)
+    live = torch.zeros(nk, 1, npw, dtype=torch.float64, device="cuda")
+    for k in range(nk):
+        live[k, :, : plan.npw[k]] = 1.0
+    rand = lambda *s: torch.randn(*s, dtype=torch.complex128, device="cuda")  # noqa: E731
+    torch.manual_seed(3)
+    psi, beta = (rand(nk, nb, npw) * live).to(dt), (rand(nk, np_, npw) * live).to(dt)
+    dij = torch.zeros(nk, np_, np_, dtype=rdt, device="cuda")
+    starts = np.concatenate([[0], np.cumsum(blocks)])
+    for a, n in zip(starts, blocks):
+        d = torch.randn(nk, n, n, device="cuda", dtype=rdt)
+        dij[:, a : a + n, a : a + n] = d + d.transpose(1, 2)
+    start = torch.as_tensor(np.repeat(starts[:-1], blocks).astype(np.int32), device="cuda")
+    length = torch.as_tensor(np.repeat(blocks, blocks).astype(np.int32), device="cuda")
+    if route == "full grid":
+        plan.set_route(prec, True)
+    try:
+        veff = ham.veff(0, prec)
+        local = plan.hpsi(psi, veff)
+        check(lib().amt_plan_set_projectors(plan.handle, prec, np_, beta.data_ptr(), dij.data_ptr(), start.data_ptr(),
+                                            length.data_ptr()), "set_projectors")
+        check(lib().amt_zgemm_set_split(prec, 1, nb, np_, npw, nk, split), "set_split")
+        out = torch.full_like(psi, float("nan"))
+        nbytes = lib().amt_hpsi_workspace(plan.handle, prec, nb, nk)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        check(lib().amt_hpsi(plan.handle, prec, psi.data_ptr(), out.data_ptr(), nb, 0, nk, veff.data_ptr(), ws.data_ptr(),
+                             nbytes, ops.stream_handle()), "hpsi")
+    finally:
+        lib().amt_zgemm_set_split(prec, 1, nb, np_, npw, nk, 0)
+        lib().amt_plan_set_projectors(plan.handle, prec, 0, None, None, None, None)
+        if route == "full grid":
+            plan.set_route(prec, False)
+    cpu = lambda t: t.cpu().to(torch.complex128)  # noqa: E731
+    p64, b64, d64 = cpu(psi), cpu(beta), cpu(dij)
+    want = cpu(local)
+    size = want.abs()
+    for k in range(nk):
+        want[k] += (p64[k] @ b64[k].conj().T.contiguous()) @ d64[k] @ b64[k]
+        size[k] += (p64[k].abs() @ b64[k].abs().T.contiguous()) @ d64[k].abs() @ b64[k].abs()
+    u = 2.0**-53 if dtype == "complex128" else 2.0**-24
+    # sums of length n err by at most about sqrt(n) u of the sum of absolute values here (random signs), 4 for the parts
+    assert ((cpu(out) - want).abs() <= 4 * np.sqrt(npw + max(blocks) + np_) * u * size + 1e-300).all()
+    assert not out[live.expand(nk, nb, npw) == 0].any() and out.isfinite().all()
