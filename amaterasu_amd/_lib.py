@@ -39,6 +39,9 @@ SIGNATURES = {
     "amt_density_part_bytes": (_c_sz, [_vp, _c_int, _c_int]),
     "amt_density": (_c_int, [_vp, _c_int, _vp, _c_int, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _vp, _vp, _vp,
                              _c_dbl, _c_dbl, _vp]),
+    "amt_density_chunk": (_c_int, [_vp, _c_int, _c_int]),
+    "amt_density_finish_bytes": (_c_sz, [_c_int]),
+    "amt_density_finish": (_c_int, [_vp, _c_int, _c_ll, _c_dbl, _vp, _vp]),
     "amt_scatter": (_c_int, [_vp, _c_int, _vp, _vp, _c_int, _c_int, _vp]),
     "amt_gather": (_c_int, [_vp, _c_int, _vp, _vp, _c_int, _c_int, _c_dbl, _vp]),
     "amt_fft_plan_create": (_c_int, [ctypes.POINTER(_vp), _c_int, _c_int, _c_int]),

@@ -591,6 +591,21 @@ int amt_density(const amt_plan_t* h, int precision, const void* psi, int nb, int
                         beta, scale, (hipStream_t)stream);
 }
 
+int amt_density_chunk(const amt_plan_t* h, int precision, int nlist) {
+  if (!h || (precision != kFP32 && precision != kFP64)) return 8;
+  return density_chunk(h->p, precision, nlist);
+}
+
+size_t amt_density_finish_bytes(int nspin) { return nspin > 0 ? density_finish_bytes(nspin) : 0; }
+
+int amt_density_finish(double* rho, int nspin, long long ngrid, double volume, double* part, void* stream) {
+  if (!rho || !part || nspin < 1 || nspin > 65535 || ngrid < 1) {
+    set_error("density_finish: bad argument");
+    return 1;
+  }
+  return launch_density_finish(rho, nspin, ngrid, volume, part, (hipStream_t)stream);
+}
+
 int amt_scatter(const amt_plan_t* h, int precision, const void* psi, void* grid, int nb, int k, void* stream) {
   if (!h || !psi || !grid || nb <= 0 || k < 0 || k >= h->p.nk) {
     set_error("scatter: bad argument");

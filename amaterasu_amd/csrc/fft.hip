@@ -320,6 +320,88 @@ __global__ void k_density_reduce(const double* __restrict__ part, int nchunk, lo
   }
 }
 
+// rho / volume, floored at zero and rescaled to the charge before the floor, per spin. Two launches:
+// block sums of x and max(x, 0) with x = rho / volume, then every block adds those up in the same
+// order and writes its part. Two reads and one write of rho (11 us at 84^3, where a division, two
+// sums, a clamp and a product with their scalar steps took 60).
+static int check(hipError_t e, const char* what);
+constexpr int kFinishBlocks = 256;
+__device__ __forceinline__ double floor_at_zero(double x) { return x < 0.0 ? 0.0 : x; }  // keeps NaN
+__global__ __launch_bounds__(256) void k_density_sums(const double* __restrict__ rho, long long ngrid, double volume,
+                                                      double* __restrict__ part) {
+  __shared__ double red[2][4];
+  const double* r = rho + (long long)blockIdx.y * ngrid;
+  double all = 0.0, kept = 0.0;
+  for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < ngrid; e += (long long)gridDim.x * 256) {
+    const double x = r[e] / volume;
+    all += x;
+    kept += floor_at_zero(x);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    all += __shfl_down(all, o, 64);
+    kept += __shfl_down(kept, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = all;
+    red[1][threadIdx.x >> 6] = kept;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const double* q = red[threadIdx.x];
+    part[((long long)blockIdx.y * gridDim.x + blockIdx.x) * 2 + threadIdx.x] = (q[0] + q[1]) + (q[2] + q[3]);
+  }
+}
+__global__ __launch_bounds__(256) void k_density_floor(double* __restrict__ rho, long long ngrid, double volume,
+                                                       const double* __restrict__ part) {
+  __shared__ double red[2][256];
+  const int t = threadIdx.x;
+  const double* p = part + (long long)blockIdx.y * gridDim.x * 2;
+  red[0][t] = t < (int)gridDim.x ? p[2 * t] : 0.0;
+  red[1][t] = t < (int)gridDim.x ? p[2 * t + 1] : 0.0;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if (t < o) {
+      red[0][t] += red[0][t + o];
+      red[1][t] += red[1][t + o];
+    }
+    __syncthreads();
+  }
+  const double before = red[0][0], after = red[1][0], scale = after > 0.0 ? before / after : 1.0;
+  double* r = rho + (long long)blockIdx.y * ngrid;
+  for (long long e = (long long)blockIdx.x * 256 + t; e < ngrid; e += (long long)gridDim.x * 256)
+    r[e] = floor_at_zero(r[e] / volume) * scale;
+}
+size_t density_finish_bytes(int nspin) { return (size_t)nspin * kFinishBlocks * 2 * sizeof(double); }
+int launch_density_finish(double* rho, int nspin, long long ngrid, double volume, double* part, hipStream_t s) {
+  const long long want = (ngrid + 255) / 256;
+  const dim3 grid((unsigned)(want < kFinishBlocks ? want : kFinishBlocks), nspin);
+  hipLaunchKernelGGL(k_density_sums, grid, dim3(256), 0, s, rho, ngrid, volume, part);
+  hipLaunchKernelGGL(k_density_floor, grid, dim3(256), 0, s, rho, ngrid, volume, part);
+  return check(hipGetLastError(), "density_finish launch");
+}
+
+// Bands per workgroup of the plane accumulation, by the rounds of workgroups the chip runs (one
+// or two per CU, by the plane's LDS) times the bands of each, one more band for a workgroup's
+// start and its write of a partial plane. 84^3 in FP64, 128 bands: 43 bands fill one round of
+// 252 workgroups (422 us), 8 take 5.25 rounds of 16 (484); 16 bands: 6 (97 us against 107 for 8);
+// 42^3, 128 bands: 11 or 22 (123, 120; 8: 131); 25^3: 4 to 8 alike.
+int density_chunk(const Plan& p, int prec, int nlist) {
+  if (!p.fast || nlist < 1) return 8;
+  const long long plane = (long long)p.dim(1) * p.dim(2) * (prec == kFP64 ? 16 : 8), n1 = p.dim(0);
+  const long long slots = 256 * (2 * (plane + 4096) <= 160 * 1024 ? 2 : 1);
+  long long best = 0, cost = 0;
+  for (long long c = 1; c <= nlist; ++c) {
+    const long long nch = (nlist + c - 1) / c;
+    if (nch > 65535) continue;
+    const long long t = (nch * n1 + slots - 1) / slots * (c + 1);
+    if (best == 0 || t <= cost) {
+      best = c;
+      cost = t;
+    }
+  }
+  return (int)best;
+}
+
 // --------------------------------------------------------------------------- full-grid route
 // For grids whose (n2 x n3) plane does not fit one workgroup's LDS at a precision (FP64 planes
 // above ~100^2): whole grids through the library's scatter, 3-D transforms and gather, a chunk

@@ -81,7 +81,9 @@ struct Plan {
   bool whole_plane[2] = {false, false};  // a whole plane fits LDS: density kernel and allocation-free call
   // launch shapes of the compile-time-length kernels (amt_plan_set_launch; an autotuner picks them)
   int plane_nth[2] = {256, 256};   // plane kernel workgroup: 256 or 512 threads
-  int fast_stick_w[2] = {64, 32};  // sticks per workgroup of the stick kernels: the default or half
+  // Sticks per workgroup of the stick kernels, until the tuner has timed both (64 and 32, 32 and 16):
+  // the narrower one won 9 of 10 passes at lengths 25, 42 and 84 by 3 to 29 % and lost one by 7 %.
+  int fast_stick_w[2] = {32, 16};
 };
 
 void set_error(const std::string& msg);
@@ -109,6 +111,9 @@ int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int
                        const void* veff, hipStream_t s);
 // sum over listed bands of w |u(r)|^2 into part[chunk][N] (double), then
 // rho = beta * rho + scale * sum_chunks part.
+int density_chunk(const Plan& p, int prec, int nlist);
+int launch_density_finish(double* rho, int nspin, long long ngrid, double volume, double* part, hipStream_t s);
+size_t density_finish_bytes(int nspin);
 int launch_density(const Plan& p, int prec, const void* psi, int nb, int k0, int nkk, const int* d_band_list,
                    const double* d_band_weight, int nlist, int chunk, void* sticks, double* part, double* rho,
                    double beta, double scale, hipStream_t s);

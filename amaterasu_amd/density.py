@@ -14,6 +14,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from . import ops
 from .hamiltonian import device_plan
 
 
@@ -42,8 +43,9 @@ def compute_density(system, wavefunctions, occupations, *, symmetrize: bool = Tr
     g = 2.0 / nspin
     occ = np.asarray(occupations.cpu() if isinstance(occupations, torch.Tensor) else occupations, dtype=float)
     weights = np.asarray(system.kpoints.weights, dtype=float)
-    rho = torch.zeros((nspin, *shape), dtype=torch.float64, device="cuda")
+    rho = torch.empty((nspin, *shape), dtype=torch.float64, device="cuda")
     for s in range(nspin):
+        beta = 0.0  # the first k-point with occupied bands writes, the others add
         for ik in range(len(system.wave_spheres)):
             f = g * weights[ik] * occ[s, ik]
             act = np.flatnonzero(f > 1e-12)
@@ -59,18 +61,18 @@ def compute_density(system, wavefunctions, occupations, *, symmetrize: bool = Tr
                 pad = torch.zeros((psi.shape[0], plan.npw_pad), dtype=psi.dtype, device=psi.device)
                 pad[:, :npw] = psi
                 psi = pad
-            plan.accumulate_density(psi.contiguous(), act.astype(np.int32), f[act], rho[s], k0=ik, beta=1.0,
-                                    scale=1.0)
-    rho /= system.grid.volume
-    if symmetrize:
-        if not _trivial_symmetry(system):
+            plan.accumulate_density(psi.contiguous(), act.astype(np.int32), f[act], rho[s], k0=ik, beta=beta,
+                                    scale=1.0, chunk=plan.density_chunk(psi.dtype, act.size))
+            beta = 1.0
+        if beta == 0.0:
+            rho[s].zero_()
+    if symmetrize and _trivial_symmetry(system):
+        rho = ops.finish_density(rho, system.grid.volume)
+    else:
+        rho /= system.grid.volume
+        if symmetrize:
             rho = torch.from_numpy(np.asarray(system.symmetrize_density(rho.cpu().numpy()))).to("cuda")
-        before = rho.sum(dim=(-3, -2, -1))
-        clipped = torch.clamp(rho, min=0.0)
-        after = clipped.sum(dim=(-3, -2, -1))
-        scale = torch.where(after > 0, before / torch.where(after > 0, after, torch.ones_like(after)),
-                            torch.ones_like(after))
-        rho = clipped * scale[:, None, None, None]
+            rho = ops.finish_density(rho.to(torch.float64).contiguous())
     return rho if device else rho.cpu().numpy()
 
 

@@ -279,6 +279,10 @@ class DevicePlan:
                                 nlist, chunk, st.data_ptr(), part.data_ptr(), rho.data_ptr(), float(beta),
                                 float(scale), ops.stream_handle()), "density")
 
+    def density_chunk(self, dtype, nlist: int) -> int:
+        """Bands per workgroup that suit ``nlist`` bands of ``dtype`` (amt_density_chunk)."""
+        return lib().amt_density_chunk(self._handle, FP64 if dtype == torch.complex128 else FP32, int(nlist))
+
     # ---------------------------------------------------------------- maps
     def scatter(self, psi: torch.Tensor, k: int) -> torch.Tensor:
         p2 = psi.unsqueeze(0) if psi.dim() == 1 else psi

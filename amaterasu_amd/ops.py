@@ -337,3 +337,17 @@ def heev_lowest_batched(a: torch.Tensor, sizes, nev: int):
           "heev_batched")
     return w, zt
 
+
+
+def finish_density(rho: torch.Tensor, volume: float = 1.0) -> torch.Tensor:
+    """``rho / volume`` per spin, floored at zero and rescaled to the charge before the floor, in
+    place (float64 ``[nspin][...]``); see amt_density_finish."""
+    _require(rho, "rho")
+    if rho.dtype != torch.float64 or rho.dim() < 2:
+        raise AmtError("finish_density: rho must be float64 [nspin][...]")
+    nspin = rho.shape[0]
+    if rho.numel():
+        part = workspace(lib().amt_density_finish_bytes(nspin), "density_finish")
+        check(lib().amt_density_finish(rho.data_ptr(), nspin, rho.numel() // nspin, float(volume), part.data_ptr(),
+                                       stream_handle()), "density_finish")
+    return rho

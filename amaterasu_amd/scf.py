@@ -508,13 +508,8 @@ def run_scf(system, settings: SCFSettings, *, density=None, wavefunctions=None, 
             f = f_all[sp].reshape(-1).cpu().numpy()
             act = np.flatnonzero(f > 1e-12)
             plan.accumulate_density(wf[sp], act.astype(np.int32), f[act], dout[sp], k0=0, beta=0.0,
-                                    scale=1.0 / system.grid.volume)
-        dout = side.symmetrize(dout)
-        before = dout.sum(dim=(-3, -2, -1))
-        clipped = torch.clamp(dout, min=0.0)
-        after = clipped.sum(dim=(-3, -2, -1))
-        dout = clipped * torch.where(after > 0, before / torch.where(after > 0, after, torch.ones_like(after)),
-                                     torch.ones_like(after))[:, None, None, None]
+                                    scale=1.0 / system.grid.volume, chunk=plan.density_chunk(wf.dtype, act.size))
+        dout = ops.finish_density(side.symmetrize(dout).to(torch.float64).contiguous())
         # energies at the output density
         eh, _ = side.hartree(dout.sum(0))
         xd = dout if core is None else dout + core[None] / nspin

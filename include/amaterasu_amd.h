@@ -142,6 +142,16 @@ int amt_density(const amt_plan_t* plan, int precision, const void* psi, int nb, 
                 const int* band_list, const double* band_weight, int nlist, int chunk, void* sticks,
                 double* part, double* rho, double beta, double scale, void* stream);
 
+/* The chunk that suits nlist bands on this plan's grid (for amt_density). */
+int amt_density_chunk(const amt_plan_t* plan, int precision, int nlist);
+/*
+ * End of compute_density (scf/density.py:71-84): per spin, x = rho / volume, floored at zero and
+ * rescaled to the sum of x. rho is float64 [nspin][ngrid], in place; part holds
+ * amt_density_finish_bytes(nspin).
+ */
+size_t amt_density_finish_bytes(int nspin);
+int amt_density_finish(double* rho, int nspin, long long ngrid, double volume, double* part, void* stream);
+
 /* FFTGrid.scatter (basis/fft.py:192-206): zero grid, place nb rows of sphere k. */
 int amt_scatter(const amt_plan_t* plan, int precision, const void* psi, void* grid, int nb, int k, void* stream);
 /* FFTGrid.gather (basis/fft.py:208-212) times `scale`; padded columns are zeroed. */

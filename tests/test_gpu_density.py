@@ -56,3 +56,57 @@ def test_density_generic_grid(si2_system):
     occ[:, :, :5] = 0.8
     got, ref = compute_density(s, wf, occ), ocd(s, wf, occ)
     assert np.abs(got - ref).max() / np.abs(ref).max() < 1e-12
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (2, 255), (1, 257), (2, 65537), (3, 200000)])
+@pytest.mark.parametrize("kind", ["mixed", "zero", "negative", "nan"])
+def test_finish_density(shape, kind):
+    """Division, floor and rescaling per spin against the formula: a sum over n numbers of
+    size 1 errs by at most n u of the sum of sizes, relative to a kept sum of at least a third of it."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    rng = np.random.default_rng(shape[1])
+    x = rng.normal(size=shape) + 0.8
+    if kind == "zero":
+        x[:] = 0.0
+    elif kind == "negative":
+        x = -np.abs(x)
+    elif kind == "nan":
+        x[0, -1] = np.nan
+    v = 3.7
+    y = x / v
+    kept = np.where(y < 0, 0.0, y)
+    before, after = y.sum(1), kept.sum(1)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        scale = np.where(after > 0, before / np.where(after > 0, after, 1.0), 1.0)
+    want = kept * scale[:, None]
+    got = ops.finish_density(torch.from_numpy(x.copy()).cuda(), v).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert (np.abs(got - want)[ok] <= 6 * shape[1] * 2.0**-53 * np.abs(kept).max(initial=0.0, where=ok) + 0.0).all()
+
+
+@pytest.mark.parametrize("dtype", ["complex64", "complex128"])
+@pytest.mark.parametrize("nlist", [1, 2, 3, 7, 12])
+def test_density_chunk_choice(si2_system, nlist, dtype):
+    """The chosen chunk sums the same squares as one band per chunk, in another order."""
+    import torch
+
+    from amaterasu_amd.hamiltonian import device_plan
+
+    plan = device_plan(si2_system)
+    psi = torch.randn(2, 6, plan.npw_pad, dtype=getattr(torch, dtype), device="cuda") / np.sqrt(plan.npw_pad)
+    for k in range(2):
+        psi[k, :, plan.npw[k] :] = 0
+    rows = np.arange(nlist, dtype=np.int32)
+    w = np.linspace(0.3, 1.7, nlist)
+    chunk = plan.density_chunk(psi.dtype, nlist)
+    assert 1 <= chunk <= max(nlist, 8)
+    out = []
+    for c in (chunk, 1):
+        rho = torch.full(plan.shape, float("nan"), dtype=torch.float64, device="cuda")
+        plan.accumulate_density(psi, rows, w, rho, beta=0.0, chunk=c)
+        out.append(rho.cpu().numpy())
+    assert np.abs(out[0] - out[1]).max() <= 2 * nlist * 2.0**-53 * np.abs(out[1]).max()
