@@ -64,6 +64,7 @@ SIGNATURES = {
     "amt_chol_workspace": (_c_sz, [_c_int, _c_int]),
     "amt_chol_inverse": (_c_int, [_c_int, _c_int, _vp, _vp, _c_int, _vp, _vp, _vp, _c_sz, _vp]),
     "amt_lowdin": (_c_int, [_c_int, _c_int, _vp, _vp, _vp, _vp]),
+    "amt_gga": (_c_int, [_c_ll, _vp, _vp, _vp, _vp, _vp, _dp, _vp, _vp]),
     "amt_mlp_param_count": (_c_int, []),
     "amt_mlp_features": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _ip, _c_dbl, _c_dbl, _vp, _vp]),
     "amt_mlp_forward": (_c_int, [_vp, _c_ll, _vp, _vp, _vp, _vp, _vp]),

@@ -19,7 +19,7 @@ BUILD = HERE / "_build"
 ARCH = os.environ.get("AMT_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["abi.cpp", "fft.hip", "fft_fast.hip", "fft_fast_a.hip", "fft_fast_b.hip", "fft_fast_c.hip",
-           "fft_fast_d.hip", "gemm.hip", "dav.hip", "mlp.hip", "eig.hip", "chol.hip",
+           "fft_fast_d.hip", "gemm.hip", "dav.hip", "mlp.hip", "eig.hip", "chol.hip", "xc.hip",
            "noalloc.hip"]
 LIBS: list = []
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

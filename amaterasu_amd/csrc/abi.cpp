@@ -596,6 +596,16 @@ int amt_density_chunk(const amt_plan_t* h, int precision, int nlist) {
   return density_chunk(h->p, precision, nlist);
 }
 
+int amt_gga(long long n, const double* up, const double* dn, const double* suu, const double* sud, const double* sdd,
+            const double* parameters, double* out, void* stream) {
+  if (n < 1 || (n + 255) / 256 > 0x7fffffff || !up || !dn || !suu || !sud || !sdd || !parameters || !out) {
+    set_error("gga: bad argument");
+    return 1;
+  }
+  double* const o[6] = {out, out + n, out + 2 * n, out + 3 * n, out + 4 * n, out + 5 * n};
+  return launch_gga(n, up, dn, suu, sud, sdd, parameters, o, (hipStream_t)stream);
+}
+
 size_t amt_density_finish_bytes(int nspin) { return nspin > 0 ? density_finish_bytes(nspin) : 0; }
 
 int amt_density_finish(double* rho, int nspin, long long ngrid, double volume, double* part, void* stream) {

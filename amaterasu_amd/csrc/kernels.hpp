@@ -111,6 +111,8 @@ int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int
                        const void* veff, hipStream_t s);
 // sum over listed bands of w |u(r)|^2 into part[chunk][N] (double), then
 // rho = beta * rho + scale * sum_chunks part.
+int launch_gga(long long n, const double* up, const double* dn, const double* suu, const double* sud, const double* sdd,
+               const double par[4], double* const out[6], hipStream_t s);
 int density_chunk(const Plan& p, int prec, int nlist);
 int launch_density_finish(double* rho, int nspin, long long ngrid, double volume, double* part, hipStream_t s);
 size_t density_finish_bytes(int nspin);

@@ -351,3 +351,19 @@ def finish_density(rho: torch.Tensor, volume: float = 1.0) -> torch.Tensor:
         check(lib().amt_density_finish(rho.data_ptr(), nspin, rho.numel() // nspin, float(volume), part.data_ptr(),
                                        stream_handle()), "density_finish")
     return rho
+
+
+def gga(up, dn, suu, sud, sdd, parameters) -> torch.Tensor:
+    """``[6][...]``: energy per particle, potentials and gradient derivatives of the PBE form at
+    every point (float64); ``parameters`` = (kappa, mu, beta, gamma). See amt_gga."""
+    fields = [f.contiguous() for f in (up, dn, suu, sud, sdd)]
+    for f in fields:
+        _require(f, "gga field")
+        if f.dtype != torch.float64 or f.shape != fields[0].shape:
+            raise AmtError("gga: float64 fields of one shape")
+    out = torch.empty((6, *fields[0].shape), dtype=torch.float64, device=fields[0].device)
+    n = fields[0].numel()
+    if n:
+        check(lib().amt_gga(n, *(f.data_ptr() for f in fields), (ctypes.c_double * 4)(*parameters), out.data_ptr(),
+                            stream_handle()), "gga")
+    return out

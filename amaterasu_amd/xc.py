@@ -5,9 +5,9 @@ The pointwise forms are those of ``amaterasu/xc/lda.py`` and ``amaterasu/xc/gga.
 enhancement factor and gradient correction written with log1p/expm1); the grid driver
 follows ``amaterasu/xc/driver.py:108-164``: an unpolarised density is evaluated as n/2
 in both spin channels, gradients and the divergence of the GGA flux are taken in
-reciprocal space with the Nyquist plane blanked (``basis/fft.py:254-304``). Every
-elementwise step is a torch FP64 operation on the device; the transforms are
-libamaterasu_amd's batched 3D FFT.
+reciprocal space with the Nyquist plane blanked (``basis/fft.py:254-304``). The
+PBE form is one pointwise kernel, the LDA's elementwise steps are torch FP64 operations on the
+device; the transforms are libamaterasu_amd's batched 3D FFT.
 """
 
 from __future__ import annotations
@@ -20,12 +20,10 @@ from . import ops
 X_FACTOR_C = 0.9305257363491000250020102180716672510262
 RS_FACTOR = 0.6203504908994000166680068120477781673508
 DENSITY_THRESHOLD = 1e-24
-X2S = 0.1282782438530421943003109254455883701296
 _FZ_DEN = 2.0 ** (4.0 / 3.0) - 2.0
 _PW92 = {"a": (0.031091, 0.015545, 0.016887), "alpha1": (0.21370, 0.20548, 0.11125),
          "beta1": (7.5957, 14.1189, 10.357), "beta2": (3.5876, 6.1977, 3.6231),
          "beta3": (1.6382, 3.3662, 0.88026), "beta4": (0.49294, 0.62517, 0.49671), "fz20": 1.709921}
-_PW92_MOD = {**_PW92, "a": (0.0310907, 0.01554535, 0.0168869), "fz20": 1.709920934161365617563962776245}
 #: Perdew-Zunger 1981 correlation, (unpolarised, polarised) (``lda.py:78-87``)
 _PZ81 = {"gamma": (-0.1423, -0.0843), "beta1": (1.0529, 1.3981), "beta2": (0.3334, 0.2611),
          "a": (0.0311, 0.01555), "b": (-0.048, -0.0269), "c": (0.0020, 0.0007), "d": (-0.0116, -0.0048)}
@@ -117,63 +115,8 @@ def _lda(up, dn, pz81: bool = False):
 
 def _gga(up, dn, suu, sud, sdd, par):
     """(eps, v_up, v_dn, vsigma_uu, vsigma_ud, vsigma_dd) of the PBE form."""
-    kappa, mu, beta, gamma = par["kappa"], par["mu"], par["beta"], par["gamma"]
-    n, rs, z = _rs_zeta(up, dn)
-    act = n > DENSITY_THRESHOLD
-    zero = torch.zeros_like(n)
-    # exchange, per spin channel
-    ex_e = zero
-    vx, vsx = [], []
-    for s, ss in ((up, suu), (dn, sdd)):
-        sp = torch.clamp(s, min=0.0)
-        safe = torch.clamp(sp, min=DENSITY_THRESHOLD)
-        n43 = safe ** (4 / 3)
-        s2 = (X2S * torch.sqrt(torch.clamp(ss, min=0.0)) / n43) ** 2
-        den = kappa + mu * s2
-        fx = 1.0 + kappa * mu * s2 / den
-        fxs = 2.0 * kappa * kappa * mu * s2 / den**2
-        keep = (sp > DENSITY_THRESHOLD) & act
-        ex_e = ex_e + torch.where(sp > DENSITY_THRESHOLD, -X_FACTOR_C * n43 * fx, zero)
-        vx.append(torch.where(keep, -(4 / 3) * X_FACTOR_C * _cbrt(safe) * (fx - fxs), zero))
-        vsx.append(torch.where(keep, -X_FACTOR_C * kappa * kappa * mu * X2S**2 / (n43 * den**2), zero))
-    ex = torch.where(act, ex_e / torch.where(act, n, torch.ones_like(n)), zero)
-    # correlation on modified PW92
-    safe = torch.clamp(n, min=DENSITY_THRESHOLD)
-    elda, dl_drs, dl_dz = _pw92_local(rs, z, _PW92_MOD)
-    opz, omz = torch.clamp(1.0 + z, min=DENSITY_THRESHOLD), torch.clamp(1.0 - z, min=DENSITY_THRESHOLD)
-    phi = 0.5 * (opz ** (2 / 3) + omz ** (2 / 3))
-    dphi = (1 / 3) * (opz ** (-1 / 3) - omz ** (-1 / 3))
-    phi3 = phi**3
-    stot = torch.clamp(suu + 2.0 * sud + sdd, min=0.0)
-    tpx = 1.0 / (4.0 * 2.0 ** (1 / 3) * phi * torch.sqrt(rs))
-    xt = torch.sqrt(stot) / safe ** (4 / 3)
-    t = tpx * xt
-    t2 = t * t
-    et = torch.expm1(-elda / (gamma * phi3))
-    es = torch.where(torch.abs(et) < 1e-300, torch.full_like(et, 1e-300), et)
-    A = beta / (gamma * es)
-    u = t2 + A * t2 * t2
-    d = 1.0 + A * u
-    w = beta * u / (gamma * d)
-    lg = torch.log1p(w)
-    H = gamma * phi3 * lg
-    pre = gamma * phi3 / (1.0 + w)
-    dh_dt = pre * beta / (gamma * d**2) * (2.0 * t + 4.0 * A * t2 * t)
-    dh_da = pre * beta * (t2 * t2 - u * u) / (gamma * d**2)
-    da_de = beta * (et + 1.0) / (gamma**2 * phi3 * es**2)
-    da_dphi = -3.0 * beta * elda * (et + 1.0) / (gamma**2 * phi**4 * es**2)
-    dh_drs = dh_da * da_de * dl_drs + dh_dt * (-t / (2.0 * rs))
-    dh_dz = 3.0 * gamma * phi * phi * lg * dphi + dh_da * (da_dphi * dphi + da_de * dl_dz) + dh_dt * (-t / phi) * dphi
-    ec = elda + H
-    de_drs = dl_drs + dh_drs
-    de_dz = dl_dz + dh_dz
-    common = ec - (rs / 3.0) * de_drs - (4 / 3) * xt * dh_dt * tpx
-    vcu = torch.where(act, common + (1.0 - z) * de_dz, zero)
-    vcd = torch.where(act, common - (1.0 + z) * de_dz, zero)
-    vst = torch.where(act, safe * phi3 * beta * (tpx**2 / safe ** (8 / 3)) * (2.0 + 4.0 * A * t2)
-                      / (2.0 * (1.0 + w) * d**2), zero)
-    ec = torch.where(act, ec, zero)
-    return ex + ec, vx[0] + vcu, vx[1] + vcd, vsx[0] + vst, 2.0 * vst, vsx[1] + vst
+    f64 = [f.to(torch.float64) for f in (up, dn, suu, sud, sdd)]
+    return ops.gga(*f64, (par["kappa"], par["mu"], par["beta"], par["gamma"])).unbind(0)
 
 
 class GridOps:

@@ -292,6 +292,14 @@ int amt_mlp_loss_grad(const float* feats, const float* target, long long npts, d
 int amt_adam(float* theta, const float* grad, float* m, float* v, int n, float lr, float beta1, float beta2,
              float eps, int step, void* stream);
 
+/*
+ * PBE-form exchange-correlation at n points (xc/gga.py:112-254), all float64 on the device: up, dn
+ * spin densities, suu, sud, sdd gradient products; parameters (host) kappa, mu, beta, gamma; out
+ * [6][n]: energy per particle, potentials up and down, derivatives by suu, sud and sdd.
+ */
+int amt_gga(long long n, const double* up, const double* dn, const double* suu, const double* sud, const double* sdd,
+            const double* parameters, double* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -49,3 +49,36 @@ def test_hartree_matches_the_oracle(si2_system):
     e, v = GridSide(si2_system).hartree(torch.from_numpy(rho).cuda())
     assert e == pytest.approx(e_ref, rel=1e-12)
     assert np.abs(v.cpu().numpy() - v_ref).max() < 1e-12 * np.abs(v_ref).max()
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 4099])
+@pytest.mark.parametrize("name", ["PBE", "PBEsol"])
+def test_gga_points_match_the_oracle(name, n):
+    """The pointwise kernel against the oracle at single points: both are chains of some hundred
+    FP64 operations, so ordinary densities agree to 1e-11 of each value plus 1e-11 of the exchange
+    scale; points at the edges (empty spin, below the threshold, zero gradient, negative) to 1e-7, as
+    the derivative by the polarisation is of size 1e8 there."""
+    import torch
+
+    from amaterasu_amd import ops
+    from amaterasu_amd.xc import _GGA
+    from oracle.xc import XCFunctional as OXC
+
+    rng = np.random.default_rng(n)
+    tot = 10.0 ** rng.uniform(-5, 1, n)
+    z = rng.uniform(-0.95, 0.95, n)
+    rho = np.stack([0.5 * tot * (1 + z), 0.5 * tot * (1 - z)], -1)
+    s = rng.uniform(0.0, 3.0, (n, 2)) * rho ** (4 / 3) * 6
+    sig = np.stack([s[:, 0] ** 2, rng.uniform(-1, 1, n) * s[:, 0] * s[:, 1], s[:, 1] ** 2], -1)
+    edge = np.array([[0.3, 0.0], [0.0, 0.2], [0.0, 0.0], [1e-25, 1e-26], [-1e-3, 0.1], [0.1, 0.1], [-0.1, -0.2]])
+    edge_sig = np.array([[0.1, 0.0, 0.0], [0.0, 0.0, 0.2], [0, 0, 0], [0, 0, 0], [0, 0, 0.1], [0, 0, 0], [0, 0, 0]])
+    par = [_GGA[name.upper()][k] for k in ("kappa", "mu", "beta", "gamma")]
+    for r, g, tol in ((rho, sig, 1e-11), (edge, edge_sig, 1e-7)):
+        with np.errstate(all="ignore"):
+            eps, v, vs = OXC(name).evaluate(r, g)
+        want = np.stack([eps, v[:, 0], v[:, 1], vs[:, 0], vs[:, 1], vs[:, 2]])
+        dev = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (r[:, 0], r[:, 1], g[:, 0], g[:, 1], g[:, 2])]
+        got = ops.gga(*dev, par).cpu().numpy()
+        scale = np.abs(want)
+        scale[:3] += np.maximum(r.sum(1), 0.0) ** (1 / 3)
+        assert (np.abs(got - want) <= tol * scale).all()
