@@ -3,8 +3,8 @@
 //
 // What bounds it: about 40 roots, powers and logarithms a point (FP64 vector work), against 11
 // numbers read and written. As some 190 elementwise operations the same formulas were bound by the
-// host issuing them (2 ms an evaluation) and by two passes over memory each: with this kernel a
-// 12-evaluation SCF run of 8 atoms takes 119 ms for 136, of 64 atoms 426 for 434.
+// host issuing them (2 ms an evaluation) and by two passes over memory each: with this kernel
+// six SCF steps of 8 atoms (12 evaluations) take 119 ms for 136, two of 64 atoms 426 for 434.
 #include "kernels.hpp"
 
 namespace amt {
