@@ -129,7 +129,7 @@ def _time_stage(plan, prec, stage, psi, out, v, st, k0, reps=REPEATS) -> float:
 
 def tune_fft_launch(plan, prec: int, psi: torch.Tensor, v: torch.Tensor, k0: int = 0) -> tuple:
     """Pick the plane kernel's workgroup (256 or 512 threads) and the stick kernels' width (the
-    default or half) for this grid length and precision by timing each candidate on the
+    wider or the narrower) for this grid length and precision by timing each candidate on the
     caller's block (read only; sticks and output go to scratch), with HIP events on the current
     stream, and set them on the plan (``amt_plan_set_launch``). The choice is remembered per
     (length, precision) and applied to later plans of that length without timing again. The
