@@ -67,6 +67,12 @@ def workspace(nbytes: int, tag: str = "ws") -> torch.Tensor:
     return buf
 
 
+def _scratch(nbytes: int) -> torch.Tensor:
+    """A buffer of one call, from the current stream's pool: safe from several threads and streams
+    (the allocation costs the host about 2 us)."""
+    return torch.empty(int(nbytes), dtype=torch.uint8, device="cuda")
+
+
 def zgemm(a: torch.Tensor, b: torch.Tensor, op: int, *, alpha: float = 1.0, beta: float = 0.0,
           out: torch.Tensor | None = None) -> torch.Tensor:
     """``alpha * a @ op(b) + beta * out`` on the matrix cores.
@@ -278,7 +284,7 @@ def chol_inverse(gram: torch.Tensor, used: torch.Tensor | None = None):
     linv = torch.empty_like(gram)
     stats = torch.empty((*gram.shape[:-2], (n + 31) // 32 + 2), dtype=torch.float64, device=gram.device)
     nbytes = int(lib().amt_chol_workspace(n, batch))
-    ws = workspace(nbytes, "chol")
+    ws = _scratch(nbytes)
     check(lib().amt_chol_inverse(precision_of(gram), n, gram.data_ptr(), None if used is None else used.data_ptr(),
                                  batch, linv.data_ptr(), stats.data_ptr(), ws.data_ptr(), nbytes, stream_handle()),
           "chol_inverse")
@@ -331,7 +337,7 @@ def heev_lowest_batched(a: torch.Tensor, sizes, nev: int):
     w = torch.empty((nk, nev), dtype=torch.float64, device=a.device)
     zt = torch.empty((nk, nev, n), dtype=torch.complex128, device=a.device)
     nbytes = int(lib().amt_heev_batched_workspace(max(sizes), nk))
-    ws = workspace(nbytes, "heev_batched")
+    ws = _scratch(nbytes)
     check(lib().amt_heev_lowest_batched(nk, (ctypes.c_int * nk)(*sizes), a.data_ptr(), a.stride(1), a.stride(0), nev,
                                         w.data_ptr(), zt.data_ptr(), n, ws.data_ptr(), nbytes, stream_handle()),
           "heev_batched")
@@ -347,7 +353,7 @@ def finish_density(rho: torch.Tensor, volume: float = 1.0) -> torch.Tensor:
         raise AmtError("finish_density: rho must be float64 [nspin][...]")
     nspin = rho.shape[0]
     if rho.numel():
-        part = workspace(lib().amt_density_finish_bytes(nspin), "density_finish")
+        part = _scratch(lib().amt_density_finish_bytes(nspin))
         check(lib().amt_density_finish(rho.data_ptr(), nspin, rho.numel() // nspin, float(volume), part.data_ptr(),
                                        stream_handle()), "density_finish")
     return rho
