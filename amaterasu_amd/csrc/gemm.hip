@@ -33,9 +33,9 @@
 // (4 p + g) * (16 / sizeof(C)) + s; any order of K is the same sum as long as A and B agree. B of
 // an NN product stays [k][column], read 8 (16) bytes at a time from rows of 72 (64) elements.
 //
-// FP32 accumulation over a long K is two-level: the MFMA's FP32 accumulators cover flush_k() of K
-// and are then added into FP64 registers, so the rounding error of a long contraction (subspace
-// overlaps over ~10^5 plane waves) grows with that length, not with K. One FP32 accumulator over
+// FP32 accumulation over a long K is two-level: the MFMA's FP32 accumulators cover 64 to 256 of K
+// (fp32_sums()) and are then added into FP64 registers, so the rounding error of a long contraction
+// (subspace overlaps over ~10^5 plane waves) grows with that length, not with K. One FP32 accumulator over
 // all of K = 81k left relative errors of ~6e-5 in the Gram matrices of a 440-band Davidson,
 // enough to stall an SCF. The additions cost 2 to 5 % of a product; split partials are summed in
 // FP64 too.
@@ -80,11 +80,6 @@ struct Mfma<double> {
 
 constexpr int BN = 64;            // columns of a tile
 constexpr int kChunks = 8;        // 16-byte chunks of one operand row and K tile
-// K between the two-level form's additions into FP64: 64 for NN products, 256 for NC ones
-template <int OP>
-constexpr int flush_k() {
-  return OP == 0 ? 64 : 256;
-}
 
 template <typename R>
 struct Vec16;  // 16 bytes of a row: two complex64 or one complex128
@@ -105,7 +100,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(int M, int N, int K, int kchun
                                                long long sA, const typename Cplx<R>::T* __restrict__ B,
                                                long long ldb, long long sB, typename Cplx<R>::T* __restrict__ Cm,
                                                long long ldc, long long sC, R alpha, R beta,
-                                               typename Cplx<R>::T* __restrict__ part, int mfast) {
+                                               typename Cplx<R>::T* __restrict__ part, int mfast, int flush_tiles) {
   using C = typename Cplx<R>::T;
   using acc_t = typename Mfma<R>::acc_t;
   using V = typename Vec16<R>::T;
@@ -312,7 +307,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(int M, int N, int K, int kchun
   // tile goes to the other buffer and its successor's loads are issued; the barrier that makes it
   // visible and the read of its first fragments lie between the two halves of the MFMAs.
   Frag f0, f1;
-  int buf = 0, tile = 0;
+  int buf = 0, tile = 0, until_flush = flush_tiles;
   auto step = [&](auto load, bool more) {
     fragments(f1, buf, 1);
     if (more) sstore(buf ^ 1);
@@ -324,7 +319,10 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(int M, int N, int K, int kchun
     products(f1);
     ++tile;
     if constexpr (kTwoLevel) {
-      if (tile % (flush_k<OP>() / BK) == 0) flush();
+      if (--until_flush == 0) {
+        flush();
+        until_flush = flush_tiles;
+      }
     }
   };
   if (nt > 0) {
@@ -418,10 +416,29 @@ static std::array<int, 6> split_key(int prec, int op, int m, int n, int k, int b
   return {prec, op, (m + 63) / 64, (n + 63) / 64, (k + 255) / 256, batch};
 }
 
-// Longest K that one FP32 accumulator covers. NC products (overlaps, projections: K the plane
-// waves) carry FP64 sums beyond 256 of K whatever their split; NN products (rotations, projector
-// applications) beyond 1024.
-constexpr int single_level_k(int op) { return op == 1 ? flush_k<1>() : 1024; }
+// Longest K that one FP32 accumulator covers without FP64 sums, and K between the additions into
+// FP64 beyond it. A product's rounding grows with the accumulator's length, so the length follows
+// from the shape and not from the split that happens to be fastest:
+//   NC (overlaps, projections: K the plane waves): 256; up to 4096 of K 128, as a few splits of at
+//     most 256 that divide such a K are shorter than that themselves; 64 for outputs of 512 tiles of
+//     64 x 64 and more, whose K is not split at all.
+//   NN (rotations, projector applications): 128 beyond 256 of K, 64 beyond 1024. Outputs of 512
+//     tiles of 80 x 64 and more keep one accumulator up to 1024: the rotations of a whole subspace,
+//     bound by the matrix cores (160 x 37 073 x 480: 154 us, with additions every 64 of K 168).
+// Measured with random operands: the projector applications 40 x 9300 x 288, 58 x 13 900 x 432 and
+// 80 x 18 500 x 576 are off by 2.8, 2.8 and 2.9e-7 in 15.2, 32.5 and 59.7 us, with one accumulator
+// over all of K by 4.4, 5.3 and 6.1e-7 in 14.7, 31.7 and 55.3, with additions every 64 of K by 2.1e-7
+// in 15.5, 33.4 and 61.0. NC products of K > 4096 with additions every 64: 2.1e-7 for 3.9e-7, 3 to 8 %
+// slower.
+struct Fp32Sums {
+  int limit, flush;
+};
+static Fp32Sums fp32_sums(int op, int m, int n, int k, int batch) {
+  auto tiles = [&](int rows) { return (long long)((m + rows - 1) / rows) * ((n + BN - 1) / BN) * batch; };
+  if (op == 0) return {k <= 256 || (k <= 1024 && tiles(80) >= 512) ? 1024 : 0, k <= 1024 ? 128 : 64};
+  const int flush = k > 1024 && tiles(64) >= 512 ? 64 : k > 4096 ? 256 : 128;
+  return {k <= 256 ? 256 : flush, flush};
+}
 constexpr int kMinChunk = 64;
 // FP32 NC products with both output sides at least this are left alone by the split tuning.
 constexpr int kBigSide = 256;
@@ -434,6 +451,7 @@ struct GemmPlan {
   int ns;       // K splits
   int kchunk;   // K per split, a multiple of the K tile
   bool two;     // FP64 second-level sums
+  int flush;    // K tiles between them
 };
 
 static bool split_is_tunable(int prec, int op, int m, int n, int k) {
@@ -449,14 +467,13 @@ static bool split_is_tunable(int prec, int op, int m, int n, int k) {
 // The first factor is what uneven rounds cost: 160 x 37 073 x 1152 (580
 // column tiles) in 32-row tiles fills its last round better than in 80-row ones. Against a sweep
 // of every W and split the choice is within 5 % on the Si8, Si64 and Si214 shapes.
-// Whether a product carries FP64 sums depends on its chunk (NC) or its K (NN) only
-// (single_level_k), so the split does not change its error: 3.7-4.1e-7 (relative norm, random
-// operands) on every NC shape above, where single accumulators over 256 to 1024 of K gave 4.1
-// to 7.9e-7.
+// No split lengthens an accumulator past fp32_sums(): 3.7-4.1e-7 (relative norm, random operands) on
+// every NC shape above, where single accumulators over 256 to 1024 of K gave 4.1 to 7.9e-7.
 static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
   const int csize = prec == kFP64 ? 16 : 8, bk = kChunks * 16 / csize;
   const double cols = (double)((n + BN - 1) / BN) * batch, out = (double)m * n * batch * csize;
-  GemmPlan best{1, 1, bk, false};
+  const Fp32Sums sums = fp32_sums(op, m, n, k, batch);
+  GemmPlan best{1, 1, bk, false, sums.flush / bk};
   double best_cost = 1e300;
   int lo = 1, hi = (k + kMinChunk - 1) / kMinChunk;
   hi = hi > 256 ? 256 : hi < 1 ? 1 : hi;
@@ -472,7 +489,7 @@ static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
     if (kchunk < bk) kchunk = bk;
     const int ns = k > 0 ? (k + kchunk - 1) / kchunk : 1;
     if (best_cost < 1e300 && (long long)batch * ns > 65535) break;
-    const bool two = prec == kFP32 && (op == 1 ? kchunk : k) > single_level_k(op);
+    const bool two = prec == kFP32 && (op == 1 ? kchunk : k) > sums.limit;
     const double tiles = kchunk / bk + 2, extra = ns > 1 ? 20.0 + 2.0 * out * ns / 1.3e6 : 0.0;
     for (int w = 1; w <= (prec == kFP64 || two ? kMaxWLong : kMaxW); ++w) {
       const double cost = (std::ceil(rows[w] * ns / 256.0) + 0.8) * tiles * (w + 0.35) * (two ? 1.1 : 1.0) + extra;
@@ -618,7 +635,7 @@ static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, lon
   C* const p = ns > 1 ? part : nullptr;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, m, n, k, kchunk, ns, (const C*)a, lda, sa, (const C*)b, ldb, sb,
-                       (C*)c, ldc, sc, (R)alpha, (R)beta, p, mfast);
+                       (C*)c, ldc, sc, (R)alpha, (R)beta, p, mfast, g.flush);
   };
 #define AMT_W(TWO, W)                \
   case W:                            \

@@ -173,3 +173,31 @@ def test_zgemm_tile_edges(dtype, m):
             bad[-1] = float("nan")
             got = ops.zgemm(bad[:, 1 : 1 + k], db, op)
             assert bool(torch.isfinite(torch.view_as_real(got[:-1])).all()) and bool(got[-1].isnan().all())
+
+
+@pytest.mark.parametrize("op,m,n,k,batch", [(0, 80, 18500, 576, 1), (0, 58, 13900, 432, 1), (0, 40, 9301, 288, 1),
+                                            (0, 17, 1830, 399, 5), (0, 5, 700, 1024, 1), (0, 9, 3000, 1500, 1),
+                                            (1, 19, 1381, 355, 5), (1, 264, 19, 391, 3), (1, 300, 270, 461, 1),
+                                            (1, 28, 3011, 6522, 11), (1, 64, 33000, 1100, 1), (1, 160, 480, 9000, 1)])
+def test_zgemm_fp32_accumulator_length(op, m, n, k, batch):
+    """K that one FP32 accumulator may cover: the equal parts of at most 256 that K divides into (to
+    the next K tile of 16), 64 where an NC product has 512 tiles of 64 x 64 outputs and more than
+    1024 of K. Integers whose sums are exact in FP32 up to that length and not beyond, so only two
+    roundings are left: of each partial product and of the result, at most u times the (positive)
+    sum each; an accumulator of twice the length loses several units in the last place."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    parts = (k + 255) // 256
+    length = (-(-k // parts) + 15) // 16 * 16
+    if op == 1 and k > 1024 and -(-m // 64) * -(-n // 64) * batch >= 512:
+        length = 64
+    top = 2**24 // length
+    g = torch.Generator(device="cuda").manual_seed(k)
+    b = torch.randint(top - top // 20, top + 1, (batch, k, n) if op == 0 else (batch, n, k), device="cuda", generator=g)
+    want = b.sum(1 if op == 0 else 2)[:, None, :].to(torch.float64)
+    a = torch.ones((batch, m, k), dtype=torch.complex64, device="cuda")
+    got = ops.zgemm(a, b.to(torch.complex64), op)
+    assert not got.imag.any()
+    assert bool(((got.real.to(torch.float64) - want).abs() <= 2 * 2.0**-24 * want).all())
