@@ -255,6 +255,7 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
     proj = torch.zeros((nk, cap, cap), dtype=torch.complex128, device=dev)
     proj[:, :nb, :nb] = _projected(basis[:, :nb], hbasis[:, :nb])
     eps, vec, hvec = _rayleigh_ritz(proj[:, :nb, :nb], basis[:, :nb], hbasis[:, :nb], [nb] * nk, nb)
+    solved = m.copy()  # rows of the projected matrices that eps belongs to
     # frozen outputs of the k-points that have returned
     out_eps, out_vec = eps, vec
     out_norm = torch.full((nk, nb), float("inf"), dtype=torch.float64, device=dev)
@@ -269,9 +270,9 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
             out_norm = norms
         else:
             out_norm[torch.as_tensor(running, device=dev)] = norms[torch.as_tensor(running, device=dev)]
-        flags = torch.stack([norms > tolerance, torch.isnan(norms)]).cpu().numpy()  # one device read
+        flags = torch.stack([norms > tolerance, torch.isnan(eps)]).cpu().numpy()  # one device read
         active = flags[0] & running[:, None]
-        if (flags[1].any(axis=1) & running & (m < NAN_SILENT)).any():
+        if (flags[1].any(axis=1) & running & (solved < NAN_SILENT)).any():
             raise_not_finite()
         finished = running & ~active.any(axis=1)
         running &= ~finished
@@ -311,6 +312,7 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
         cols = _bgram(basis[:, :cur], hnew)  # conj of <b_r|H|new_j>, rows of new past kept are zero
         ops.append_projected(cols, proj, grown)
         m = m + kept
+        solved = np.where(running, m, solved)
         eps_n, vec_n, hvec_n = _rayleigh_ritz(proj[:, :cur, :cur], basis[:, :cur], hbasis[:, :cur], m, nb)
         if running.all():
             eps, vec, hvec = eps_n, vec_n, hvec_n
@@ -331,7 +333,9 @@ def solve_batched(apply_block, guess: torch.Tensor, kinetic: torch.Tensor, npw, 
             proj[k].zero_()
             proj[k, :nb, :nb] = _projected(basis[k : k + 1, :nb], hbasis[k : k + 1, :nb])[0]
             m[k] = nb
-    conv = (out_norm <= tolerance).all(dim=1).cpu().numpy()
+    conv, failed = torch.stack([(out_norm <= tolerance).all(dim=1), torch.isnan(out_eps).any(dim=1)]).cpu().numpy()
+    if (failed & (solved < NAN_SILENT)).any():
+        raise_not_finite()
     return BatchedResult(out_eps, out_vec, out_norm, iters, conv)
 
 

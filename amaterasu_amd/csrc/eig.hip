@@ -1060,7 +1060,9 @@ __device__ __forceinline__ double wave_sum(double v) {
 // Eigenvalue k (0-based, ascending) of T for k < m, one workgroup per eigenvalue: each
 // step evaluates the Sturm count at 512 points of the bracket (two independent recurrences
 // per thread), so it narrows the bracket 513-fold. scal[0] = the Gershgorin bound of ||T||,
-// scal[1] = pivmin (written by eigenvalue 0's workgroup).
+// scal[1] = pivmin (written by eigenvalue 0's workgroup). A T that is not finite (the reduction
+// carries every entry of A that is not into d or e) has eigenvalues NaN, all of them: the minima and
+// Sturm counts below pass over a NaN, and would give numbers.
 __device__ __forceinline__ double recip(double q) {
   // v_rcp_f64 refined by two Newton steps: a correctly signed reciprocal to about 1 ulp,
   // a third of the latency of the IEEE division sequence on the recurrence's critical path
@@ -1081,9 +1083,11 @@ __global__ __launch_bounds__(eig::NT) void k_tri_bisect(const double* __restrict
   const int k = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (k >= m) return;
   double lo = DBL_MAX, hi = -DBL_MAX, emax2 = 0.0;
+  bool finite = true;
   for (int i = tid; i < n; i += eig::NT) {
     const double di = d[i];
     const double ea = i > 0 ? fabs(e[i - 1]) : 0.0, eb = i + 1 < n ? fabs(e[i]) : 0.0;
+    finite = finite && fabs(di) <= DBL_MAX && eb <= DBL_MAX;
     dl[i] = di;
     e2[i] = eb * eb;
     emax2 = fmax(emax2, eb * eb);
@@ -1100,7 +1104,14 @@ __global__ __launch_bounds__(eig::NT) void k_tri_bisect(const double* __restrict
     red[3 * wave + 1] = hi;
     red[3 * wave + 2] = emax2;
   }
-  __syncthreads();
+  if (__syncthreads_or(!finite)) {
+    if (tid == 0) wb[k] = __longlong_as_double(0x7ff8000000000000ll);
+    if (k == 0 && tid == 0) {
+      scal[0] = 0.0;
+      scal[1] = DBL_MIN;
+    }
+    return;
+  }
   for (int w = 0; w < eig::NT / 64; ++w) {
     lo = fmin(lo, red[3 * w]);
     hi = fmax(hi, red[3 * w + 1]);

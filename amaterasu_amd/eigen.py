@@ -457,7 +457,7 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
     h_basis[:nbands] = op(v0)
     if sg is not None and op.host:
         raise AmtError("davidson: graph replay needs an operator that takes device blocks")
-    m = nbands
+    m = solved = nbands  # solved: rows of the projected matrix that eps belongs to
     proj[:m, :m] = _hermitian(_gram(basis[:m], h_basis[:m]).conj())
     eps, vec, hvec = _ritz(proj[:m, :m], basis[:m], h_basis[:m], nbands)
     res, next_norms = ops.residual(hvec, vec, eps)
@@ -467,10 +467,8 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
         iteration = step
         # the residuals of this pass's Ritz pairs (a graph's replay overwrites its outputs)
         norms = next_norms if sg is None else next_norms.clone()
-        active = torch.nonzero(norms > tolerance).flatten()
+        active = torch.nonzero(norms > tolerance).flatten()  # none for NaN eigenvalues: reported below
         if active.numel() == 0:
-            if m < NAN_SILENT and bool(torch.isnan(norms).any()):
-                raise_not_finite()
             break
         corr = ops.precondition(res, vec, kin, active, rows_checked=True)  # rows of nonzero(norms)
         new = orthogonalize_against(corr, basis[:m], overwrite=True)
@@ -485,6 +483,7 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
         else:
             eps, vec, hvec, res, next_norms = body()
         m += nn
+        solved = m
         if m + nbands > max_subspace:
             basis[:nbands] = vec
             h_basis[:nbands] = hvec
@@ -492,7 +491,9 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
             proj[:m, :m] = _hermitian(_gram(basis[:m], h_basis[:m]).conj())
     if sg is not None:  # graph outputs are overwritten by the next replay
         eps, vec = eps.clone(), vec.clone()
-    converged = bool((norms <= tolerance).all().item())
+    converged, failed = torch.stack([(norms <= tolerance).all(), torch.isnan(eps).any()]).tolist()
+    if failed and solved < NAN_SILENT:
+        raise_not_finite()
     if host:
         return DavidsonResult(eps.cpu().numpy(), vec.to(torch.complex128).cpu().numpy(), norms.cpu().numpy(),
                               iteration, converged)
@@ -506,8 +507,9 @@ def davidson(apply_hamiltonian, guess, kinetic, *, tolerance: float = 1e-8, max_
 HEEV_MIN = 2
 HEEV_MAX = 2048
 
-#: zheevd reports a matrix that is not finite, the library's solver returns NaN: below this size,
-#: where zheevd used to be the solver, the iteration raises its error when it finds NaN residuals.
+#: zheevd reports a matrix that is not finite, the library's solver returns NaN eigenvalues. Below
+#: this size the iterations raise zheevd's error for them; they read the flag with the residual norms
+#: of the same Ritz pairs, or with the last ones, so that it costs no host read of its own.
 NAN_SILENT = 96
 
 

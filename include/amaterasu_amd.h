@@ -232,7 +232,8 @@ int amt_kb_dij(int precision, const void* proj, const void* dij, const int* blk_
  * Householder tridiagonalisation on the device (one launch per column); the lowest
  * eigenpairs of the tridiagonal by multisection bisection and inverse iteration, with a
  * Rayleigh-Ritz step inside clusters of close eigenvalues; back-transformation on the
- * device. a is not modified; ws must hold amt_heev_workspace(n) bytes.
+ * device. a is not modified; ws must hold amt_heev_workspace(n) bytes. A matrix with an entry that is
+ * not finite gives NaN in every eigenvalue.
  */
 size_t amt_heev_workspace(int n);
 int amt_heev_lowest(int n, const void* a, int nev, double* w, void* zt, void* ws, size_t ws_bytes, void* stream);

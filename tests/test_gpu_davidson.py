@@ -246,3 +246,47 @@ def test_inverse_cholesky_factor(dtype, n):
     assert float(emax.max()) == max(np.abs(e.real).max(), np.abs(e.imag).max())
     v[n // 2, 0] = float("nan")
     assert np.isnan(float(ops.lowdin(v.cuda())[1].cpu().max()))
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("last", [1, 2, 6])
+def test_operator_that_stops_being_finite(bad, last):
+    """One entry of H x that is not finite, in application ``last`` + 1 of ``last`` allowed iterations:
+    the per-k and the k-batched iteration raise, also where no iteration is left to see it, and also
+    when only one k-point is concerned; before, both return."""
+    import torch
+
+    from amaterasu_amd.batched import solve_batched
+    from amaterasu_amd.eigen import davidson
+
+    n, nb, nk = 200, 4, 2
+    g = torch.Generator(device="cuda").manual_seed(last)
+    kin = torch.linspace(0.1, 30.0, n, dtype=torch.float64, device="cuda").repeat(nk, 1)
+    a = 0.2 * torch.randn((n, n), dtype=torch.complex128, device="cuda", generator=g)
+    a = (a + a.mH) / 2 + torch.diag(kin[0].to(torch.complex128))
+    guess = torch.randn((nk, nb, n), dtype=torch.complex128, device="cuda", generator=g) / (1 + kin[:, None, :])
+
+    def operator(at):
+        calls = []
+
+        def apply(x):
+            calls.append(1)
+            out = x @ a.T.contiguous()
+            if len(calls) == at:
+                out[..., -1, 3] = bad
+                if out.dim() == 3:
+                    out[0] = x[0] @ a.T.contiguous()
+            return out
+
+        return apply
+
+    for at, raises in ((last + 2, False), (last + 1, True), (1, True)):
+        if raises:
+            with pytest.raises(torch.linalg.LinAlgError):
+                davidson(operator(at), guess[0], kin[0], tolerance=1e-10, max_iterations=last)
+            with pytest.raises(torch.linalg.LinAlgError):
+                solve_batched(operator(at), guess, kin, [n] * nk, tolerance=1e-10, max_iterations=last)
+        else:
+            one = davidson(operator(at), guess[0], kin[0], tolerance=1e-10, max_iterations=last)
+            both = solve_batched(operator(at), guess, kin, [n] * nk, tolerance=1e-10, max_iterations=last)
+            assert bool(torch.isfinite(one.eigenvalues).all()) and bool(torch.isfinite(both.eigenvalues).all())

@@ -131,3 +131,24 @@ def test_heev_chain_longer_than_a_cluster(spacing):
     assert np.abs(w - ref).max() < 1e-13 * 3
     assert np.abs(a @ z - z * w).max() < 1e-12 * 3
     assert np.abs(z.conj().T @ z - np.eye(nev)).max() < 1e-12 * 3
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("n", [2, 3, 20, 65, 66, 95, 130])
+def test_heev_of_a_matrix_that_is_not_finite(n, bad):
+    """One entry that is not finite, on the diagonal or off it, in a dense matrix and in a diagonal one
+    (whose reflectors are all H = I), gives NaN in every eigenvalue; the other matrices of a batch
+    keep their own values."""
+    from amaterasu_amd import ops
+
+    nev = max(n // 3, 1)
+    good = torch.from_numpy(_hermitian(n, n)).cuda()
+    alone = ops.heev_lowest(good, nev)[0]
+    for base in (good, torch.diag(torch.arange(n, device="cuda")).to(torch.complex128)):
+        for r, c in ((0, 0), (n - 1, n - 1), (n // 2, 0), (n - 1, n - 2)):
+            a = base.clone()
+            a[r, c] = bad
+            a[c, r] = bad
+            assert bool(ops.heev_lowest(a, nev)[0].isnan().all()), (r, c)
+            w, _ = ops.heev_lowest_batched(torch.stack([good, a, good]), [n] * 3, nev)
+            assert torch.equal(w[0], alone) and torch.equal(w[2], alone) and bool(w[1].isnan().all())
