@@ -518,10 +518,12 @@ def raise_not_finite():
 
 
 def _lowest_eigenpairs(proj: torch.Tensor, nbands: int, workspace_tag: str = "heev"):
-    """(w[:nbands], rows of eigenvectors) of a Hermitian FP64 matrix."""
+    """(w[:nbands], rows of eigenvectors) of a Hermitian FP64 matrix. Solves on several threads or
+    streams do not share scratch below 96 rows (0.7 MB a call); above, ``workspace_tag`` names a
+    cached buffer (up to 0.3 GB), one per concurrent caller."""
     m = proj.shape[0]
     if HEEV_MIN <= m <= HEEV_MAX:
-        return ops.heev_lowest(proj.contiguous(), nbands, workspace_tag=workspace_tag)
+        return ops.heev_lowest(proj.contiguous(), nbands, workspace_tag=None if m < 96 else workspace_tag)
     w, vec = torch.linalg.eigh(proj)
     return w[:nbands], vec[:, :nbands].T.contiguous()
 

@@ -304,10 +304,11 @@ def lowdin(gram: torch.Tensor):
     return rot, emax
 
 
-def heev_lowest(a: torch.Tensor, nev: int, *, workspace_tag: str = "heev"):
+def heev_lowest(a: torch.Tensor, nev: int, *, workspace_tag: str | None = "heev"):
     """Lowest ``nev`` eigenpairs of a Hermitian complex128 matrix on the device: (w, zt) with
     w ascending (float64) and zt[k] the k-th eigenvector (row). See amt_heev_lowest. Calls
-    that may run at the same time (on different streams) need different ``workspace_tag``s."""
+    that may run at the same time (on different streams) need different ``workspace_tag``s; ``None``
+    takes scratch of this call."""
     _require(a, "a")
     if a.dtype != torch.complex128 or a.dim() != 2 or a.shape[0] != a.shape[1]:
         raise AmtError("heev: a must be a square complex128 device matrix")
@@ -317,7 +318,7 @@ def heev_lowest(a: torch.Tensor, nev: int, *, workspace_tag: str = "heev"):
     w = torch.empty(nev, dtype=torch.float64, device=a.device)
     zt = torch.empty((nev, n), dtype=torch.complex128, device=a.device)
     nbytes = int(lib().amt_heev_workspace(n))
-    ws = workspace(nbytes, workspace_tag)
+    ws = _scratch(nbytes) if workspace_tag is None else workspace(nbytes, workspace_tag)
     check(lib().amt_heev_lowest(n, a.data_ptr(), nev, w.data_ptr(), zt.data_ptr(), ws.data_ptr(), nbytes,
                                 stream_handle()), "heev")
     return w, zt

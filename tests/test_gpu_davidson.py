@@ -290,3 +290,41 @@ def test_operator_that_stops_being_finite(bad, last):
             one = davidson(operator(at), guess[0], kin[0], tolerance=1e-10, max_iterations=last)
             both = solve_batched(operator(at), guess, kin, [n] * nk, tolerance=1e-10, max_iterations=last)
             assert bool(torch.isfinite(one.eigenvalues).all()) and bool(torch.isfinite(both.eigenvalues).all())
+
+
+def test_small_eigensolves_share_no_scratch(monkeypatch):
+    """Projected matrices of 2 to 95 rows: no cached workspace is used, and solves on two threads,
+    each on its own stream, give the bits of solves alone."""
+    import threading
+
+    import torch
+
+    from amaterasu_amd import eigen, ops
+
+    g = torch.Generator(device="cuda").manual_seed(0)
+    mats = [torch.randn((n, n), dtype=torch.complex128, device="cuda", generator=g) for n in (2, 20, 80, 95)]
+    mats = [a + a.mH for a in mats]
+    alone = [eigen._lowest_eigenpairs(a, max(len(a) // 4, 1)) for a in mats]
+    torch.cuda.synchronize()
+
+    def refuse(*args):
+        raise AssertionError("a cached workspace was asked for")
+
+    monkeypatch.setattr(ops, "workspace", refuse)
+    different, finished = [], []
+
+    def work(order):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                got = [(i, eigen._lowest_eigenpairs(mats[i], max(len(mats[i]) // 4, 1))) for i in order]
+                torch.cuda.current_stream().synchronize()
+                different.extend(i for i, (w, z) in got
+                                 if not (torch.equal(w, alone[i][0]) and torch.equal(z, alone[i][1])))
+        finished.append(order)
+
+    threads = [threading.Thread(target=work, args=(order,)) for order in ((0, 1, 2, 3), (3, 2, 1, 0))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(finished) == 2 and not different
