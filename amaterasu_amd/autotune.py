@@ -94,7 +94,8 @@ def tune_zgemm(run, prec: int, op: int, m: int, n: int, k: int, batch: int) -> i
 
 
 # ----------------------------------------------------------------------- FFT launch shapes
-#: (length of a cubic grid or shape, precision) -> (plane workgroup, sticks per workgroup) chosen so far
+#: (length of a cubic grid or shape, precision, one-lane plane kernel) -> (plane workgroup, sticks per
+#: workgroup) chosen so far; the one-lane kernel has no choice of workgroup: 0
 _FFT: dict = {}
 
 
@@ -132,14 +133,19 @@ def tune_fft_launch(plan, prec: int, psi: torch.Tensor, v: torch.Tensor, k0: int
     wider or the narrower) for this grid length and precision by timing each candidate on the
     caller's block (read only; sticks and output go to scratch), with HIP events on the current
     stream, and set them on the plan (``amt_plan_set_launch``). The choice is remembered per
-    (length, precision) and applied to later plans of that length without timing again. The
+    (length, precision) and applied to later plans of that length without timing again. Plans whose
+    spheres are narrow enough for the one-lane plane kernel, which has a workgroup of its own, have
+    an entry of their own without one, so that a wide plan of the same length is timed. The
     result of H.psi does not depend on it (every stick and plane is transformed by the same
     arithmetic whatever the grouping)."""
     n1, n2, n3 = plan.shape
-    key = (n1 if n1 == n2 == n3 else plan.shape, prec)
     info = plan.info
+    one_lane = bool(info[16 + prec])
+    key = (n1 if n1 == n2 == n3 else plan.shape, prec, one_lane)
     if key not in _FFT:
-        info[12 + prec] = info[14 + prec] = -1  # the timing below leaves the plan on its last candidate
+        info[14 + prec] = -1  # the timing below leaves the plan on its last candidates
+        if not one_lane:
+            info[12 + prec] = -1
         nkk, nb, _ = psi.shape
         wdef = 32 if prec == 1 else 64
         st = torch.empty(lib().amt_plan_stick_bytes(plan.handle, prec, nkk * nb), dtype=torch.uint8,
@@ -150,18 +156,18 @@ def tune_fft_launch(plan, prec: int, psi: torch.Tensor, v: torch.Tensor, k0: int
             check(lib().amt_plan_set_launch(plan.handle, prec, 0, w), "plan_set_launch")
             times[("w", w)] = _time_stage(plan, prec, 1, psi, out, v, st, k0) + \
                 _time_stage(plan, prec, 3, psi, out, v, st, k0)
-        for nth in (256, 512):
+        for nth in () if one_lane else (256, 512):
             check(lib().amt_plan_set_launch(plan.handle, prec, nth, 0), "plan_set_launch")
             _time_stage(plan, prec, 1, psi, out, v, st, k0, reps=1)  # fresh sticks for the in-place plane pass
             times[("p", nth)] = _time_stage(plan, prec, 2, psi, out, v, st, k0)
         best_w = min((w for (kind, w) in times if kind == "w"), key=lambda w: times[("w", w)])
-        best_p = min((n for (kind, n) in times if kind == "p"), key=lambda n: times[("p", n)])
+        best_p = min((n for (kind, n) in times if kind == "p"), key=lambda n: times[("p", n)], default=0)
         _FFT[key] = (best_p, best_w)
         del st, out
     nth, w = _FFT[key]
-    if (info[12 + prec], info[14 + prec]) != (nth, w):
+    if (nth and info[12 + prec] != nth) or info[14 + prec] != w:
         check(lib().amt_plan_set_launch(plan.handle, prec, nth, w), "plan_set_launch")
-        info[12 + prec], info[14 + prec] = nth, w
+        info[12 + prec], info[14 + prec] = nth or info[12 + prec], w
     return nth, w
 
 

@@ -321,13 +321,15 @@ int amt_plan_info(const amt_plan_t* h, int* info, int len) {
     return 1;
   }
   const Plan& p = h->p;
-  const int v[16] = {p.n1,           p.n2,           p.n3,
+  auto lane = [&](int prec) { return p.fast && p.narrow && lane_plane_supported(p.dim(1), prec) ? 1 : 0; };
+  const int v[18] = {p.n1,           p.n2,           p.n3,
                      p.nk,           p.npw_pad,      p.smax,
                      p.stick_w[0],   p.stick_w[1],   p.stick_threads[0],
                      p.stick_threads[1], p.plane_threads[0], p.plane_threads[1],
                      p.fast ? p.plane_nth[0] : 0, p.fast ? p.plane_nth[1] : 0,
-                     p.fast ? p.fast_stick_w[0] : 0, p.fast ? p.fast_stick_w[1] : 0};
-  for (int i = 0; i < len && i < 16; ++i) info[i] = v[i];
+                     p.fast ? p.fast_stick_w[0] : 0, p.fast ? p.fast_stick_w[1] : 0,
+                     lane(kFP32), lane(kFP64)};
+  for (int i = 0; i < len && i < 18; ++i) info[i] = v[i];
   return 0;
 }
 

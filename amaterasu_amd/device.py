@@ -67,8 +67,8 @@ class DevicePlan:
                                     miller.ctypes.data_as(ctypes.POINTER(ctypes.c_int)),
                                     kin.ctypes.data_as(ctypes.POINTER(ctypes.c_double))), "plan_create")
         self._handle = handle
-        info = (ctypes.c_int * 16)()
-        check(lib().amt_plan_info(handle, info, 16), "plan_info")
+        info = (ctypes.c_int * 18)()
+        check(lib().amt_plan_info(handle, info, 18), "plan_info")
         self.info = list(info)
         self.smax = self.info[5]
         self.plane_ok = {FP32: self.info[10] > 0, FP64: self.info[11] > 0}
@@ -244,8 +244,8 @@ class DevicePlan:
         """Send this precision's local H.psi and density through the library's full-grid route
         (``full_grid=True``) even where the plane kernels fit, or back (amt_plan_set_route)."""
         check(lib().amt_plan_set_route(self._handle, prec, 1 if full_grid else 0), "plan_set_route")
-        info = (ctypes.c_int * 16)()
-        check(lib().amt_plan_info(self._handle, info, 16), "plan_info")
+        info = (ctypes.c_int * 18)()
+        check(lib().amt_plan_info(self._handle, info, 18), "plan_info")
         self.info = list(info)
         self.plane_ok = {FP32: self.info[10] > 0, FP64: self.info[11] > 0}
 

@@ -48,10 +48,12 @@ int amt_device_info(char* buf, int len);
 int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int* npw, int npw_pad,
                     const int* miller, const double* kinetic);
 int amt_plan_destroy(amt_plan_t* plan);
-/* info[0..15] = n1, n2, n3, nk, npw_pad, smax, stick_w{fp32,fp64}, stick_threads{fp32,fp64},
+/* info[0..17] = n1, n2, n3, nk, npw_pad, smax, stick_w{fp32,fp64}, stick_threads{fp32,fp64},
  * plane_threads{fp32,fp64} (0 = plane does not fit LDS at that precision: full-grid route),
  * and for grids with compile-time-length kernels (else 0) the launch shapes of
- * amt_plan_set_launch: plane workgroup{fp32,fp64}, sticks per workgroup{fp32,fp64}. */
+ * amt_plan_set_launch: plane workgroup{fp32,fp64}, sticks per workgroup{fp32,fp64}; then
+ * {fp32,fp64} 1 where the plane kernel with one to four lanes per row runs, which has a workgroup
+ * of its own. The first `len` of them are written. */
 int amt_plan_info(const amt_plan_t* plan, int* info, int len);
 /* Tuning hook, no counterpart in the reference: the launch shape of the compile-time-length
  * H.psi kernels at `precision` -- plane kernel workgroup of 256 or 512 threads, stick kernels

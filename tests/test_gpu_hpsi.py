@@ -413,3 +413,46 @@ def test_projector_contraction_and_padding(si2_system, blocks, dtype, split, rou
     # sums of length n err by at most about sqrt(n) u of the sum of absolute values here (random signs), 4 for the parts
     assert ((cpu(out) - want).abs() <= 4 * np.sqrt(npw + max(blocks) + np_) * u * size + 1e-300).all()
     assert not out[live.expand(nk, nb, npw) == 0].any() and out.isfinite().all()
+
+
+@pytest.mark.parametrize("n,prec,one_lane", [(24, 0, True), (24, 1, True), (42, 0, True), (108, 1, True), (63, 0, False),
+                                             (72, 0, False), (84, 1, False)])
+def test_launch_tuning_by_plane_kernel(monkeypatch, n, prec, one_lane):
+    """A narrow plan of a length with a one-lane plane kernel does not time plane workgroups, which
+    that kernel has none to choose from; a wide plan of the same length has an entry of its own and
+    is timed, whichever comes first."""
+    import torch
+
+    from amaterasu_amd import autotune
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    cell = np.eye(3) * n / 4.0
+    monkeypatch.setenv("AMT_AUTOTUNE_FFT", "1")
+    monkeypatch.setattr(autotune, "_FFT", {})
+    stages = []
+    timed = autotune._time_stage
+
+    def record(plan, p, stage, *args, **kwargs):
+        stages.append(stage)
+        return timed(plan, p, stage, *args, **kwargs)
+
+    monkeypatch.setattr(autotune, "_time_stage", record)
+    v = torch.randn((n, n, n), dtype=torch.float64, device="cuda")
+    for half, lanes in ((n / 4.0 - 0.4, one_lane), (n / 4.0 + 3.0, False)):
+        plan = DevicePlan((n, n, n), [GSphere.build(cell, 0.5 * (half * 2.0 * np.pi / (n / 4.0)) ** 2)])
+        assert bool(plan.info[16 + prec]) == lanes
+        if not plan.plane_ok[prec]:
+            continue  # a wide FP64 plane past LDS takes whole grids and has no launch shape
+        psi = torch.randn((1, 2, plan.npw_pad), dtype=torch.complex128 if prec else torch.complex64, device="cuda")
+        known = (n, prec, lanes) in autotune._FFT
+        stages.clear()
+        plan.hpsi(psi, v)
+        assert (1 in stages) == (not known) and (2 in stages) == (not known and not lanes)
+        stages.clear()
+        plan.hpsi(psi, v)
+        assert not stages and -1 not in (plan.info[12 + prec], plan.info[14 + prec])
+    lanes_seen = {key[2] for key in autotune._FFT}
+    assert lanes_seen == ({True, False} if one_lane and n <= 100 else {one_lane})
+    for key, (nth, width) in autotune._FFT.items():
+        assert (nth == 0) == key[2] and width in (16, 32, 64)
