@@ -135,7 +135,8 @@ def tune_fft_launch(plan, prec: int, psi: torch.Tensor, v: torch.Tensor, k0: int
     stream, and set them on the plan (``amt_plan_set_launch``). The choice is remembered per
     (length, precision) and applied to later plans of that length without timing again. Plans whose
     spheres are narrow enough for the one-lane plane kernel, which has a workgroup of its own, have
-    an entry of their own without one, so that a wide plan of the same length is timed. The
+    an entry of their own without one, so that a wide plan of the same length is timed. A call under
+    graph capture cannot time anything and leaves an unknown length as the plan has it. The
     result of H.psi does not depend on it (every stick and plane is transformed by the same
     arithmetic whatever the grouping)."""
     n1, n2, n3 = plan.shape
@@ -143,6 +144,8 @@ def tune_fft_launch(plan, prec: int, psi: torch.Tensor, v: torch.Tensor, k0: int
     one_lane = bool(info[16 + prec])
     key = (n1 if n1 == n2 == n3 else plan.shape, prec, one_lane)
     if key not in _FFT:
+        if torch.cuda.is_current_stream_capturing():
+            return info[12 + prec], info[14 + prec]
         info[14 + prec] = -1  # the timing below leaves the plan on its last candidates
         if not one_lane:
             info[12 + prec] = -1

@@ -456,3 +456,40 @@ def test_launch_tuning_by_plane_kernel(monkeypatch, n, prec, one_lane):
     assert lanes_seen == ({True, False} if one_lane and n <= 100 else {one_lane})
     for key, (nth, width) in autotune._FFT.items():
         assert (nth == 0) == key[2] and width in (16, 32, 64)
+
+
+@pytest.mark.parametrize("shape", [(24, 20, 20), (20, 20, 24), (24, 24, 24)])
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_first_call_of_a_length_under_capture(monkeypatch, shape, precision):
+    """H.psi captured into a graph before its launch shapes are known: nothing is timed (that would
+    wait for events inside the capture), and every replay, with eager calls and synchronisations in
+    between, gives the eager result."""
+    import torch
+
+    from amaterasu_amd import autotune
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    n = min(shape)
+    cell = np.diag(np.array(shape) / 4.0)
+    dt = torch.complex64 if precision == "fp32" else torch.complex128
+    plan = DevicePlan(shape, [GSphere.build(cell, 0.5 * ((n / 4.0 - 0.4) * 2.0 * np.pi / (n / 4.0)) ** 2)])
+    g = torch.Generator(device="cuda").manual_seed(n)
+    psi = torch.randn((1, 3, plan.npw_pad), dtype=dt, device="cuda", generator=g)
+    v = torch.randn(shape, dtype=torch.float64 if precision == "fp64" else torch.float32, device="cuda", generator=g)
+    monkeypatch.setattr(autotune, "_FFT", {})
+    monkeypatch.setenv("AMT_AUTOTUNE_FFT", "0")
+    out = torch.empty_like(psi)
+    want = plan.hpsi(psi, v, out=out).clone()  # sizes the workspace
+    monkeypatch.setenv("AMT_AUTOTUNE_FFT", "1")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.hpsi(psi, v, out=out)
+    assert not autotune._FFT
+    for _ in range(4):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(plan.hpsi(psi, v), want)
+    assert len(autotune._FFT) == 1
