@@ -364,24 +364,24 @@ int amt_plan_nsticks(const amt_plan_t* h, int* out) {
   return 0;
 }
 
-// Bytes of the local H.psi / density workspace for `rows` band rows: their sticks (and V_eff in
-// the plan's axes), or, where the plane does not fit LDS (full-grid route), whole grids for
-// min(rows, ~1 GiB of grids).
-static size_t local_ws_bytes(const Plan& p, int prec, long long rows) {
+// Bytes of the local H.psi workspace for `rows` band rows: their sticks (and V_eff in the plan's
+// axes), or, on the full-grid route, whole grids for min(rows, ~1 GiB of grids). `density`: enough
+// for the density as well, which takes whole grids where only H.psi has a plane kernel.
+static size_t local_ws_bytes(const Plan& p, int prec, long long rows, bool density) {
   if (rows <= 0 || (prec != kFP32 && prec != kFP64)) return 0;
   const size_t elem = prec == kFP64 ? 16 : 8;
   const size_t sticks = p.plane_threads[prec] > 0 ? p.field_bytes(prec) + (size_t)rows * p.dim(0) * p.smax * elem : 0;
-  if (sticks > 0 && p.whole_plane[prec]) return sticks;
+  if (sticks > 0 && (p.whole_plane[prec] || !density)) return sticks;
   const size_t grid = (size_t)p.n1 * p.n2 * p.n3 * elem;
   long long g = (long long)((size_t(1) << 30) / grid);
   if (g < 1) g = 1;
-  const size_t grids = (size_t)(rows < g ? rows : g) * grid;  // the density takes them where only H.psi has a kernel
+  const size_t grids = (size_t)(rows < g ? rows : g) * grid;
   return sticks > grids ? sticks : grids;
 }
 
 size_t amt_plan_stick_bytes(const amt_plan_t* h, int precision, int nbands) {
   if (!h || nbands <= 0) return 0;
-  return local_ws_bytes(h->p, precision, nbands);
+  return local_ws_bytes(h->p, precision, nbands, true);
 }
 
 int amt_plan_set_route(amt_plan_t* h, int precision, int full_grid) {
@@ -428,7 +428,7 @@ int amt_hpsi_local(const amt_plan_t* h, int precision, const void* psi, void* hp
   }
   if (p.plane_threads[precision] == 0)
     return launch_hpsi_full_grid(p, precision, psi, hpsi, nb, k0, nkk, veff, sticks,
-                                 local_ws_bytes(p, precision, (long long)nb * nkk), (hipStream_t)stream);
+                                 local_ws_bytes(p, precision, (long long)nb * nkk, true), (hipStream_t)stream);
   return launch_hpsi_local(p, precision, psi, hpsi, nb, k0, nkk, veff, sticks, (hipStream_t)stream);
 }
 
@@ -460,7 +460,7 @@ struct HpsiLayout {
 HpsiLayout hpsi_layout(const Plan& p, int prec, int nb, int nkk) {
   HpsiLayout l;
   const size_t elem = prec == kFP64 ? 16 : 8;
-  l.sticks = align_up(local_ws_bytes(p, prec, (long long)nb * nkk));
+  l.sticks = align_up(local_ws_bytes(p, prec, (long long)nb * nkk, false));
   const int np = p.nproj[prec];
   if (np > 0) {
     l.proj = align_up((size_t)nkk * nb * np * elem);
@@ -583,7 +583,7 @@ int amt_density(const amt_plan_t* h, int precision, const void* psi, int nb, int
   }
   if (p.plane_threads[precision] == 0 || !p.whole_plane[precision])
     return launch_density_full_grid(p, precision, psi, nb, k0, band_list, band_weight, nlist, sticks,
-                                    local_ws_bytes(p, precision, (long long)nb * nkk), part, rho, beta, scale,
+                                    local_ws_bytes(p, precision, (long long)nb * nkk, true), part, rho, beta, scale,
                                     (hipStream_t)stream);
   if (nlist > 0 && (nlist + chunk - 1) / chunk > 65535) {
     set_error("density: too many chunks");

@@ -493,3 +493,35 @@ def test_first_call_of_a_length_under_capture(monkeypatch, shape, precision):
         assert torch.equal(out, want)
         assert torch.equal(plan.hpsi(psi, v), want)
     assert len(autotune._FFT) == 1
+
+
+def test_operator_workspace_holds_sticks_only():
+    """An FP64 plane past LDS whose H.psi has the kernel with four lanes per row (108^2): amt_hpsi
+    asks for the sticks of its rows and not for whole grids, which only the density takes there, and
+    stays inside what it asked for."""
+    import torch
+
+    from amaterasu_amd import ops
+    from amaterasu_amd._lib import FP64, check, lib
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    n, nb = 108, 3
+    ecut = 0.5 * ((n / 4.0 - 0.4) * 2.0 * np.pi / (n / 4.0)) ** 2
+    plan = DevicePlan((n, n, n), [GSphere.build(np.eye(3) * n / 4.0, ecut)])
+    sticks = nb * n * plan.smax * 16
+    nbytes = lib().amt_hpsi_workspace(plan.handle, FP64, nb, 1)
+    assert sticks <= nbytes < sticks + 256
+    assert lib().amt_plan_stick_bytes(plan.handle, FP64, nb) == nb * n**3 * 16
+    g = torch.Generator(device="cuda").manual_seed(5)
+    psi = torch.randn((1, nb, plan.npw_pad), dtype=torch.complex128, device="cuda", generator=g)
+    v = torch.randn((n, n, n), dtype=torch.float64, device="cuda", generator=g)
+    want = plan.hpsi(psi, v)
+    ws = torch.full((nbytes + 4096,), 90, dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(psi)
+    check(lib().amt_hpsi(plan.handle, FP64, psi.data_ptr(), out.data_ptr(), nb, 0, 1, v.data_ptr(), ws.data_ptr(), nbytes,
+                         ops.stream_handle()), "hpsi")
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and bool((ws[nbytes:] == 90).all())
+    plan.set_route(FP64, True)
+    assert lib().amt_hpsi_workspace(plan.handle, FP64, nb, 1) >= nb * n**3 * 16
