@@ -394,12 +394,12 @@ int amt_plan_set_route(amt_plan_t* h, int precision, int full_grid) {
   return 0;
 }
 
-static int check_plane(const Plan& p, int prec, bool whole = false) {
+static int check_plane(const Plan& p, int prec) {
   if (prec != kFP32 && prec != kFP64) {
     set_error("precision must be 0 (fp32) or 1 (fp64)");
     return 1;
   }
-  if (p.plane_threads[prec] == 0 || (whole && !p.whole_plane[prec])) {
+  if (p.plane_threads[prec] == 0) {
     set_error("the " + std::to_string(p.n2) + "x" + std::to_string(p.n3) + " plane does not fit one workgroup's LDS at " +
               (prec == kFP64 ? "fp64" : "fp32"));
     return 1;
@@ -532,7 +532,13 @@ int amt_hpsi_local_noalloc(const amt_plan_t* h, int precision, const void* psi, 
     return 1;
   }
   const Plan& p = h->p;
-  if (check_plane(p, precision, true)) return 1;
+  if (check_plane(p, precision)) return 1;
+  if (!p.whole_plane[precision]) {
+    set_error("hpsi_local_noalloc: takes grids whose whole plane fits one workgroup's LDS (" + std::to_string(p.n2) + "x" +
+              std::to_string(p.n3) + " does not at " + (precision == kFP64 ? "fp64" : "fp32") +
+              "); use amt_hpsi_local with a workspace");
+    return 1;
+  }
   if (nb <= 0 || nkk <= 0 || k0 < 0 || k0 + nkk > p.nk) {
     set_error("hpsi_local_noalloc: band/k range outside the plan");
     return 1;

@@ -49,7 +49,9 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
                     const int* miller, const double* kinetic);
 int amt_plan_destroy(amt_plan_t* plan);
 /* info[0..17] = n1, n2, n3, nk, npw_pad, smax, stick_w{fp32,fp64}, stick_threads{fp32,fp64},
- * plane_threads{fp32,fp64} (0 = plane does not fit LDS at that precision: full-grid route),
+ * plane_threads{fp32,fp64} (0 = no plane kernel at that precision: full-grid route; FP64 planes
+ * above ~100^2 do not fit LDS whole, but H.psi has a kernel for them that keeps only the rows with
+ * sticks: then amt_density still takes whole grids and amt_hpsi_local_noalloc refuses the plan),
  * and for grids with compile-time-length kernels (else 0) the launch shapes of
  * amt_plan_set_launch: plane workgroup{fp32,fp64}, sticks per workgroup{fp32,fp64}; then
  * {fp32,fp64} 1 where the plane kernel with one to four lanes per row runs, which has a workgroup
@@ -63,10 +65,10 @@ int amt_plan_info(const amt_plan_t* plan, int* info, int len);
 int amt_plan_set_launch(amt_plan_t* plan, int precision, int plane_threads, int stick_width);
 int amt_plan_nsticks(const amt_plan_t* plan, int* out);
 /* Bytes of the local H.psi / density workspace for `nbands` band rows (all k of one launch):
- * their sticks, or, where the (n2 x n3) plane does not fit one workgroup's LDS at this
- * precision (info[10 + precision] = 0, e.g. FP64 planes above ~100^2), whole grids for
+ * their sticks (and V_eff in the plan's order of axes), or, where the (n2 x n3) plane does not fit
+ * one workgroup's LDS at this precision (e.g. FP64 planes above ~100^2), whole grids for
  * min(nbands, ~1 GiB of grids) rows -- the full-grid route (the plan's scatter, 3-D
- * transforms and gather, a chunk of rows at a time). */
+ * transforms and gather, a chunk of rows at a time), which at least the density takes there. */
 size_t amt_plan_stick_bytes(const amt_plan_t* plan, int precision, int nbands);
 /* Tuning hook, no counterpart in the reference: full_grid = 1 sends this precision's local
  * H.psi and density through the full-grid route even where the plane fits (for comparison);
@@ -119,7 +121,9 @@ int amt_hpsi(const amt_plan_t* plan, int precision, const void* psi, void* hpsi,
  * held by each GPU that runs it until the process ends; rows go through it in launches of
  * at most that many bytes of sticks (whole k-points, or band slices of one k-point), with
  * results bit-identical to amt_hpsi_local. Fails with an error if a single band row needs
- * more sticks than the array holds (n1 * smax * 8 bytes in fp32, 16 in fp64). All calls on
+ * more sticks than the array holds (n1 * smax * 8 bytes in fp32, 16 in fp64; grids whose two equal
+ * axes are not the last two also keep V_eff there), and for grids whose whole (n2 x n3) plane does
+ * not fit one workgroup's LDS, also where amt_hpsi_local has a plane kernel. All calls on
  * one GPU share its array: calls that overlap on one device (other streams, other host
  * threads) race; calls on one stream are ordered.
  */

@@ -130,3 +130,31 @@ def test_noalloc_rejects_a_row_beyond_the_scratch():
     with pytest.raises(AmtError, match="more than the fixed scratch"):
         check(lib().amt_hpsi_local_noalloc(plan.handle, FP32, psi.data_ptr(), out.data_ptr(), 1, 0, 1,
                                            v.data_ptr(), ctypes.c_void_p(0)), "hpsi_local_noalloc")
+
+
+def test_noalloc_names_why_it_refuses_a_plane():
+    """An FP64 plane past LDS (108^2) is refused, as before amt_hpsi_local had a plane kernel for it,
+    with the call that takes it; FP32 runs."""
+    import torch
+
+    from amaterasu_amd import ops
+    from amaterasu_amd._lib import FP32, FP64, AmtError, check, lib
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    n = 108
+    plan = DevicePlan((n, n, n), [GSphere.build(np.eye(3) * n / 4.0, 0.5 * (26.0 * 2.0 * np.pi / (n / 4.0)) ** 2)])
+    assert plan.plane_ok[FP32] and plan.plane_ok[FP64]
+    for prec, dt in ((FP64, torch.complex128), (FP32, torch.complex64)):
+        psi = torch.randn((1, 1, plan.npw_pad), dtype=dt, device="cuda")
+        out, v = torch.empty_like(psi), torch.randn((n, n, n), dtype=ops.real_dtype(prec), device="cuda")
+        call = lambda: check(lib().amt_hpsi_local_noalloc(  # noqa: E731
+            plan.handle, prec, psi.data_ptr(), out.data_ptr(), 1, 0, 1, v.data_ptr(), ctypes.c_void_p(0)), "noalloc")
+        if prec == FP64:
+            with pytest.raises(AmtError, match="use amt_hpsi_local with a workspace"):
+                call()
+        else:
+            torch.cuda.synchronize()
+            call()
+            torch.cuda.synchronize()
+            assert bool(torch.isfinite(torch.view_as_real(out)).all())
