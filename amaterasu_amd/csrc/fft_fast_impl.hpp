@@ -483,7 +483,7 @@ __device__ __forceinline__ double quad_perm(double v) {
   return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
                           __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
 }
-// Length-N transforms of one row or column by P neighbouring lanes (P = 1, 2 or 4), M = N / P
+// Length-N transforms of one row or column by P neighbouring lanes (P = 1 or 4), M = N / P
 // points in each lane's registers. Inverse: lane p computes outputs P q + p from the live inputs
 // at slot(j) * stride:
 //   y_p[j] = w_N^{p j} sum_s i^{p s} x[j + s M] (P = 4),  u[P q + p] = DFT_M(y_p)[q],
@@ -493,17 +493,14 @@ __device__ __forceinline__ void pruned_inverse(C (&y)[N / P], const Get& get, in
   using R = decltype(C::x);
   using Pr = Prune<N>;
   constexpr int M = N / P;
-  // i^(p s) of the P = 4 first step for s = 1 (its conjugate for s = 3), (-1)^p for s = 2 and P = 2
+  static_assert(P == 1 || P == 4, "one lane per row or a quad");
+  // i^(p s) of the P = 4 first step for s = 1 (its conjugate for s = 3), (-1)^p for s = 2
   const R cr = p == 0 ? (R)1 : p == 2 ? (R)-1 : (R)0, ci = p == 1 ? (R)1 : p == 3 ? (R)-1 : (R)0;
   const R sg = p & 1 ? (R)-1 : (R)1;
   static_for<M>([&](auto j_) {
     constexpr int j = j_;
     C v = cmake<C>(0, 0);
     if constexpr (Pr::live(j)) v = get(j_);
-    if constexpr (P == 2 && Pr::live(j + M)) {
-      const C x = get(std::integral_constant<int, j + M>{});
-      v = cmake<C>(v.x + sg * x.x, v.y + sg * x.y);
-    }
     if constexpr (P == 4) {
       if constexpr (Pr::live(j + M)) {
         const C x = get(std::integral_constant<int, j + M>{});
@@ -536,28 +533,23 @@ __device__ __forceinline__ void pruned_forward(C (&y)[N / P], const Range& range
   constexpr int M = N / P;
   lane_dft<M, -1>(y);
   if constexpr (P > 1) {
-    const R sa = (P == 4 ? p >= 2 : p == 1) ? (R)-1 : (R)1, sb = p & 1 ? (R)-1 : (R)1;
+    const R sa = p >= 2 ? (R)-1 : (R)1, sb = p & 1 ? (R)-1 : (R)1;
     const R c3 = p == 3 ? (R)0 : (R)1, s3 = p == 3 ? (R)1 : (R)0;
     static_for<M>([&](auto k_) {
       constexpr int k = k_;
-      constexpr int ctrl = P == 4 ? 0x4E : 0xB1;  // lanes 2 3 0 1, or 1 0 3 2
       if constexpr (k > 0) y[k] = cmul(y[k], tw[p * M + k]);
-      R zx = quad_perm<ctrl>(y[k].x) + sa * y[k].x, zy = quad_perm<ctrl>(y[k].y) + sa * y[k].y;
-      if constexpr (P == 4) {
-        const R rx = zx * c3 - zy * s3, ry = zy * c3 + zx * s3;  // lane 3: times i
-        zx = quad_perm<0xB1>(rx) + sb * rx;
-        zy = quad_perm<0xB1>(ry) + sb * ry;
-      }
-      y[k].x = zx;
-      y[k].y = zy;
+      const R zx = quad_perm<0x4E>(y[k].x) + sa * y[k].x, zy = quad_perm<0x4E>(y[k].y) + sa * y[k].y;  // lanes 2 3 0 1
+      const R rx = zx * c3 - zy * s3, ry = zy * c3 + zx * s3;                                          // lane 3: times i
+      y[k].x = quad_perm<0xB1>(rx) + sb * rx;  // lanes 1 0 3 2
+      y[k].y = quad_perm<0xB1>(ry) + sb * ry;
     });
   }
-  const int s = P < 4 ? p : p == 0 ? 0 : p == 1 ? 2 : p == 2 ? 3 : 1;
+  const int s = p == 0 ? 0 : p == 1 ? 2 : p == 2 ? 3 : 1;
   const auto put = range(s);
   static_for<M>([&](auto k_) {
     constexpr int k = k_;
     constexpr unsigned mask = (Pr::live(k) ? 1u : 0u) | (P > 1 && Pr::live(k + M) ? 2u : 0u) |
-                              (P == 4 && Pr::live(k + 2 * M) ? 4u : 0u) | (P == 4 && Pr::live(k + 3 * M) ? 8u : 0u);
+                              (P > 1 && Pr::live(k + 2 * M) ? 4u : 0u) | (P > 1 && Pr::live(k + 3 * M) ? 8u : 0u);
     if constexpr (P == 1) {
       if constexpr (mask != 0) put(k_, y[k]);
     } else {
