@@ -589,7 +589,7 @@ __device__ __forceinline__ void slots_forward(C (&y)[N / P], C* base, int stride
 // 108^3, 440 bands 1.92 against 2.62 ms, 42^3, 1024 bands 199 against 223 us; FP64 108^3, 45 bands
 // 0.42 ms where whole-grid transforms took 5.9 ms. What bounds it: VALU issue for one lane per row
 // (a third of the lanes idle at N = 42), the waits around five barriers with four. Which lengths
-// take it, and both sides' times: lane_count().
+// take it, and both sides' times: lane_count(); from how many planes on: lane_planes().
 template <int N, int P, typename C, typename R, int NTH, int WAVES>
 __global__ __launch_bounds__(NTH, WAVES) void k_plane_lane_n(C* __restrict__ sticks, const int* __restrict__ stick_jk,
                                                              const int* __restrict__ nsticks,
@@ -714,8 +714,9 @@ int stick_t(const Plan& p, int pass, const void* psi, void* hpsi, void* sticks, 
              : stick_pass<N, R, W>(p, pass, psi, hpsi, sticks, nb, k0, nkb, s);
 }
 
+// lane: the call is to take the one-lane kernel (Plan::lane_from).
 template <int N, typename R>
-int plane_t(const Plan& p, void* sticks_, const void* veff_, int nb, int k0, int nkb, hipStream_t s) {
+int plane_t(const Plan& p, bool lane, void* sticks_, const void* veff_, int nb, int k0, int nkb, hipStream_t s) {
   using C = typename Cplx<R>::T;
   constexpr int prec = sizeof(R) == 8 ? kFP64 : kFP32;
   C* sticks = static_cast<C*>(sticks_);
@@ -723,7 +724,7 @@ int plane_t(const Plan& p, void* sticks_, const void* veff_, int nb, int k0, int
   const int a = p.axis[1], n1 = p.dim(0);
   const C* tw = prec == kFP64 ? (const C*)p.d_tw64[a] : (const C*)p.d_tw32[a];
   if constexpr (LanePlane<N, R>::use) {
-    if (p.narrow) {
+    if (lane) {
       using L = LanePlane<N, R>;
       constexpr size_t lds = (size_t)Prune<N>::ROWS * Prune<N>::LD * sizeof(C);
       hipLaunchKernelGGL((k_plane_lane_n<N, L::lanes, C, R, L::threads, L::waves>),
@@ -777,13 +778,13 @@ int AMT_PART_FN(fast_stick)(const Plan& p, int prec, int pass, const void* psi, 
   }
 }
 
-int AMT_PART_FN(fast_plane)(const Plan& p, int prec, void* sticks, const void* veff, int nb, int k0, int nkb,
-                            hipStream_t s) {
+int AMT_PART_FN(fast_plane)(const Plan& p, int prec, bool lane, void* sticks, const void* veff, int nb, int k0,
+                            int nkb, hipStream_t s) {
   switch (p.dim(1)) {
 #define AMT_CASE(N)                                                              \
   case N:                                                                        \
-    return prec == kFP64 ? plane_t<N, double>(p, sticks, veff, nb, k0, nkb, s) \
-                         : plane_t<N, float>(p, sticks, veff, nb, k0, nkb, s);
+    return prec == kFP64 ? plane_t<N, double>(p, lane, sticks, veff, nb, k0, nkb, s) \
+                         : plane_t<N, float>(p, lane, sticks, veff, nb, k0, nkb, s);
     AMT_PART(AMT_CASE)
 #undef AMT_CASE
     default:
