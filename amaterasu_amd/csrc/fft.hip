@@ -16,6 +16,7 @@
 #include <cmath>
 #include <vector>
 
+#include "fft_reg.hpp"
 #include "kernels.hpp"
 
 namespace amt {
@@ -380,20 +381,34 @@ int launch_density_finish(double* rho, int nspin, long long ngrid, double volume
   return check(hipGetLastError(), "density_finish launch");
 }
 
-// Bands per workgroup of the plane accumulation, by the rounds of workgroups the chip runs (one
-// or two per CU, by the plane's LDS) times the bands of each, one more band for a workgroup's
-// start and its write of a partial plane. 84^3 in FP64, 128 bands: 43 bands fill one round of
-// 252 workgroups (422 us), 8 take 5.25 rounds of 16 (484); 16 bands: 6 (97 us against 107 for 8);
-// 42^3, 128 bands: 11 or 22 (123, 120; 8: 131); 25^3: 4 to 8 alike.
+// Bands per workgroup of the plane accumulation, by the rounds of workgroups the chip runs (one or
+// two per CU, by the plane's LDS) times the bands of each, and a workgroup's start and its write of a
+// partial plane. 84^3 in FP64, 128 bands: 43 bands fill one round of 252 workgroups (422 us), 8 take
+// 5.25 rounds of 16 (484); 16 bands: 6 (97 us against 107 for 8); 42^3, 128 bands: 22 (86; 8: 95).
+// Two FP64 workgroups on a CU share its FP64 units: a round of them takes nearly twice as long (64
+// bands at 32^3 27 us in chunks of 8, one a CU, 32 in chunks of 4; 40 bands at 42^3 38 against 42; short
+// odd lengths, whose columns meet no bank conflicts, less: 64 bands at 25^3 24 against 21). FP32
+// rounds of two cost no more than rounds of one (64 bands at 42^3: 6 35 us, 11 40), but for the lengths
+// 4 a, a of 7 or more points, whose second phase meets bank conflicts (64 bands at 32^3: 4 30 us, 8 26).
+// More bands in one FP64 accumulator round more often than chunks of 8 did: 128 bands at 84^3 are off
+// by 2.5e-16 of the 64-bit value where they were by 2.2e-16.
 int density_chunk(const Plan& p, int prec, int nlist) {
   if (!p.fast || nlist < 1) return 8;
-  const long long plane = (long long)p.dim(1) * p.dim(2) * (prec == kFP64 ? 16 : 8), n1 = p.dim(0);
-  const long long slots = 256 * (2 * (plane + 4096) <= 160 * 1024 ? 2 : 1);
-  long long best = 0, cost = 0;
+  const bool fp64 = prec == kFP64;
+  const long long n = p.dim(1), n1 = p.dim(0);
+  const int per_cu = 2 * (n * n * (fp64 ? 16 : 8) + 4096) <= 160 * 1024 ? 2 : 1;
+  const int a = split_n1((int)n);
+  const bool shared = fp64 ? !(n % 2 == 1 && n <= 25) : a >= 7 && a * 4 == n;
+  const double pair = shared ? 1.85 : fp64 ? 1.55 : 1.0;           // a round of two per CU, in rounds of one
+  const double extra = fp64 && shared && per_cu == 2 ? 2.0 : 1.0;  // a workgroup's start and end, in bands
+  long long best = 0;
+  double cost = 0.0;
   for (long long c = 1; c <= nlist; ++c) {
     const long long nch = (nlist + c - 1) / c;
     if (nch > 65535) continue;
-    const long long t = (nch * n1 + slots - 1) / slots * (c + 1);
+    const long long wg = nch * n1, full = wg / (256 * per_cu), rest = wg % (256 * per_cu);
+    const double rounds = (per_cu == 2 ? pair : 1.0) * (double)full + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : pair);
+    const double t = rounds * ((double)c + extra);
     if (best == 0 || t <= cost) {
       best = c;
       cost = t;

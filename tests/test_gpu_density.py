@@ -110,3 +110,21 @@ def test_density_chunk_choice(si2_system, nlist, dtype):
         plan.accumulate_density(psi, rows, w, rho, beta=0.0, chunk=c)
         out.append(rho.cpu().numpy())
     assert np.abs(out[0] - out[1]).max() <= 2 * nlist * 2.0**-53 * np.abs(out[1]).max()
+
+
+@pytest.mark.parametrize("n,bands,dtype,rounds", [(32, 64, "complex128", 1), (42, 40, "complex128", 1),
+                                                  (28, 64, "complex128", 1), (25, 64, "complex128", 2),
+                                                  (84, 128, "complex128", 1), (32, 64, "complex64", 1),
+                                                  (44, 40, "complex64", 1), (42, 64, "complex64", 2)])
+def test_chunk_counts_a_cu_shared_by_two_workgroups(n, bands, dtype, rounds):
+    """Partial sums that one workgroup a CU can hold are not split over two (n planes times the chunks: at
+    most 256 workgroups) where two in FP64, or in FP32 at the lengths 4 a, would wait for each other;
+    other FP32 lengths and short odd FP64 ones gain from two."""
+    import torch
+
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    sphere = GSphere.build(np.eye(3) * n / 4.0, 0.5 * ((n / 4.0 - 0.4) * 2.0 * np.pi / (n / 4.0)) ** 2)
+    chunk = DevicePlan((n, n, n), [sphere]).density_chunk(getattr(torch, dtype), bands)
+    assert 1 <= chunk <= bands and -(-(-(-bands // chunk) * n) // 256) == rounds
