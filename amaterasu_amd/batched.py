@@ -171,6 +171,14 @@ def _solve_streams(count: int) -> list:
     return have[:count]
 
 
+#: Two or three matrices with more rows than this keep a chain and a stream each: their column steps
+#: fill the chip alone, and in a shared launch the matrices wait for each other's last workgroups. One
+#: chain against one per stream (ms): two of 1024 rows 12.5/15.5, 1200 18.4/19.0, 1400 27.1/25.6, 1760
+#: 46.3/41.0; three of 1200 22.5/24.0, 1400 33.5/31.9, 1760 61.6/51.7; four, where the host issuing four
+#: chains is the bound, of 1400 41.9/51.5, 2048 111/114.
+CHAIN_ROWS = 1280
+
+
 def _lowest(proj: torch.Tensor, used, nbands: int):
     """Lowest ``nbands`` eigenpairs of the leading used[k] x used[k] block of each projected
     matrix, at its own size with the per-k Davidson's solver (the library's for 2..2048 rows):
@@ -181,10 +189,10 @@ def _lowest(proj: torch.Tensor, used, nbands: int):
     self-consistent run against one chain per k-point on its own stream, together with the
     appends and the preconditioner in one launch each, since the host issuing launches was the
     bound). Sizes it does not take run concurrently, one side stream per k, ordered against the
-    caller's stream by events."""
+    caller's stream by events, and so do two or three matrices past ``CHAIN_ROWS``."""
     nk, n = proj.shape[0], proj.shape[-1]
     used = [int(u) for u in used]
-    if all(HEEV_MIN <= c <= HEEV_MAX for c in used):
+    if all(HEEV_MIN <= c <= HEEV_MAX for c in used) and not (nk in (2, 3) and max(used) > CHAIN_ROWS):
         return ops.heev_lowest_batched(proj, used, nbands)
     w = torch.empty((nk, nbands), dtype=torch.float64, device=proj.device)
     rot = torch.zeros((nk, nbands, n), dtype=proj.dtype, device=proj.device)

@@ -200,3 +200,29 @@ def test_subspace_growth_kernels(dtype, npw, width):
             else:
                 one = ops.precondition(res, vec, kin[k], torch.tensor([rows[k, i]], device="cuda"))
                 assert torch.equal(out[k, i], one[0])
+
+
+@pytest.mark.parametrize("sizes", [[1281, 1279], [1300, 1300, 1290]])
+def test_few_large_projected_matrices_keep_a_stream_each(monkeypatch, sizes):
+    """Two or three matrices past the size up to which one chain of launches is faster are solved on
+    streams of their own, with the bits of the one-matrix solver; smaller ones and four share a chain."""
+    import torch
+
+    from amaterasu_amd import batched, ops
+
+    g = torch.Generator(device="cuda").manual_seed(len(sizes))
+    n = max(sizes)
+    a = torch.randn((len(sizes), n, n), dtype=torch.complex128, device="cuda", generator=g)
+    a = a + a.mH
+    calls = []
+    chain = ops.heev_lowest_batched
+    monkeypatch.setattr(ops, "heev_lowest_batched", lambda *args: calls.append(1) or chain(*args))
+    w, z = batched._lowest(a, sizes, 9)
+    assert not calls
+    for k, c in enumerate(sizes):
+        ws, zs = ops.heev_lowest(a[k, :c, :c].contiguous(), 9)
+        assert torch.equal(w[k], ws) and torch.equal(z[k, :, :c], zs) and not z[k, :, c:].any()
+    small = a[:, :60, :60]
+    batched._lowest(small, [60] * len(sizes), 9)
+    batched._lowest(torch.cat([a, a])[:4], [sizes[0] - 2] * 4, 3)
+    assert len(calls) == 2
