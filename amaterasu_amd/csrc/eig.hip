@@ -46,9 +46,9 @@ constexpr int kInverseRounds = 2;
 
 // The matrices of one launch set: matrix z = blockIdx.z has n[z] rows, and its workspace buffers lie
 // z stride bytes after those of the first. The chains of the matrices are independent and each
-// launch leaves most of the chip idle, so the matrices of a set share every launch. (Four of 20 to
-// 80 rows: one chain of 14 launches where four chains on four streams kept the host busy for
-// 0.5 ms a step.)
+// launch leaves most of the chip idle, so the matrices of a set share every launch. (A chain is 11
+// launches and one more for each trailing length above 64, 26 at 80 rows: one of them for four
+// matrices of 20 to 80 rows, where four chains on four streams kept the host busy for 0.5 ms a step.)
 constexpr int kHeevBatch = 16;
 struct HeevBatch {
   int n[kHeevBatch];

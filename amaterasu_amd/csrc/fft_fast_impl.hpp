@@ -679,7 +679,10 @@ struct LanePlane {
   // eight where LDS holds one plane per CU. (A workgroup of six leaves SIMDs uneven: 84^2 FP32
   // 511 us against 322.)
   static constexpr int threads = lanes == 1 ? 64 : fp64 && N > 100 ? 512 : 256;
-  // wavefronts per SIMD that the registers are held to
+  // Wavefronts per SIMD that the registers are held to: by the LDS of a plane with four lanes, and
+  // for one lane 4 up to the length whose row just fits 128 registers, 3 up to 60, 2 in FP64. The
+  // lengths next to a step spill (FP32 10 to 48 registers at 44, 45 and 48, 24 to 61 at 55, 56 and 60) and
+  // are still ahead of the four-step kernel where lane_planes() uses them.
   static constexpr int waves = lanes == 1 ? (fp64 ? 2 : N <= 48 ? 4 : 3) : fp64 && N > 100 ? 1 : 2;
 };
 

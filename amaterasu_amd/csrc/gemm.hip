@@ -16,10 +16,10 @@
 // accumulator differs (measured on gfx950): accumulator element q of lane l is
 // D[4 (l / 16) + q][l % 16] for FP32 and D[l / 16 + 4 q][l % 16] for FP64.
 //
-// Tiling: a 256-thread workgroup computes 16 W rows x 64 columns, W = 1..7 chosen for the row
-// count (plan_gemm): each of the four wavefronts owns 16 columns and all 16 W rows, so 8 bands
-// compute 16 rows, 45 compute 48, 160 two times 80, 440 four times 112, where fixed 64-row tiles
-// computed 64, 64, 192 and 448. K advances 128 bytes of a row at a time (16 complex64, 8
+// Tiling: a 256-thread workgroup computes 16 W rows x 64 columns, W = 1..5 (7 in FP32 without FP64
+// sums, which take the registers) chosen for the row count (plan_gemm): each of the four wavefronts
+// owns 16 columns and all 16 W rows, so 8 bands compute 16 rows, 45 compute 48 and 160 compute 160,
+// where fixed 64-row tiles computed 64, 64 and 192. K advances 128 bytes of a row at a time (16 complex64, 8
 // complex128) through two LDS buffers: the next tile's 16-byte global loads are issued before
 // this tile's MFMAs and stored after them, one barrier per tile. Rows past M are clamped to the
 // last row and columns of an NN product past N to the last ones (their results are not stored),
