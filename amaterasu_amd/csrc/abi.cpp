@@ -220,6 +220,7 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
     for (int j = 0; j < q2; ++j)
       if (used[j]) rows[(size_t)k * q2 + nrows[k]++] = j;
   }
+  p.narrow = narrow;
   // per-row stick masks and first-stick indices for the compile-time plane kernels
   std::vector<unsigned long long> rowmask, livemask;
   std::vector<int> rowstart;
@@ -266,9 +267,7 @@ int amt_plan_create(amt_plan_t** out, int n1, int n2, int n3, int nk, const int*
     // The one-lane kernel (narrow plans) holds the rows with sticks only and needs neither.
     if (p.fast) {
       p.whole_plane[prec] = plds + 24LL * q2 <= lds_max;
-      const long long planes = narrow ? lane_plane_planes(q2, prec) : 0;
-      if (planes > 0) p.lane_from[prec] = p.whole_plane[prec] ? (int)((planes + q1 - 1) / q1) : 1;
-      p.plane_threads[prec] = p.whole_plane[prec] || p.lane_from[prec] > 0 ? 256 : 0;
+      p.plane_threads[prec] = p.whole_plane[prec] || (narrow && lane_plane_supported(q2, prec)) ? 256 : 0;
     } else {
       p.plane_threads[prec] = (pt <= 1024 && plds <= lds_max) ? pt : 0;
       p.whole_plane[prec] = p.plane_threads[prec] > 0;
@@ -322,13 +321,14 @@ int amt_plan_info(const amt_plan_t* h, int* info, int len) {
     return 1;
   }
   const Plan& p = h->p;
+  auto lane = [&](int prec) { return p.fast && p.narrow && lane_plane_supported(p.dim(1), prec) ? 1 : 0; };
   const int v[18] = {p.n1,           p.n2,           p.n3,
                      p.nk,           p.npw_pad,      p.smax,
                      p.stick_w[0],   p.stick_w[1],   p.stick_threads[0],
                      p.stick_threads[1], p.plane_threads[0], p.plane_threads[1],
                      p.fast ? p.plane_nth[0] : 0, p.fast ? p.plane_nth[1] : 0,
                      p.fast ? p.fast_stick_w[0] : 0, p.fast ? p.fast_stick_w[1] : 0,
-                     p.lane_from[0], p.lane_from[1]};
+                     lane(kFP32), lane(kFP64)};
   for (int i = 0; i < len && i < 18; ++i) info[i] = v[i];
   return 0;
 }

@@ -525,9 +525,9 @@ static int hpsi_local_t(const Plan& p, const void* psi_, void* hpsi_, int nb, in
 }
 
 int launch_hpsi_local(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                      const void* veff, void* sticks, hipStream_t s, int stage, bool pad, int rows) {
+                      const void* veff, void* sticks, hipStream_t s, int stage, bool pad) {
   if (p.fast) {
-    if (launch_hpsi_fast(p, prec, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage, pad, rows)) {
+    if (launch_hpsi_fast(p, prec, psi, hpsi, nb, k0, nkk, veff, sticks, s, stage, pad)) {
       set_error(std::string("hpsi (compile-time length) launch: ") + hipGetErrorString(hipGetLastError()));
       return 1;
     }

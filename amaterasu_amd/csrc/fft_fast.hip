@@ -14,7 +14,7 @@ bool fast_length_supported(int n) {
   }
 }
 
-long long lane_plane_planes(int n, int prec) { return fast_length_supported(n) ? lane_planes(n, prec == kFP64) : 0; }
+bool lane_plane_supported(int n, int prec) { return fast_length_supported(n) && lane_count(n, prec == kFP64) > 0; }
 int lane_plane_half_width(int n) { return lane_half_width(n); }
 
 // The first part that knows the length answers (-1: not its length).
@@ -29,9 +29,8 @@ static int stick(const Plan& p, int prec, int pass, const void* psi, void* hpsi,
                  int nkb, hipStream_t s) {
   AMT_FIRST_PART(fast_stick, p, prec, pass, psi, hpsi, sticks, nb, k0, nkb, s);
 }
-static int plane(const Plan& p, int prec, bool lane, void* sticks, const void* veff, int nb, int k0, int nkb,
-                 hipStream_t s) {
-  AMT_FIRST_PART(fast_plane, p, prec, lane, sticks, veff, nb, k0, nkb, s);
+static int plane(const Plan& p, int prec, void* sticks, const void* veff, int nb, int k0, int nkb, hipStream_t s) {
+  AMT_FIRST_PART(fast_plane, p, prec, sticks, veff, nb, k0, nkb, s);
 }
 static int density(const Plan& p, int prec, const void* sticks, int nb, int k0, const int* list, const double* weight,
                    int nlist, int chunk, double* part, hipStream_t s) {
@@ -50,9 +49,8 @@ __global__ void k_permute_field(const R* __restrict__ src, R* __restrict__ dst, 
 }
 
 int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                     const void* veff, void* ws, hipStream_t s, int stage, bool pad, int rows) {
+                     const void* veff, void* ws, hipStream_t s, int stage, bool pad) {
   const int nkb = nb * nkk;
-  const bool lane = p.lane_from[prec] > 0 && (rows > 0 ? rows : nkb) >= p.lane_from[prec];
   void* sticks = static_cast<unsigned char*>(ws) + p.field_bytes(prec);
   if (stage == 0 || stage == 1)
     if (stick(p, prec, kStickInverse, psi, nullptr, sticks, nb, k0, nkb, s)) return 1;
@@ -70,7 +68,7 @@ int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int n
       if (hipGetLastError() != hipSuccess) return 1;
       v = ws;
     }
-    if (plane(p, prec, lane, sticks, v, nb, k0, nkb, s)) return 1;
+    if (plane(p, prec, sticks, v, nb, k0, nkb, s)) return 1;
   }
   if (stage == 0 || stage == 3)
     if (stick(p, prec, pad ? kStickForwardPad : kStickForward, psi, hpsi, sticks, nb, k0, nkb, s)) return 1;

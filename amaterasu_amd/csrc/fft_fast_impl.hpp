@@ -589,7 +589,7 @@ __device__ __forceinline__ void slots_forward(C (&y)[N / P], C* base, int stride
 // 108^3, 440 bands 1.92 against 2.62 ms, 42^3, 1024 bands 199 against 223 us; FP64 108^3, 45 bands
 // 0.42 ms where whole-grid transforms took 5.9 ms. What bounds it: VALU issue for one lane per row
 // (a third of the lanes idle at N = 42), the waits around five barriers with four. Which lengths
-// take it, and both sides' times: lane_count(); from how many planes on: lane_planes().
+// take it, and both sides' times: lane_count().
 template <int N, int P, typename C, typename R, int NTH, int WAVES>
 __global__ __launch_bounds__(NTH, WAVES) void k_plane_lane_n(C* __restrict__ sticks, const int* __restrict__ stick_jk,
                                                              const int* __restrict__ nsticks,
@@ -682,7 +682,7 @@ struct LanePlane {
   // Wavefronts per SIMD that the registers are held to: by the LDS of a plane with four lanes, and
   // for one lane 4 up to the length whose row just fits 128 registers, 3 up to 60, 2 in FP64. The
   // lengths next to a step spill (FP32 10 to 48 registers at 44, 45 and 48, 24 to 61 at 55, 56 and 60) and
-  // are still ahead of the four-step kernel where lane_planes() uses them.
+  // are still ahead of the four-step kernel where lane_count() has them.
   static constexpr int waves = lanes == 1 ? (fp64 ? 2 : N <= 48 ? 4 : 3) : fp64 && N > 100 ? 1 : 2;
 };
 
@@ -717,9 +717,8 @@ int stick_t(const Plan& p, int pass, const void* psi, void* hpsi, void* sticks, 
              : stick_pass<N, R, W>(p, pass, psi, hpsi, sticks, nb, k0, nkb, s);
 }
 
-// lane: the call is to take the one-lane kernel (Plan::lane_from).
 template <int N, typename R>
-int plane_t(const Plan& p, bool lane, void* sticks_, const void* veff_, int nb, int k0, int nkb, hipStream_t s) {
+int plane_t(const Plan& p, void* sticks_, const void* veff_, int nb, int k0, int nkb, hipStream_t s) {
   using C = typename Cplx<R>::T;
   constexpr int prec = sizeof(R) == 8 ? kFP64 : kFP32;
   C* sticks = static_cast<C*>(sticks_);
@@ -727,7 +726,7 @@ int plane_t(const Plan& p, bool lane, void* sticks_, const void* veff_, int nb, 
   const int a = p.axis[1], n1 = p.dim(0);
   const C* tw = prec == kFP64 ? (const C*)p.d_tw64[a] : (const C*)p.d_tw32[a];
   if constexpr (LanePlane<N, R>::use) {
-    if (lane) {
+    if (p.narrow) {
       using L = LanePlane<N, R>;
       constexpr size_t lds = (size_t)Prune<N>::ROWS * Prune<N>::LD * sizeof(C);
       hipLaunchKernelGGL((k_plane_lane_n<N, L::lanes, C, R, L::threads, L::waves>),
@@ -781,13 +780,13 @@ int AMT_PART_FN(fast_stick)(const Plan& p, int prec, int pass, const void* psi, 
   }
 }
 
-int AMT_PART_FN(fast_plane)(const Plan& p, int prec, bool lane, void* sticks, const void* veff, int nb, int k0,
-                            int nkb, hipStream_t s) {
+int AMT_PART_FN(fast_plane)(const Plan& p, int prec, void* sticks, const void* veff, int nb, int k0, int nkb,
+                            hipStream_t s) {
   switch (p.dim(1)) {
 #define AMT_CASE(N)                                                              \
   case N:                                                                        \
-    return prec == kFP64 ? plane_t<N, double>(p, lane, sticks, veff, nb, k0, nkb, s) \
-                         : plane_t<N, float>(p, lane, sticks, veff, nb, k0, nkb, s);
+    return prec == kFP64 ? plane_t<N, double>(p, sticks, veff, nb, k0, nkb, s) \
+                         : plane_t<N, float>(p, sticks, veff, nb, k0, nkb, s);
     AMT_PART(AMT_CASE)
 #undef AMT_CASE
     default:

@@ -53,9 +53,7 @@ struct Plan {
   bool fast = false;
   int axis[3] = {0, 1, 2};
   bool permuted = false;
-  // Band rows of a call from which the one-lane plane kernel runs, [prec]: 0 where the length has
-  // none or a plane-axis Miller index is past lane_plane_half_width, 1 where no other kernel fits LDS.
-  int lane_from[2] = {0, 0};
+  bool narrow = false;         // plane-axis Miller indices within lane_plane_half_width
   int length(int natural) const { return natural == 0 ? n1 : natural == 1 ? n2 : n3; }
   int dim(int a) const { return length(axis[a]); }
   long long stride(int a) const { return axis[a] == 0 ? (long long)n2 * n3 : axis[a] == 1 ? n3 : 1; }
@@ -96,19 +94,17 @@ enum StickPass { kStickForward = 0, kStickInverse = 1, kStickForwardPad = 2 };
 
 // Compile-time-length kernels (fft_fast.hip) for grids with two axes of one listed length.
 bool fast_length_supported(int n);
-long long lane_plane_planes(int n, int prec);
+bool lane_plane_supported(int n, int prec);
 int lane_plane_half_width(int n);
 int launch_hpsi_fast(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                     const void* veff, void* sticks, hipStream_t s, int stage, bool pad, int rows);
+                     const void* veff, void* sticks, hipStream_t s, int stage, bool pad = false);
 int launch_density_fast(const Plan& p, int prec, const void* psi, int nb, int k0, int nkk, const int* list,
                         const double* weight, int nlist, int chunk, void* sticks, double* part, hipStream_t s);
 
 // Local part of H.psi (kinetic + V_eff) for nbk = nkb bands laid out [kb][npw_pad],
-// kb = k * nb + b for k in [k0, k0 + nkb / nb). `sticks` is nkb * n1 * smax complex. `rows`: the band
-// rows of the whole call where this launch is a part of it (0: all), which choose the plane kernel.
+// kb = k * nb + b for k in [k0, k0 + nkb / nb). `sticks` is nkb * n1 * smax complex.
 int launch_hpsi_local(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
-                      const void* veff, void* sticks, hipStream_t s, int stage = 0, bool pad = false,
-                      int rows = 0);
+                      const void* veff, void* sticks, hipStream_t s, int stage = 0, bool pad = false);
 // launch_hpsi_local over the library's fixed scratch array (noalloc.hip).
 long long noalloc_rows_per_launch(const Plan& p, int prec);
 int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,

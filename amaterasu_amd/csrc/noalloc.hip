@@ -63,8 +63,7 @@ long long noalloc_rows_per_launch(const Plan& p, int prec) {
 
 // amt_hpsi_local over the scratch array: the [nkk][nb] rows go in launches of whole k-points
 // when a k-point's bands fit, else in band slices of one k-point at a time (rows are
-// independent, and the whole call's rows choose the plane kernel, so the split does not change a
-// single bit of the result).
+// independent, so the split does not change a single bit of the result).
 int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int nb, int k0, int nkk,
                        const void* veff, hipStream_t s) {
   const long long rows_max = noalloc_rows_per_launch(p, prec);
@@ -77,8 +76,6 @@ int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int
   }
   unsigned char* ws = static_cast<unsigned char*>(scratch_on_current_device());
   if (!ws) return 1;
-  const long long all = (long long)nb * nkk;
-  const int rows = (int)(all < 0x7fffffff ? all : 0x7fffffff);
   const size_t elem = prec == kFP64 ? 16 : 8;
   const size_t row_stride = (size_t)p.npw_pad * elem;
   const unsigned char* in = static_cast<const unsigned char*>(psi);
@@ -88,7 +85,7 @@ int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int
     for (int kk = 0; kk < nkk; kk += kper) {
       const int nk_here = nkk - kk < kper ? nkk - kk : kper;
       const size_t off = (size_t)kk * nb * row_stride;
-      if (launch_hpsi_local(p, prec, in + off, out + off, nb, k0 + kk, nk_here, veff, ws, s, 0, false, rows)) return 1;
+      if (launch_hpsi_local(p, prec, in + off, out + off, nb, k0 + kk, nk_here, veff, ws, s)) return 1;
     }
     return 0;
   }
@@ -96,7 +93,7 @@ int hpsi_local_noalloc(const Plan& p, int prec, const void* psi, void* hpsi, int
     for (int b0 = 0; b0 < nb; b0 += (int)rows_max) {
       const int nbc = nb - b0 < rows_max ? nb - b0 : (int)rows_max;
       const size_t off = ((size_t)kk * nb + b0) * row_stride;
-      if (launch_hpsi_local(p, prec, in + off, out + off, nbc, k0 + kk, 1, veff, ws, s, 0, false, rows)) return 1;
+      if (launch_hpsi_local(p, prec, in + off, out + off, nbc, k0 + kk, 1, veff, ws, s)) return 1;
     }
   }
   return 0;

@@ -521,7 +521,7 @@ def hpsi_bench(steps: int, warmup: int) -> tuple:
     achieved = alg_bytes / (plane_ms * 1e-3) / 1e9
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": _traffic_from_profile(),
-                "kernel": "k_plane_lane_n (fp32)" if 0 < plan.info[16] <= nb * plan.nk else "k_plane_vloc_n (fp32)",
+                "kernel": "k_plane_lane_n (fp32)" if plan.info[16] else "k_plane_vloc_n (fp32)",
                 "algorithmic_bytes_per_launch": alg_bytes,
                 "avg_launch_ms": round(plane_ms, 5)}
     # the stick kernels against the same roofline: sticks S n1 s read or written, psi (and H psi) npw s

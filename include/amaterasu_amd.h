@@ -54,8 +54,8 @@ int amt_plan_destroy(amt_plan_t* plan);
  * sticks: then amt_density still takes whole grids and amt_hpsi_local_noalloc refuses the plan),
  * and for grids with compile-time-length kernels (else 0) the launch shapes of
  * amt_plan_set_launch: plane workgroup{fp32,fp64}, sticks per workgroup{fp32,fp64}; then
- * {fp32,fp64} the band rows of a call from which the plane kernel with one to four lanes per row
- * runs, which has a workgroup of its own (0: at no size). The first `len` of them are written. */
+ * {fp32,fp64} 1 where the plane kernel with one to four lanes per row runs, which has a workgroup
+ * of its own. The first `len` of them are written. */
 int amt_plan_info(const amt_plan_t* plan, int* info, int len);
 /* Tuning hook, no counterpart in the reference: the launch shape of the compile-time-length
  * H.psi kernels at `precision` -- plane kernel workgroup of 256 or 512 threads, stick kernels

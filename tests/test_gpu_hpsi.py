@@ -418,9 +418,9 @@ def test_projector_contraction_and_padding(si2_system, blocks, dtype, split, rou
 @pytest.mark.parametrize("n,prec,one_lane", [(24, 0, True), (24, 1, True), (42, 0, True), (108, 1, True), (63, 0, False),
                                              (72, 0, False), (84, 1, False)])
 def test_launch_tuning_by_plane_kernel(monkeypatch, n, prec, one_lane):
-    """A call that takes the one-lane plane kernel does not time plane workgroups, which that kernel
-    has none to choose from; a call of few bands, or a wide plan of the same length, has an entry of
-    its own and is timed, whichever comes first."""
+    """A narrow plan of a length with a one-lane plane kernel does not time plane workgroups, which
+    that kernel has none to choose from; a wide plan of the same length has an entry of its own and
+    is timed, whichever comes first."""
     import torch
 
     from amaterasu_amd import autotune
@@ -439,23 +439,21 @@ def test_launch_tuning_by_plane_kernel(monkeypatch, n, prec, one_lane):
 
     monkeypatch.setattr(autotune, "_time_stage", record)
     v = torch.randn((n, n, n), dtype=torch.float64, device="cuda")
-    for half, narrow in ((n / 4.0 - 0.4, True), (n / 4.0 + 3.0, False)):
+    for half, lanes in ((n / 4.0 - 0.4, one_lane), (n / 4.0 + 3.0, False)):
         plan = DevicePlan((n, n, n), [GSphere.build(cell, 0.5 * (half * 2.0 * np.pi / (n / 4.0)) ** 2)])
-        start = plan.info[16 + prec]
-        assert (start > 0) == (narrow and one_lane) and (start == 1) == (narrow and (n, prec) == (108, 1))
+        assert bool(plan.info[16 + prec]) == lanes
         if not plan.plane_ok[prec]:
             continue  # a wide FP64 plane past LDS takes whole grids and has no launch shape
-        for nb in (max(start, 2), 1):
-            psi = torch.randn((1, nb, plan.npw_pad), dtype=torch.complex128 if prec else torch.complex64, device="cuda")
-            lane = 0 < start <= nb
-            known = (n, prec, lane) in autotune._FFT
-            stages.clear()
-            plan.hpsi(psi, v)
-            assert (1 in stages) == (not known) and (2 in stages) == (not known and not lane)
-            stages.clear()
-            plan.hpsi(psi, v)
-            assert not stages and -1 not in (plan.info[12 + prec], plan.info[14 + prec])
-    assert {key[2] for key in autotune._FFT} == ({True} if (n, prec) == (108, 1) else {True, False} if one_lane else {False})
+        psi = torch.randn((1, 2, plan.npw_pad), dtype=torch.complex128 if prec else torch.complex64, device="cuda")
+        known = (n, prec, lanes) in autotune._FFT
+        stages.clear()
+        plan.hpsi(psi, v)
+        assert (1 in stages) == (not known) and (2 in stages) == (not known and not lanes)
+        stages.clear()
+        plan.hpsi(psi, v)
+        assert not stages and -1 not in (plan.info[12 + prec], plan.info[14 + prec])
+    lanes_seen = {key[2] for key in autotune._FFT}
+    assert lanes_seen == ({True, False} if one_lane and n <= 100 else {one_lane})
     for key, (nth, width) in autotune._FFT.items():
         assert (nth == 0) == key[2] and width in (16, 32, 64)
 
@@ -527,52 +525,3 @@ def test_operator_workspace_holds_sticks_only():
     assert torch.equal(out, want) and bool((ws[nbytes:] == 90).all())
     plan.set_route(FP64, True)
     assert lib().amt_hpsi_workspace(plan.handle, FP64, nb, 1) >= nb * n**3 * 16
-
-
-LENGTHS = [20, 21, 22, 24, 25, 27, 28, 30, 32, 33, 35, 36, 40, 42, 44, 45, 48, 49, 50, 54, 55, 56, 60, 63, 64, 66, 70, 72,
-           75, 77, 80, 81, 84, 88, 90, 96, 98, 99, 100, 105, 108, 110, 112, 120, 121, 126, 128]
-
-
-@pytest.mark.parametrize("n", LENGTHS)
-def test_plane_kernels_of_every_length(monkeypatch, n):
-    """Every compile-time length against the library's full-grid route, on a sphere of the usual half
-    width at a shifted k-point: the one-lane kernel from its first call size on and the four-step
-    kernel one band below it, or, where a length has the four-step kernel only, three bands; the
-    four-step kernel in both workgroups, whose results are equal bits. A call that is not large
-    enough for one wavefront or workgroup per CU never takes the one-lane kernel while the plane
-    fits LDS whole. Bound as for the orders of axes above: 64 log2(N) unit roundoffs."""
-    import torch
-
-    from amaterasu_amd._lib import FP32, FP64, check, lib
-    from amaterasu_amd.basis import GSphere
-    from amaterasu_amd.device import DevicePlan
-
-    monkeypatch.setenv("AMT_AUTOTUNE_FFT", "0")
-    shape = (n, n, n)
-    sphere = GSphere.build(np.eye(3) * n / 4.0, 0.5 * ((n / 4.0 - 0.4) * 2.0 * np.pi / (n / 4.0)) ** 2,
-                           kpoint=np.array((0.4, -0.3, 0.1)))
-    g = torch.Generator(device="cuda").manual_seed(n)
-    v = torch.randn(shape, dtype=torch.float64, device="cuda", generator=g)
-    for prec, dt, u in ((FP32, torch.complex64, 2.0**-24), (FP64, torch.complex128, 2.0**-53)):
-        plan = DevicePlan(shape, [sphere])
-        start, whole = plan.info[16 + prec], n * n * (16 if prec else 8) + 24 * n <= 160 * 1024
-        if not plan.plane_ok[prec]:
-            assert prec == FP64 and not whole and start == 0
-            continue
-        assert start != 1 or not whole
-        assert start == 0 or not whole or start * n > 256
-        nb = max(start, 3)
-        psi = torch.randn((1, nb, plan.npw_pad), dtype=dt, device="cuda", generator=g)
-        got = {nb: plan.hpsi(psi, v)}
-        for few in {max(start - 1, 1), 2} if whole else ():
-            both = []
-            for threads in (256, 512):
-                check(lib().amt_plan_set_launch(plan.handle, prec, threads, 0), "plan_set_launch")
-                both.append(plan.hpsi(psi[:, :few].contiguous(), v))
-            assert torch.equal(both[0], both[1])
-            got[few] = both[0]
-        plan.set_route(prec, True)
-        want = plan.hpsi(psi, v)
-        scale = want.abs().max()
-        for rows, h in got.items():
-            assert float((h - want[:, :rows]).abs().max() / scale) < 64 * u * np.log2(np.prod(shape)), (prec, rows)

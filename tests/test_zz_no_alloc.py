@@ -158,31 +158,3 @@ def test_noalloc_names_why_it_refuses_a_plane():
             call()
             torch.cuda.synchronize()
             assert bool(torch.isfinite(torch.view_as_real(out)).all())
-
-
-def test_noalloc_slices_keep_the_plane_kernel_of_the_whole_call():
-    """A block whose rows are past the call size of the one-lane plane kernel (56^3 in FP32), in slices
-    that are not: bit-identical to amt_hpsi_local all the same."""
-    import torch
-
-    from amaterasu_amd import ops
-    from amaterasu_amd._lib import FP32, check, lib
-    from amaterasu_amd.basis import GSphere
-    from amaterasu_amd.device import DevicePlan
-
-    n = 56
-    plan = DevicePlan((n, n, n), [GSphere.build(np.eye(3) * n / 4.0, 0.5 * (13.6 * 2.0 * np.pi / (n / 4.0)) ** 2)])
-    nb = plan.info[16 + FP32] + 7
-    assert nb > (64 << 20) // (n * plan.smax * 8) > 0 and plan.info[16 + FP32] > (64 << 20) // (n * plan.smax * 8)
-    g = torch.Generator(device="cuda").manual_seed(1)
-    psi = torch.randn((1, nb, plan.npw_pad), dtype=torch.complex64, device="cuda", generator=g)
-    v = torch.randn((n, n, n), dtype=torch.float32, device="cuda", generator=g)
-    ws = torch.empty(lib().amt_plan_stick_bytes(plan.handle, FP32, nb), dtype=torch.uint8, device="cuda")
-    a, b = torch.zeros_like(psi), torch.zeros_like(psi)
-    stream = ops.stream_handle()
-    check(lib().amt_hpsi_local(plan.handle, FP32, psi.data_ptr(), a.data_ptr(), nb, 0, 1, v.data_ptr(), ws.data_ptr(),
-                               stream), "hpsi_local")
-    check(lib().amt_hpsi_local_noalloc(plan.handle, FP32, psi.data_ptr(), b.data_ptr(), nb, 0, 1, v.data_ptr(), stream),
-          "noalloc")
-    torch.cuda.synchronize()
-    assert torch.equal(a, b)
