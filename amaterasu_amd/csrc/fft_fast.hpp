@@ -1,6 +1,7 @@
 // Entry points of the compile-time-length kernels (fft_fast_impl.hpp, compiled in four parts).
 #pragma once
 
+#include "fft_reg.hpp"
 #include "kernels.hpp"
 
 namespace amt {
@@ -20,14 +21,19 @@ constexpr int lane_half_width(int n) { return n / 4 + 1; }
 //     on its registers leave too few wavefronts (64: 240/322).
 //   FP32, four lanes: 84 347/310, 108 458/348, 112 444/318, 120 477/309, 128 378/373; up to 96 the
 //     lengths of an 8-point second factor are faster in four steps (72 270/318, 96 308/355).
-//   FP64, one lane: 24 642/429, 32 496/404, 40 483/339, 45 455/399, 48 441/351; 36 = 6 x 6 and
-//     42 = 7 x 6, whose 6-point tasks fill the four-step workgroup, gain nothing (440/432, 440/441;
-//     the 16 x 64-band Si8 batch takes 821/843 us).
+//   FP64, one lane: 24 642/429, 32 496/404, 40 483/339, 45 455/399, 48 441/351. Factors of 6 and 7
+//     points keep both four-step phases short and their tasks even: 36 = 6 x 6 and 42 = 7 x 6 gain nothing
+//     (440/432, 440/441; the three passes of a local H.psi 644/660 and 656/664, with a tenth of the planes
+//     70/74 and 71/77; a factor of 5 leaves them even: 30 703/705, 35 688/699).
 //   FP64, four lanes: 72 767/519, 80 723/670 (64 471/496, 84 690/736, 96 624/877), and above 100,
 //     where a whole plane does not fit LDS.
+// With fewer planes than about six wavefronts a CU the four-step kernel is faster (one band at 48^3 in
+// FP32 16 us against 24) and is not used all the same: one-lane results are nearer to 64 bits (24^3 in
+// FP64 3.4e-16 against 4.2e-16, 84^3 in FP32 2.24e-7 against 2.35e-7), and an iteration whose calls
+// change kernels with their size converges later.
 constexpr int lane_count(int n, bool fp64) {
-  if (fp64 && (n == 6 * 6 || n == 7 * 6)) return 0;
-  if (n <= (fp64 ? 48 : 60)) return 1;
+  const int a = split_n1(n), b = n / a;  // the four-step factors
+  if (n <= (fp64 ? 48 : 60)) return fp64 && b >= 6 && a <= 7 ? 0 : 1;
   if (n % 4) return 0;
   if (fp64) return (n > 64 && n <= 80) || n * n * 16LL + 24LL * n > 160 * 1024 ? 4 : 0;
   return n >= 84 && !(n % 8 == 0 && n <= 96) ? 4 : 0;

@@ -525,3 +525,44 @@ def test_operator_workspace_holds_sticks_only():
     assert torch.equal(out, want) and bool((ws[nbytes:] == 90).all())
     plan.set_route(FP64, True)
     assert lib().amt_hpsi_workspace(plan.handle, FP64, nb, 1) >= nb * n**3 * 16
+
+
+LENGTHS = [20, 21, 22, 24, 25, 27, 28, 30, 32, 33, 35, 36, 40, 42, 44, 45, 48, 49, 50, 54, 55, 56, 60, 63, 64, 66, 70, 72,
+           75, 77, 80, 81, 84, 88, 90, 96, 98, 99, 100, 105, 108, 110, 112, 120, 121, 126, 128]
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_plane_kernels_of_every_length(monkeypatch, n):
+    """Every compile-time length against the library's full-grid route at a shifted k-point: on a
+    sphere of the usual half width the one-lane kernel where the length has one, and on a wide one
+    (and where it has none) the four-step kernel in both its workgroups, whose results are equal bits.
+    Bound as for the orders of axes above: 64 log2(N) unit roundoffs of the largest value."""
+    import torch
+
+    from amaterasu_amd._lib import FP32, FP64, check, lib
+    from amaterasu_amd.basis import GSphere
+    from amaterasu_amd.device import DevicePlan
+
+    monkeypatch.setenv("AMT_AUTOTUNE_FFT", "0")
+    shape, nb = (n, n, n), 3
+    g = torch.Generator(device="cuda").manual_seed(n)
+    v = torch.randn(shape, dtype=torch.float64, device="cuda", generator=g)
+    for half, wide in ((n / 4.0 - 0.4, False), (min(n / 4.0 + 3.0, n / 2.0 - 2.0), True)):
+        sphere = GSphere.build(np.eye(3) * n / 4.0, 0.5 * (half * 2.0 * np.pi / (n / 4.0)) ** 2,
+                               kpoint=np.array((0.4, -0.3, 0.1)))
+        for prec, dt, u in ((FP32, torch.complex64, 2.0**-24), (FP64, torch.complex128, 2.0**-53)):
+            plan = DevicePlan(shape, [sphere])
+            lane, whole = plan.info[16 + prec], n * n * (16 if prec else 8) + 24 * n <= 160 * 1024
+            assert not (wide and lane) and plan.plane_ok[prec] == bool(whole or lane)
+            if not plan.plane_ok[prec]:
+                continue
+            psi = torch.randn((1, nb, plan.npw_pad), dtype=dt, device="cuda", generator=g)
+            got = []
+            for threads in (256, 512):
+                check(lib().amt_plan_set_launch(plan.handle, prec, threads, 0), "plan_set_launch")
+                got.append(plan.hpsi(psi, v))
+            assert torch.equal(got[0], got[1])
+            plan.set_route(prec, True)
+            want = plan.hpsi(psi, v)
+            err = float((got[0] - want).abs().max() / want.abs().max())
+            assert err < 64 * u * np.log2(np.prod(shape)), (prec, wide)
