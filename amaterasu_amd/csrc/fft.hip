@@ -390,8 +390,9 @@ int launch_density_finish(double* rho, int nspin, long long ngrid, double volume
 // odd lengths, whose columns meet no bank conflicts, less: 64 bands at 25^3 24 against 21). FP32
 // rounds of two cost no more than rounds of one (64 bands at 42^3: 6 35 us, 11 40), but for the lengths
 // 4 a, a of 7 or more points, whose second phase meets bank conflicts (64 bands at 32^3: 4 30 us, 8 26).
-// More bands in one FP64 accumulator round more often than chunks of 8 did: 128 bands at 84^3 are off
-// by 2.5e-16 of the 64-bit value where they were by 2.2e-16.
+// The sum's error is least with about as many bands in a chunk as chunks (256 bands at 30^3: 3.1e-16 of the
+// 64-bit value in chunks of 8, 2.9 in 16, 2.8 in 32, 5.3 in one); 128 bands at 84^3 in chunks of 43 are
+// off by 2.5e-16 where chunks of 8 were by 2.2e-16.
 int density_chunk(const Plan& p, int prec, int nlist) {
   if (!p.fast || nlist < 1) return 8;
   const bool fp64 = prec == kFP64;
