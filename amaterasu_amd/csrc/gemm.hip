@@ -16,8 +16,8 @@
 // accumulator differs (measured on gfx950): accumulator element q of lane l is
 // D[4 (l / 16) + q][l % 16] for FP32 and D[l / 16 + 4 q][l % 16] for FP64.
 //
-// Tiling: a 256-thread workgroup computes 16 W rows x 64 columns, W = 1..5 (7 in FP32 without FP64
-// sums, which take the registers) chosen for the row count (plan_gemm): each of the four wavefronts
+// Tiling: a 256-thread workgroup computes 16 W rows x 64 columns, W = 1..5 (7 in FP32 without second
+// sums, 4 in FP64 with them: registers) chosen for the row count (plan_gemm): each of the four wavefronts
 // owns 16 columns and all 16 W rows, so 8 bands compute 16 rows, 45 compute 48 and 160 compute 160,
 // where fixed 64-row tiles computed 64, 64 and 192. K advances 128 bytes of a row at a time (16 complex64, 8
 // complex128) through two LDS buffers: the next tile's 16-byte global loads are issued before
@@ -33,12 +33,12 @@
 // (4 p + g) * (16 / sizeof(C)) + s; any order of K is the same sum as long as A and B agree. B of
 // an NN product stays [k][column], read 8 (16) bytes at a time from rows of 72 (64) elements.
 //
-// FP32 accumulation over a long K is two-level: the MFMA's FP32 accumulators cover 64 to 256 of K
-// (fp32_sums()) and are then added into FP64 registers, so the rounding error of a long contraction
+// Accumulation over a long K is two-level: the MFMA's FP32 accumulators cover 64 to 256 of K
+// (inner_sums()) and are then added into FP64 registers, so the rounding error of a long contraction
 // (subspace overlaps over ~10^5 plane waves) grows with that length, not with K. One FP32 accumulator over
 // all of K = 81k left relative errors of ~6e-5 in the Gram matrices of a 440-band Davidson,
 // enough to stall an SCF. The additions cost 2 to 5 % of a product; split partials are summed in
-// FP64 too.
+// FP64 too. FP64 products of a middling K have second sums of the same kind.
 //
 // What bounds it: the matrix cores. Of a wavefront's cycles on 440 x 3852 x 40 000 (FP32, NC) 81 %
 // are MFMA at the 2.14 GHz the chip holds under them. Measured (TFLOP/s at 8 real flops per
@@ -47,6 +47,7 @@
 //   122 (100), 45 x 3852 x 80989 NC 127 (84), 440 x 80989 x 3852 NN 149 (113), 440 x 3852 x 80989
 //   NC 150 (107); FP64 160 x 1152 x 37073 NC 73 (46), its NN 76 (53), 45 x 3852 x 80989 NC 65 (39).
 #include <array>
+#include <climits>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(int M, int N, int K, int kchun
   // C_re and C_im of one accumulator element; conj(B) turns the signs of the P2 terms
   auto re_of = [](auto t1, auto t2) { return OP == 0 ? t1 - t2 : t1 + t2; };
   auto im_of = [](auto t1, auto t2, auto t3) { return OP == 0 ? t3 - t1 - t2 : t3 - t1 + t2; };
-  // second-level FP64 sums of the FP32 accumulators (two-level form only)
+  // second-level FP64 sums of the accumulators (two-level form only)
   double sumr[kTwoLevel ? W : 1][4], sumi[kTwoLevel ? W : 1][4];
   auto flush = [&]() {
     if constexpr (kTwoLevel) {
@@ -416,8 +417,8 @@ static std::array<int, 6> split_key(int prec, int op, int m, int n, int k, int b
   return {prec, op, (m + 63) / 64, (n + 63) / 64, (k + 255) / 256, batch};
 }
 
-// Longest K that one FP32 accumulator covers without FP64 sums, and K between the additions into
-// FP64 beyond it. A product's rounding grows with the accumulator's length, so the length follows
+// Longest K that one accumulator covers without second sums, and K between the additions into them
+// beyond it. A product's rounding grows with the accumulator's length, so the length follows
 // from the shape and not from the split that happens to be fastest:
 //   NC (overlaps, projections: K the plane waves): 256; up to 4096 of K 128, as a few splits of at
 //     most 256 that divide such a K are shorter than that themselves; 64 for outputs of 512 tiles of
@@ -430,11 +431,19 @@ static std::array<int, 6> split_key(int prec, int op, int m, int n, int k, int b
 // over all of K by 4.4, 5.3 and 6.1e-7 in 14.7, 31.7 and 55.3, with additions every 64 of K by 2.1e-7
 // in 15.5, 33.4 and 61.0. NC products of K > 4096 with additions every 64: 2.1e-7 for 3.9e-7, 3 to 8 %
 // slower.
-struct Fp32Sums {
+// FP64: 192, then additions every 160 of K, where the output has fewer than 512 tiles of 80 x 64 and
+// K is 257 to 1024 (NN) or 16 384 (NC). Past these the products of a whole subspace and the
+// projections of 10^5 plane waves, bound by the matrix cores, keep one accumulator per split. Error
+// (1e-16) and time, with single accumulators and so: NN 58 x 13 900 x 432 10.4 in 56.2 us and 5.9 in
+// 57.2, 80 x 18 500 x 576 10.3 in 109 and 5.4 in 112, 80 x 18 500 x 1000 15.7 in 188 and 5.7 in 202;
+// NC 5 of 19 x 1381 x 355 8.7 in 20.9 and 5.5 in 21.5, 16 of 64 x 144 x 4954 8.8 in 118 and 6.1 in
+// 121, 4 of 40 x 288 x 9300 7.9 in 73.5 and 5.8 in 76.6.
+struct InnerSums {
   int limit, flush;
 };
-static Fp32Sums fp32_sums(int op, int m, int n, int k, int batch) {
+static InnerSums inner_sums(int prec, int op, int m, int n, int k, int batch) {
   auto tiles = [&](int rows) { return (long long)((m + rows - 1) / rows) * ((n + BN - 1) / BN) * batch; };
+  if (prec == kFP64) return {k > 256 && k <= (op == 0 ? 1024 : 16384) && tiles(80) < 512 ? 192 : INT_MAX, 160};
   if (op == 0) return {k <= 256 || (k <= 1024 && tiles(80) >= 512) ? 1024 : 0, k <= 1024 ? 128 : 64};
   const int flush = k > 1024 && tiles(64) >= 512 ? 64 : k > 4096 ? 256 : 128;
   return {k <= 256 ? 256 : flush, flush};
@@ -444,13 +453,13 @@ constexpr int kMinChunk = 64;
 constexpr int kBigSide = 256;
 
 // Tile rows in 16s, widest kernel of each kind (registers: two wavefronts per SIMD).
-constexpr int kMaxW = 7, kMaxWLong = 5;
+constexpr int kMaxW = 7, kMaxWLong = 5, kMaxW64 = 5, kMaxW64Long = 4;
 
 struct GemmPlan {
   int w;        // rows of a tile in 16s
   int ns;       // K splits
   int kchunk;   // K per split, a multiple of the K tile
-  bool two;     // FP64 second-level sums
+  bool two;     // second-level sums
   int flush;    // K tiles between them
 };
 
@@ -467,12 +476,12 @@ static bool split_is_tunable(int prec, int op, int m, int n, int k) {
 // The first factor is what uneven rounds cost: 160 x 37 073 x 1152 (580
 // column tiles) in 32-row tiles fills its last round better than in 80-row ones. Against a sweep
 // of every W and split the choice is within 5 % on the Si8, Si64 and Si214 shapes.
-// No split lengthens an accumulator past fp32_sums(): 3.7-4.1e-7 (relative norm, random operands) on
+// No split lengthens an accumulator past inner_sums(): 3.7-4.1e-7 (relative norm, random operands) on
 // every NC shape above, where single accumulators over 256 to 1024 of K gave 4.1 to 7.9e-7.
 static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
   const int csize = prec == kFP64 ? 16 : 8, bk = kChunks * 16 / csize;
   const double cols = (double)((n + BN - 1) / BN) * batch, out = (double)m * n * batch * csize;
-  const Fp32Sums sums = fp32_sums(op, m, n, k, batch);
+  const InnerSums sums = inner_sums(prec, op, m, n, k, batch);
   GemmPlan best{1, 1, bk, false, sums.flush / bk};
   double best_cost = 1e300;
   int lo = 1, hi = (k + kMinChunk - 1) / kMinChunk;
@@ -482,6 +491,7 @@ static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
     auto it = g_split_table.find(split_key(prec, op, m, n, k, batch));
     if (it != g_split_table.end()) lo = hi = it->second < hi ? it->second : hi;
   }
+  const auto widest = [&](bool two) { return prec == kFP64 ? (two ? kMaxW64Long : kMaxW64) : two ? kMaxWLong : kMaxW; };
   double rows[kMaxW + 1];
   for (int w = 1; w <= kMaxW; ++w) rows[w] = (double)((m + 16 * w - 1) / (16 * w)) * cols;
   for (int want = lo; want <= hi; want += 1 + want / 8) {
@@ -489,10 +499,11 @@ static GemmPlan plan_gemm(int prec, int op, int m, int n, int k, int batch) {
     if (kchunk < bk) kchunk = bk;
     const int ns = k > 0 ? (k + kchunk - 1) / kchunk : 1;
     if (best_cost < 1e300 && (long long)batch * ns > 65535) break;
-    const bool two = prec == kFP32 && (op == 1 ? kchunk : k) > sums.limit;
+    const bool two = (op == 1 || prec == kFP64 ? kchunk : k) > sums.limit;
     const double tiles = kchunk / bk + 2, extra = ns > 1 ? 20.0 + 2.0 * out * ns / 1.3e6 : 0.0;
-    for (int w = 1; w <= (prec == kFP64 || two ? kMaxWLong : kMaxW); ++w) {
-      const double cost = (std::ceil(rows[w] * ns / 256.0) + 0.8) * tiles * (w + 0.35) * (two ? 1.1 : 1.0) + extra;
+    for (int w = 1; w <= widest(two); ++w) {
+      const double cost =
+          (std::ceil(rows[w] * ns / 256.0) + 0.8) * tiles * (w + 0.35) * (two && prec == kFP32 ? 1.1 : 1.0) + extra;
       if (cost < best_cost) {
         best_cost = cost;
         best.w = w;
@@ -654,7 +665,11 @@ static int zgemm_t(int op, int m, int n, int k, double alpha, const void* a, lon
       }
     }
   } else {
-    switch (g.w) { AMT_W(false, 1) AMT_W(false, 2) AMT_W(false, 3) AMT_W(false, 4) AMT_W(false, 5) }
+    if (g.two) {
+      switch (g.w) { AMT_W(true, 1) AMT_W(true, 2) AMT_W(true, 3) AMT_W(true, 4) }
+    } else {
+      switch (g.w) { AMT_W(false, 1) AMT_W(false, 2) AMT_W(false, 3) AMT_W(false, 4) AMT_W(false, 5) }
+    }
   }
 #undef AMT_W
   hipError_t e = hipGetLastError();

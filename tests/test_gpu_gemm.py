@@ -201,3 +201,27 @@ def test_zgemm_fp32_accumulator_length(op, m, n, k, batch):
     got = ops.zgemm(a, b.to(torch.complex64), op)
     assert not got.imag.any()
     assert bool(((got.real.to(torch.float64) - want).abs() <= 2 * 2.0**-24 * want).all())
+
+
+@pytest.mark.parametrize("op,m,n,k,batch", [(0, 80, 18500, 576, 1), (0, 58, 13900, 432, 1), (0, 80, 18500, 1000, 1),
+                                            (0, 52, 5241, 272, 4), (0, 133, 7390, 288, 2), (0, 178, 8418, 621, 1),
+                                            (1, 19, 1381, 355, 5), (1, 83, 7159, 265, 2), (1, 133, 7946, 303, 2),
+                                            (1, 180, 3826, 1382, 1), (1, 40, 288, 9300, 4)])
+def test_zgemm_fp64_accumulator_length(op, m, n, k, batch):
+    """FP64 products of 257 and more of K sum it in pieces of at most 192, of 1 to 4 tile heights.
+    Integers whose sums are exact up to that length: what is left is one rounding for each piece
+    added, of half a unit of the (positive) sum at most, and no more than K / 64 + 1 of them; one
+    accumulator over all of K rounds at every fourth of K past 192."""
+    import torch
+
+    from amaterasu_amd import ops
+
+    top = 2**53 // 192
+    g = torch.Generator(device="cuda").manual_seed(k)
+    b = torch.randint(top - top // 20, top + 1, (batch, k, n) if op == 0 else (batch, n, k), device="cuda", generator=g)
+    want = b.sum(1 if op == 0 else 2)[:, None, :]
+    a = torch.ones((batch, m, k), dtype=torch.complex128, device="cuda")
+    got = ops.zgemm(a, b.to(torch.complex128), op)
+    assert not got.imag.any()
+    bound = (k / 64 + 1) * 2.0**-53 * want.to(torch.float64)
+    assert bool(((got.real.to(torch.int64) - want).abs().to(torch.float64) <= bound).all())
